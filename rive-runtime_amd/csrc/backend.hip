@@ -103,7 +103,7 @@ struct rive_hip_context
     MappedBuffer bufs[RIVE_HIP_BUFFER_KIND_COUNT];
     // pipeline scratch (grow-only)
     DevBuf spanTexelCounts, spanTexelOffsets, scanPartials, scalars;
-    DevBuf tess, prims, cells, cellCount, cellOffset, cellCursor, cellBackdrop, binned, cellPacked, pathDraws;
+    DevBuf tess, prims, cells, cellCursor, binned, cellPacked, pathDraws, pathBins, pathBase;
     DevBuf pathRaster, pathPaint, ramps, drawTess, verts;
     DevBuf geoCounts, geoRecords, geoContours, geoSpans, geoSpanCounts, geoSpanOffsets;
     uint32_t lastMode = 0, lastRecordCount = 0, lastTessVertexCount = 0;
@@ -189,16 +189,17 @@ struct rive_hip_context
 namespace
 {
 // The scratch buffers of a context (every DevBuf member), in one list.
-constexpr int kDevBufCount = 40;
+constexpr int kDevBufCount = 39;
 // The device scalars of a flush (totals, counters), 32 words: the pipeline
 // uses slots 0-7, device counting 8-13, guard-box pieces kFarSlot .. +3.
 constexpr size_t kScalarBytes = 128;
 constexpr int kFarSlot = 16;
+constexpr int kSharedSlot = kFarSlot + 4; // set when a path is not binned solo
 void devbufs(rive_hip_context* c, DevBuf** out)
 {
     DevBuf* all[kDevBufCount] = {&c->spanTexelCounts, &c->spanTexelOffsets, &c->scanPartials, &c->scalars,
-                                 &c->tess, &c->prims, &c->cells, &c->cellCount, &c->cellOffset,
-                                 &c->cellCursor, &c->cellBackdrop, &c->binned, &c->pathRaster,
+                                 &c->tess, &c->prims, &c->cells, &c->pathBins, &c->pathBase,
+                                 &c->cellCursor, &c->binned, &c->pathRaster,
                                  &c->ramps, &c->drawTess, &c->geoCounts, &c->geoRecords,
                                  &c->geoContours, &c->geoSpans, &c->geoSpanCounts, &c->geoSpanOffsets,
                                  &c->verts, &c->imageTable, &c->pathImage, &c->canvasTable,
@@ -435,6 +436,13 @@ int rive_hip_create(int device, rive_hip_context** out)
         feather_tables_host(tables.data());
         e = hipMemcpy(ctx->featherTables, tables.data(), sizeof(float) * tables.size(), hipMemcpyHostToDevice);
     }
+    // the binning of large grids takes more LDS than a launch may by default
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bin_count_solo_kernel<1024>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kBinLargeCells * 4);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bin_scatter_solo_kernel<1024>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kBinLargeCells * 4);
     ctx->evSets.reserve(kMaxFrameEventSets);
     ctx->evSets.emplace_back();
     ctx->evSets[0].fill(nullptr);
@@ -1275,8 +1283,7 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
         HIP_TRY(hipHostMalloc((void**)&ctx->hostCanvases, sizeof(CanvasDev) * canvasCount, hipHostMallocDefault));
         ctx->hostCanvasesCap = canvasCount;
     }
-    uint32_t tileTotal = 0;
-    int maxTilesY = 1;
+    uint32_t tileTotal = 0, maxTiles = 1;
     for (uint32_t c = 0; c < canvasCount; ++c)
     {
         const rive_hip_canvas& cv = ctx->lastCanvases[c];
@@ -1293,7 +1300,7 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
         cd.clearPremul = premul_clear(cv.clear_color);
         cd.loadPreserve = cv.load_action == 1 ? 1u : 0u;
         tileTotal += (uint32_t)(cd.tilesX * cd.tilesY);
-        maxTilesY = std::max(maxTilesY, cd.tilesY);
+        maxTiles = std::max(maxTiles, (uint32_t)(cd.tilesX * cd.tilesY));
     }
     RIVE_TRY(ensure(ctx, ctx->canvasTable, sizeof(CanvasDev) * std::max<uint32_t>(canvasCount, 1)));
     RIVE_TRY(upload_table(ctx, ctx->canvasTable.ptr, ctx->hostCanvases, sizeof(CanvasDev) * canvasCount));
@@ -1385,14 +1392,21 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
     cells_layout_kernel<<<1, 1024, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
                                                      P<uint32_t>(ctx->pathCanvas), P<CanvasDev>(ctx->canvasTable),
                                                      scal + 1);
+    RIVE_TRY(ensure(ctx, ctx->pathDraws, (size_t)(pathCount + 1) * 4));
+    RIVE_TRY(clear(ctx, ctx->pathDraws.ptr, 0, (size_t)(pathCount + 1) * 4));
+    if (drawCount > 0)
+        path_draws_kernel<<<(drawCount + 255) / 256, 256, 0, ctx->stream>>>(
+            drawTess, drawCount, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), scal + kSharedSlot);
     HIP_TRY(hipGetLastError());
     // Cell total, the count of texels naming no ContourData record, and the
-    // primitives leaving the guard box with their piece total.
+    // primitives leaving the guard box with their piece total; whether a path
+    // is not solo.
     RIVE_TRY(fetch(ctx, ctx->hostScalars, scal + 1, 20));
-    RIVE_TRY(fetch(ctx, ctx->hostScalars + 5, scal + kFarSlot, 8));
+    RIVE_TRY(fetch(ctx, ctx->hostScalars + 5, scal + kFarSlot, 20));
     RIVE_TRY(settle(ctx));
     const uint32_t totalCells = ctx->hostScalars[0];
     const uint32_t farPrims = ctx->hostScalars[5], pieces = ctx->hostScalars[6];
+    bool shared = ctx->hostScalars[5 + kSharedSlot - kFarSlot] != 0;
     if (ctx->hostScalars[4] != 0)
         return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT,
                     "tessellated vertices name contour IDs outside 1..contour_count");
@@ -1427,31 +1441,49 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
         HIP_TRY(hipGetLastError());
         binDraws = P<DrawTess>(ctx->drawTessAll);
         binDrawCount = drawCount * 2;
+        // the pieces' draws bin into their paths too
+        RIVE_TRY(clear(ctx, ctx->pathDraws.ptr, 0, (size_t)(pathCount + 1) * 4));
+        path_draws_kernel<<<(binDrawCount + 255) / 256, 256, 0, ctx->stream>>>(
+            binDraws, binDrawCount, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), scal + kSharedSlot);
+        shared = true;
     }
-    RIVE_TRY(ensure(ctx, ctx->cellCount, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(ensure(ctx, ctx->cellOffset, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(ensure(ctx, ctx->cellCursor, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(ensure(ctx, ctx->cellBackdrop, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->cellCount.ptr, 0, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->cellCursor.ptr, 0, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->cellBackdrop.ptr, 0, (size_t)(totalCells + 1) * 4));
-    RIVE_TRY(ensure(ctx, ctx->pathDraws, (size_t)(pathCount + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->pathDraws.ptr, 0, (size_t)(pathCount + 1) * 4));
-    if (totalPrims > 0 && drawCount > 0)
-        bin_count_draw_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
-            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->cellCount),
-            P<int32_t>(ctx->cellBackdrop), P<uint32_t>(ctx->pathDraws));
-    rc = device_scan(ctx, P<uint32_t>(ctx->cellCount), totalCells, P<uint32_t>(ctx->cellOffset), scal + 2);
+    RIVE_TRY(ensure(ctx, ctx->cellPacked, (size_t)std::max<uint32_t>(totalCells, 1) * sizeof(uint2)));
+    RIVE_TRY(ensure(ctx, ctx->pathBins, (size_t)(pathCount + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->pathBase, (size_t)(pathCount + 2) * 4));
+    RIVE_TRY(clear(ctx, ctx->pathBins.ptr, 0, (size_t)(pathCount + 1) * 4));
+    // The solo kernels' LDS: as many words as the largest canvas has tiles,
+    // up to the small limit; a second launch takes the larger grids.
+    const bool bin = totalPrims > 0 && drawCount > 0 && totalCells > 0;
+    const uint32_t smallCells = std::min(maxTiles, kBinSmallCells), largeCells = std::min(maxTiles, kBinLargeCells);
+    if (bin)
+    {
+        bin_count_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
+            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins));
+        if (largeCells > smallCells)
+            bin_count_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
+                P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
+                largeCells, P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins));
+    }
+    if (bin && shared)
+    {
+        RIVE_TRY(ensure(ctx, ctx->cellCursor, (size_t)totalCells * 4));
+        shared_clear_kernel<<<pathCount + 1, 256, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
+                                                                    P<uint32_t>(ctx->pathDraws),
+                                                                    P<uint2>(ctx->cellPacked),
+                                                                    P<uint32_t>(ctx->cellCursor));
+        shared_count_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(P<Prim>(ctx->prims), binDraws,
+                                                                   P<PathCells>(ctx->cells),
+                                                                   P<uint32_t>(ctx->pathDraws),
+                                                                   P<uint2>(ctx->cellPacked));
+        shared_layout_kernel<<<pathCount + 1, 256, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
+                                                                     P<uint32_t>(ctx->pathDraws),
+                                                                     P<uint2>(ctx->cellPacked),
+                                                                     P<uint32_t>(ctx->pathBins));
+    }
+    rc = device_scan(ctx, P<uint32_t>(ctx->pathBins), pathCount + 1, P<uint32_t>(ctx->pathBase), scal + 2);
     if (rc)
         return rc;
-    RIVE_TRY(ensure(ctx, ctx->cellPacked, (size_t)(totalCells + 1) * sizeof(uint2)));
-    {
-        int maxRows = maxTilesY;
-        const uint64_t threads = std::max<uint64_t>((uint64_t)(pathCount + 1) * (uint64_t)maxRows * 64u, 1);
-        backdrop_prefix_kernel<<<(uint32_t)((threads + 255) / 256), 256, 0, ctx->stream>>>(
-            P<PathCells>(ctx->cells), pathCount + 1, maxRows, P<int32_t>(ctx->cellBackdrop),
-            P<uint32_t>(ctx->cellOffset), totalCells, P<uint2>(ctx->cellPacked));
-    }
     uint32_t totalPairs = 0;
     rc = read_total(ctx, scal + 2, &totalPairs, "binned (primitive, tile) pairs");
     if (rc)
@@ -1460,10 +1492,21 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
     ctx->stats.prim_count = totalPrims;
     ctx->stats.tile_count = tileTotal;
     RIVE_TRY(ensure(ctx, ctx->binned, (size_t)std::max<uint32_t>(totalPairs, 1) * 4));
-    if (totalPrims > 0 && drawCount > 0)
-        bin_scatter_draw_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
-            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->cellOffset),
-            P<uint32_t>(ctx->cellCursor), P<uint32_t>(ctx->pathDraws), P<uint32_t>(ctx->binned));
+    if (bin)
+    {
+        bin_scatter_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
+            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+        if (largeCells > smallCells)
+            bin_scatter_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
+                P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
+                largeCells, P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+    }
+    if (bin && shared)
+        shared_scatter_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
+            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws),
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->cellCursor),
+            P<uint32_t>(ctx->binned));
     RIVE_TRY(ensure(ctx, ctx->pathRaster, (size_t)(pathCount + 1) * sizeof(PathRaster)));
     RIVE_TRY(ensure(ctx, ctx->pathPaint, (size_t)(pathCount + 1) * sizeof(PathPaint)));
     path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
@@ -1505,7 +1548,7 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
                        : tileTotal;
         raster_fn(feathered, persistent, waves)<<<grid, kWgThreads, 0, ctx->stream>>>(
             P<PathCells>(ctx->cells), P<PathRaster>(ctx->pathRaster), P<PathPaint>(ctx->pathPaint),
-            P<uint2>(ctx->cellPacked),
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
             P<uint32_t>(ctx->binned), P<Prim>(ctx->prims),
             P<uint32_t>(ctx->ramps), gradRows, P<ImageDesc>(ctx->imageTable), P<CanvasDev>(ctx->canvasTable),
             canvasCount, d->dither, ctx->featherTables, order, tileTotal, queue + 2 * kCostClasses);

@@ -1549,7 +1549,6 @@ __global__ void cells_init_kernel(PathCells* __restrict__ cells, uint32_t n)
     cells[i] = c;
 }
 
-// Single block: sizes each path's grid and assigns bases (exclusive scan).
 // The canvas of each path (0xffffffff for paths outside every canvas): one
 // block per canvas.
 __global__ void path_canvas_kernel(const CanvasDev* __restrict__ canvases, uint32_t* __restrict__ pathCanvas)
@@ -1559,6 +1558,7 @@ __global__ void path_canvas_kernel(const CanvasDev* __restrict__ canvases, uint3
         pathCanvas[p] = blockIdx.x;
 }
 
+// Single block: sizes each path's grid and assigns bases (exclusive scan).
 __global__ void cells_layout_kernel(PathCells* __restrict__ cells, uint32_t n,
                                     const uint32_t* __restrict__ pathCanvas,
                                     const CanvasDev* __restrict__ canvases, uint32_t* __restrict__ totalCells)
@@ -1584,7 +1584,7 @@ __global__ void cells_layout_kernel(PathCells* __restrict__ cells, uint32_t n,
             c.tx1 = min(c.tx1, tilesX);
             c.ty1 = min(c.ty1, tilesY);
             if (c.tx0 < c.tx1 && c.ty0 < c.ty1)
-                area = (uint32_t)((c.tx1 - c.tx0) * (c.ty1 - c.ty0));
+                area = (uint32_t)((c.tx1 - c.tx0) * (c.ty1 - c.ty0)) + 1u; // and the end entry
             else
             {
                 c.tx0 = c.ty0 = 0;
@@ -1779,194 +1779,305 @@ __device__ __forceinline__ void for_prim_crossings(const Prim& p, const PathCell
     }
 }
 
-// Binning per draw: one 256-thread workgroup takes one draw's primitives and
-// accumulates its (primitive, tile) counts and corner crossings over its
-// path's cell grid in LDS, then adds them to the global grids once per cell.
-// Grids larger than kBinLdsCells use global atomics directly.
-constexpr uint32_t kBinLdsCells = 8192;
+// ---- binning per draw
+//
+// A path's grid takes nCells + 1 consecutive entries of `packed`: entry i is
+// (the cell's first bin, counted from the path's own first bin; the winding at
+// the cell's corner), the last one the path's bin total.  The raster adds the
+// path's first bin (pathBase, a scan over the paths' totals).
+//
+// A path drawn by one draw with a grid that fits LDS (a "solo" path) is binned
+// by one workgroup without global atomics: the (primitive, tile) counts and
+// corner crossings accumulate in LDS, the crossings become windings (prefix
+// along each row) and the counts bin offsets (prefix over the grid) there,
+// and every entry is stored once, 8 bytes, coalesced.  What it replaces
+// cleared, counted, scanned and packed the grids in global memory, about 45
+// bytes moved per cell in seven launches; grids are most of binning's traffic
+// (25 M cells in the 1080p 5000-path frame).  Grids of more than kBinSmallCells
+// cells (a canvas beyond 8192 tiles) take the same kernel with up to 160 KB of
+// LDS and 1024 threads, one workgroup per CU; they used to go through one
+// global atomic per (primitive, tile).  Measured on MI355X, the whole pass
+// (expansion included): 1080p 5000-path frame 3.53 -> 3.00 ms, 3840x2160
+// 20 000-path frame 126.8 -> 46.7 ms, 48-canvas batch 2.14 -> 1.79 ms.
+//
+// Other paths (several draws, as with guard-box pieces; 32768 primitives or
+// more, which the packed LDS word cannot count; grids beyond the large LDS)
+// take the shared_* kernels with global atomics.
+constexpr uint32_t kBinSmallCells = 8192;
+constexpr uint32_t kBinLargeCells = 40000;
+constexpr uint32_t kBinSoloPrims = 32768;
 
 __device__ __forceinline__ uint32_t grid_cells(const PathCells& c)
 {
     return c.tx0 < c.tx1 && c.ty0 < c.ty1 ? c.width * (uint32_t)(c.ty1 - c.ty0) : 0u;
 }
 
-__global__ __launch_bounds__(256) void bin_count_draw_kernel(const Prim* __restrict__ prims,
-                                                             const DrawTess* __restrict__ draws,
-                                                             const PathCells* __restrict__ cells,
-                                                             uint32_t* __restrict__ cellCount,
-                                                             int32_t* __restrict__ cellBackdrop,
-                                                             uint32_t* __restrict__ pathDraws)
+// Counts the draws that bin into each path's grid (a path is solo when its
+// count is 1; a draw that cannot be binned in LDS counts twice); flags a path
+// that is not solo.
+__global__ void path_draws_kernel(const DrawTess* __restrict__ draws, uint32_t drawCount,
+                                  const PathCells* __restrict__ cells, uint32_t* __restrict__ pathDraws,
+                                  uint32_t* __restrict__ anyShared)
 {
-    // One word per cell: the primitive count in the low 16 bits and the
-    // corner-crossing sum, two's complement, in the high 16.  A draw with
-    // fewer than 32768 primitives keeps the count below 2^15 (no carry) and
-    // the sum within +-2^15 (each primitive adds at most +-1 to a cell), so
-    // both halves are exact; larger draws use global atomics.  32 KB of LDS
-    // keeps five workgroups per CU.
-    __shared__ uint32_t sCell[kBinLdsCells];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= drawCount)
+        return;
+    const DrawTess d = draws[i];
+    if (d.pathID == 0u || d.forwardCount == 0u)
+        return;
+    const uint32_t nCells = grid_cells(cells[d.pathID]);
+    if (nCells == 0u)
+        return;
+    const uint32_t add = nCells > kBinLargeCells || d.forwardCount >= kBinSoloPrims ? 2u : 1u;
+    if (atomicAdd(&pathDraws[d.pathID], add) + add > 1u)
+        *anyShared = 1u; // every writer stores the same value
+}
+
+__device__ __forceinline__ int32_t wave_scan_add(int32_t v, int lane)
+{
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+    {
+        const int32_t t = __shfl_up(v, d);
+        if (lane >= d)
+            v += t;
+    }
+    return v;
+}
+
+// One workgroup per draw of a solo path whose grid has [minCells, maxCells]
+// cells (LDS: one word per cell).  The word holds the primitive count in its
+// low 16 bits and the corner-crossing sum, two's complement, in the high 16: a
+// draw of fewer than 32768 primitives keeps the count below 2^15 (no carry)
+// and every sum of crossings within +-2^15 (each primitive adds at most +-1 to
+// a row), so both halves and the windings formed in place are exact.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
+    const Prim* __restrict__ prims, const DrawTess* __restrict__ draws, const PathCells* __restrict__ cells,
+    const uint32_t* __restrict__ pathDraws, uint32_t minCells, uint32_t maxCells, uint2* __restrict__ packed,
+    uint32_t* __restrict__ pathBins)
+{
+    extern __shared__ uint32_t sCell[];
+    __shared__ uint32_t sWaveSum[THREADS / 64];
     const DrawTess d = draws[blockIdx.x];
-    if (d.pathID == 0 || d.forwardCount == 0)
+    if (d.pathID == 0u || d.forwardCount == 0u)
         return;
     const PathCells c = cells[d.pathID];
     const uint32_t nCells = grid_cells(c);
-    if (nCells == 0)
+    if (nCells < minCells || nCells > maxCells || pathDraws[d.pathID] != 1u)
         return;
-    if (threadIdx.x == 0)
-        atomicAdd(&pathDraws[d.pathID], 1u); // draws binning into this path's grid
-    const bool local = nCells <= kBinLdsCells && d.forwardCount < 32768u;
-    if (local)
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = threadIdx.x >> 6, waves = THREADS / 64;
+    for (uint32_t i = threadIdx.x; i < nCells; i += THREADS)
+        sCell[i] = 0;
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < d.forwardCount; k += THREADS)
     {
-        for (uint32_t i = threadIdx.x; i < nCells; i += blockDim.x)
-            sCell[i] = 0;
-        __syncthreads();
+        const Prim p = prims[d.primBase + k];
+        if (p.flags & kPrimEmpty)
+            continue;
+        for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&sCell[cell], 1u); });
+        for_prim_crossings(p, c, [&](uint32_t cell, int v) { atomicAdd(&sCell[cell], (uint32_t)v << 16); });
     }
-    uint32_t* gCount = cellCount + c.base;
-    int32_t* gBack = cellBackdrop + c.base;
+    __syncthreads();
+    // corner windings: a prefix along each row, one wave per row
+    const uint32_t rows = (uint32_t)(c.ty1 - c.ty0);
+    for (uint32_t r = wave; r < rows; r += waves)
+    {
+        int32_t carry = 0;
+        for (uint32_t x0 = 0; x0 < c.width; x0 += 64)
+        {
+            const uint32_t x = x0 + (uint32_t)lane;
+            const uint32_t w = x < c.width ? sCell[r * c.width + x] : 0u;
+            const int32_t v = wave_scan_add((int32_t)w >> 16, lane) + carry;
+            if (x < c.width)
+                sCell[r * c.width + x] = (w & 0xffffu) | ((uint32_t)v << 16);
+            carry = __shfl(v, 63);
+        }
+    }
+    __syncthreads();
+    // bin offsets: a prefix of the counts over the grid, each wave one run of
+    // whole 64-cell steps
+    const uint32_t steps = (nCells + 63u) / 64u, perWave = (steps + waves - 1u) / waves;
+    const uint32_t first = wave * perWave * 64u, end = min(first + perWave * 64u, nCells);
+    uint32_t sum = 0;
+    for (uint32_t i = first + (uint32_t)lane; i < end; i += 64u)
+        sum += sCell[i] & 0xffffu;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1)
+        sum += (uint32_t)__shfl_xor((int)sum, s);
+    if (lane == 0)
+        sWaveSum[wave] = sum;
+    __syncthreads();
+    uint32_t carry = 0, total = 0;
+    for (uint32_t w = 0; w < waves; ++w)
+    {
+        carry += w < wave ? sWaveSum[w] : 0u;
+        total += sWaveSum[w];
+    }
+    for (uint32_t i0 = first; i0 < end; i0 += 64u)
+    {
+        const uint32_t i = i0 + (uint32_t)lane;
+        const uint32_t w = i < end ? sCell[i] : 0u;
+        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)(w & 0xffffu), lane);
+        if (i < end)
+            packed[c.base + i] = make_uint2(carry + incl - (w & 0xffffu), (uint32_t)((int32_t)w >> 16));
+        carry += (uint32_t)__shfl((int)incl, 63);
+    }
+    if (threadIdx.x == 0)
+    {
+        packed[c.base + nCells] = make_uint2(total, 0u);
+        pathBins[d.pathID] = total;
+    }
+}
+
+// Writes each primitive's index into its cells' bins: LDS cursors start at the
+// cells' bin offsets, so a solo path's bins need no global atomics.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void bin_scatter_solo_kernel(
+    const Prim* __restrict__ prims, const DrawTess* __restrict__ draws, const PathCells* __restrict__ cells,
+    const uint32_t* __restrict__ pathDraws, uint32_t minCells, uint32_t maxCells,
+    const uint2* __restrict__ packed, const uint32_t* __restrict__ pathBase, uint32_t* __restrict__ binned)
+{
+    extern __shared__ uint32_t sCell[];
+    const DrawTess d = draws[blockIdx.x];
+    if (d.pathID == 0u || d.forwardCount == 0u)
+        return;
+    const PathCells c = cells[d.pathID];
+    const uint32_t nCells = grid_cells(c);
+    if (nCells < minCells || nCells > maxCells || pathDraws[d.pathID] != 1u)
+        return;
+    const uint32_t base = pathBase[d.pathID];
+    for (uint32_t i = threadIdx.x; i < nCells; i += THREADS)
+        sCell[i] = base + packed[c.base + i].x;
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < d.forwardCount; k += THREADS)
+    {
+        const uint32_t g = d.primBase + k;
+        const Prim p = prims[g];
+        if (!(p.flags & kPrimEmpty))
+            for_prim_cells(p, c, [&](uint32_t cell) { binned[atomicAdd(&sCell[cell], 1u)] = g; });
+    }
+}
+
+// ---- paths that are not solo: counts and crossings by global atomics on the
+// cleared grid, the prefixes by one workgroup per path, then scatter cursors.
+__global__ __launch_bounds__(256) void shared_clear_kernel(const PathCells* __restrict__ cells, uint32_t pathCount,
+                                                           const uint32_t* __restrict__ pathDraws,
+                                                           uint2* __restrict__ packed,
+                                                           uint32_t* __restrict__ cellCursor)
+{
+    const uint32_t path = blockIdx.x;
+    if (path >= pathCount || pathDraws[path] < 2u)
+        return;
+    const PathCells c = cells[path];
+    const uint32_t nCells = grid_cells(c);
+    for (uint32_t i = threadIdx.x; i <= nCells; i += blockDim.x)
+    {
+        packed[c.base + i] = make_uint2(0u, 0u);
+        cellCursor[c.base + i] = 0u;
+    }
+}
+
+__global__ __launch_bounds__(256) void shared_count_kernel(const Prim* __restrict__ prims,
+                                                           const DrawTess* __restrict__ draws,
+                                                           const PathCells* __restrict__ cells,
+                                                           const uint32_t* __restrict__ pathDraws,
+                                                           uint2* __restrict__ packed)
+{
+    const DrawTess d = draws[blockIdx.x];
+    if (d.pathID == 0u || d.forwardCount == 0u || pathDraws[d.pathID] < 2u)
+        return;
+    const PathCells c = cells[d.pathID];
+    uint2* grid = packed + c.base;
     for (uint32_t k = threadIdx.x; k < d.forwardCount; k += blockDim.x)
     {
         const Prim p = prims[d.primBase + k];
         if (p.flags & kPrimEmpty)
             continue;
-        if (local)
-        {
-            for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&sCell[cell], 1u); });
-            for_prim_crossings(p, c, [&](uint32_t cell, int v) { atomicAdd(&sCell[cell], (uint32_t)v << 16); });
-        }
-        else
-        {
-            for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&gCount[cell], 1u); });
-            for_prim_crossings(p, c, [&](uint32_t cell, int v) { atomicAdd(&gBack[cell], v); });
-        }
-    }
-    if (local)
-    {
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < nCells; i += blockDim.x)
-        {
-            const uint32_t w = sCell[i];
-            if ((w & 0xffffu) != 0)
-                atomicAdd(&gCount[i], w & 0xffffu);
-            if ((w >> 16) != 0)
-                atomicAdd(&gBack[i], (int32_t)w >> 16);
-        }
+        for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&grid[cell].x, 1u); });
+        for_prim_crossings(p, c, [&](uint32_t cell, int v) { atomicAdd(&grid[cell].y, (uint32_t)v); });
     }
 }
 
-// Writes each primitive index into its cells' bins.  A path binned by this
-// draw alone owns its cells' ranges, so LDS cursors from 0 hand out slots
-// after the cell offsets; a path shared by several draws counts in LDS,
-// reserves once per cell on the global cursors, then hands out slots.
-__global__ __launch_bounds__(256) void bin_scatter_draw_kernel(const Prim* __restrict__ prims,
-                                                               const DrawTess* __restrict__ draws,
-                                                               const PathCells* __restrict__ cells,
-                                                               const uint32_t* __restrict__ cellOffset,
-                                                               uint32_t* __restrict__ cellCursor,
-                                                               const uint32_t* __restrict__ pathDraws,
-                                                               uint32_t* __restrict__ binned)
+__global__ __launch_bounds__(256) void shared_layout_kernel(const PathCells* __restrict__ cells, uint32_t pathCount,
+                                                            const uint32_t* __restrict__ pathDraws,
+                                                            uint2* __restrict__ packed,
+                                                            uint32_t* __restrict__ pathBins)
 {
-    __shared__ uint32_t sCur[kBinLdsCells];
+    __shared__ uint32_t sWaveSum[4];
+    const uint32_t path = blockIdx.x;
+    if (path >= pathCount || pathDraws[path] < 2u)
+        return;
+    const PathCells c = cells[path];
+    const uint32_t nCells = grid_cells(c), rows = nCells != 0u ? (uint32_t)(c.ty1 - c.ty0) : 0u;
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = threadIdx.x >> 6;
+    uint2* grid = packed + c.base;
+    for (uint32_t r = wave; r < rows; r += 4u)
+    {
+        int32_t carry = 0;
+        for (uint32_t x0 = 0; x0 < c.width; x0 += 64)
+        {
+            const uint32_t x = x0 + (uint32_t)lane;
+            const int32_t v = wave_scan_add(x < c.width ? (int32_t)grid[r * c.width + x].y : 0, lane) + carry;
+            if (x < c.width)
+                grid[r * c.width + x].y = (uint32_t)v;
+            carry = __shfl(v, 63);
+        }
+    }
+    // counts -> offsets, 256 cells per step; a total beyond 2^32-1 saturates
+    // and the host rejects the flush
+    uint64_t carry = 0;
+    for (uint32_t i0 = 0; i0 < nCells; i0 += 256u)
+    {
+        const uint32_t i = i0 + threadIdx.x;
+        const uint32_t v = i < nCells ? grid[i].x : 0u;
+        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)v, lane);
+        if (lane == 63)
+            sWaveSum[wave] = incl;
+        __syncthreads();
+        uint32_t pre = 0, step = 0;
+        for (uint32_t w = 0; w < 4u; ++w)
+        {
+            pre += w < wave ? sWaveSum[w] : 0u;
+            step += sWaveSum[w];
+        }
+        if (i < nCells)
+            grid[i].x = (uint32_t)carry + pre + incl - v;
+        carry += step;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+    {
+        const uint32_t total = (uint32_t)min(carry, (uint64_t)0xffffffffu);
+        grid[nCells] = make_uint2(total, 0u);
+        pathBins[path] = total;
+    }
+}
+
+__global__ __launch_bounds__(256) void shared_scatter_kernel(const Prim* __restrict__ prims,
+                                                             const DrawTess* __restrict__ draws,
+                                                             const PathCells* __restrict__ cells,
+                                                             const uint32_t* __restrict__ pathDraws,
+                                                             const uint2* __restrict__ packed,
+                                                             const uint32_t* __restrict__ pathBase,
+                                                             uint32_t* __restrict__ cellCursor,
+                                                             uint32_t* __restrict__ binned)
+{
     const DrawTess d = draws[blockIdx.x];
-    if (d.pathID == 0 || d.forwardCount == 0)
+    if (d.pathID == 0u || d.forwardCount == 0u || pathDraws[d.pathID] < 2u)
         return;
     const PathCells c = cells[d.pathID];
-    const uint32_t nCells = grid_cells(c);
-    if (nCells == 0)
-        return;
-    const uint32_t* gOffset = cellOffset + c.base;
-    uint32_t* gCursor = cellCursor + c.base;
-    if (nCells > kBinLdsCells)
-    {
-        for (uint32_t k = threadIdx.x; k < d.forwardCount; k += blockDim.x)
-        {
-            const uint32_t g = d.primBase + k;
-            const Prim p = prims[g];
-            if (p.flags & kPrimEmpty)
-                continue;
-            for_prim_cells(p, c, [&](uint32_t cell) { binned[gOffset[cell] + atomicAdd(&gCursor[cell], 1u)] = g; });
-        }
-        return;
-    }
-    if (pathDraws[d.pathID] == 1u)
-    {
-        // the cursors start at the cells' bin offsets (read once, coalesced)
-        for (uint32_t i = threadIdx.x; i < nCells; i += blockDim.x)
-            sCur[i] = gOffset[i];
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < d.forwardCount; k += blockDim.x)
-        {
-            const uint32_t g = d.primBase + k;
-            const Prim p = prims[g];
-            if (!(p.flags & kPrimEmpty))
-                for_prim_cells(p, c, [&](uint32_t cell) { binned[atomicAdd(&sCur[cell], 1u)] = g; });
-        }
-        return;
-    }
-    for (uint32_t i = threadIdx.x; i < nCells; i += blockDim.x)
-        sCur[i] = 0;
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < d.forwardCount; k += blockDim.x)
-    {
-        const Prim p = prims[d.primBase + k];
-        if (!(p.flags & kPrimEmpty))
-            for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&sCur[cell], 1u); });
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nCells; i += blockDim.x)
-        if (sCur[i] != 0)
-            sCur[i] = gOffset[i] + atomicAdd(&gCursor[i], sCur[i]);
-    __syncthreads();
+    const uint32_t base = pathBase[d.pathID];
+    const uint2* grid = packed + c.base;
+    uint32_t* cursor = cellCursor + c.base;
     for (uint32_t k = threadIdx.x; k < d.forwardCount; k += blockDim.x)
     {
         const uint32_t g = d.primBase + k;
         const Prim p = prims[g];
         if (!(p.flags & kPrimEmpty))
-            for_prim_cells(p, c, [&](uint32_t cell) { binned[atomicAdd(&sCur[cell], 1u)] = g; });
-    }
-}
-
-// Each cell's first bin and corner winding side by side, so the raster reads
-// one 8-byte entry (and the next entry's offset for the count) per
-// (path, tile) instead of two arrays.
-// Prefix-sum of corner crossings along each row of each path's grid: one
-// wave64 per (path, row), 64 cells per step with a carried running sum.  Each
-// cell's result goes out with its bin offset as the raster's packed
-// (offset, corner winding) entry; entry totalCells is the end sentinel.
-__global__ __launch_bounds__(256) void backdrop_prefix_kernel(const PathCells* __restrict__ cells,
-                                                              uint32_t pathCount, int maxRows,
-                                                              const int32_t* __restrict__ cellBackdrop,
-                                                              const uint32_t* __restrict__ cellOffset,
-                                                              uint32_t totalCells, uint2* __restrict__ packed)
-{
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        packed[totalCells] = make_uint2(cellOffset[totalCells], 0u);
-    if (maxRows <= 0)
-        return;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    const uint32_t path = wave / (uint32_t)maxRows;
-    const int row = (int)(wave % (uint32_t)maxRows);
-    if (path >= pathCount)
-        return;
-    const PathCells c = cells[path];
-    if (row >= c.ty1 - c.ty0)
-        return;
-    const uint32_t rowBase = c.base + (uint32_t)row * c.width;
-    const int32_t* r = cellBackdrop + rowBase;
-    int32_t carry = 0;
-    for (uint32_t x0 = 0; x0 < c.width; x0 += 64)
-    {
-        const uint32_t x = x0 + (uint32_t)lane;
-        int32_t v = x < c.width ? r[x] : 0;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1)
-        {
-            const int32_t t = __shfl_up(v, d);
-            if (lane >= d)
-                v += t;
-        }
-        if (x < c.width)
-            packed[rowBase + x] = make_uint2(cellOffset[rowBase + x], (uint32_t)(carry + v));
-        carry += __shfl(v, 63);
+            for_prim_cells(p, c, [&](uint32_t cell) { binned[base + grid[cell].x + atomicAdd(&cursor[cell], 1u)] = g; });
     }
 }
 
@@ -3211,7 +3322,8 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const uint32_t* __restr
 template <bool FEATHER, bool PERSISTENT, int WAVES>
 __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
     const PathCells* __restrict__ cells, const PathRaster* __restrict__ raster,
-    const PathPaint* __restrict__ pathPaint, const uint2* __restrict__ cellPacked, const uint32_t* __restrict__ binned, const Prim* __restrict__ prims,
+    const PathPaint* __restrict__ pathPaint, const uint2* __restrict__ cellPacked,
+    const uint32_t* __restrict__ pathBase, const uint32_t* __restrict__ binned, const Prim* __restrict__ prims,
     const uint32_t* __restrict__ ramps, uint32_t gradHeight, const ImageDesc* __restrict__ images,
     const CanvasDev* __restrict__ canvases, uint32_t canvasCount, uint32_t dither,
     const float* __restrict__ featherTable, const uint32_t* __restrict__ tileOrder, uint32_t tileTotal,
@@ -3302,8 +3414,8 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                 {
                     const uint32_t cell = c.base + (uint32_t)(ty - c.ty0) * c.width + (uint32_t)(tx - c.tx0);
                     const uint2 here = cellPacked[cell];
-                    off = here.x;
-                    n = cellPacked[cell + 1].x - off;
+                    n = cellPacked[cell + 1].x - here.x;
+                    off = here.x + pathBase[p];
                     C = (int32_t)here.y;
                     // A path with no primitives here covers the tile with its corner
                     // winding's coverage; when that is zero it draws nothing, and a
