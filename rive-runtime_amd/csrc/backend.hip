@@ -119,6 +119,9 @@ struct rive_hip_context
     // the raster's tile order: cost class per tile, the order, and the
     // class histogram, class cursors and tile queue head (2 * 256 + 1 words)
     DevBuf tileClass, tileOrder, tileQueue;
+    // the last path hiding everything before it in each tile, and how far back
+    // each 64 paths' clip reads reach
+    DevBuf tileCover, clipFirst;
     rive_hip_raster_config rasterConfig = {0u, 0u, 6u, 0u};
     bool interiorTriangulation = false; // the front end's layout of large fills
     int cuCount = 256;
@@ -189,7 +192,7 @@ struct rive_hip_context
 namespace
 {
 // The scratch buffers of a context (every DevBuf member), in one list.
-constexpr int kDevBufCount = 39;
+constexpr int kDevBufCount = 41;
 // The device scalars of a flush (totals, counters), 32 words: the pipeline
 // uses slots 0-7, device counting 8-13, guard-box pieces kFarSlot .. +3.
 constexpr size_t kScalarBytes = 128;
@@ -206,7 +209,7 @@ void devbufs(rive_hip_context* c, DevBuf** out)
                                  &c->pathCanvas, &c->cellPacked, &c->pathDraws, &c->pathPaint,
                                  &c->patchTable, &c->patchWork, &c->specialList, &c->farList, &c->drawPieces,
                                  &c->drawPieceOffset, &c->pieceCursor, &c->drawTessAll, &c->tileClass,
-                                 &c->tileOrder, &c->tileQueue};
+                                 &c->tileOrder, &c->tileQueue, &c->tileCover, &c->clipFirst};
     for (int i = 0; i < kDevBufCount; ++i)
         out[i] = all[i];
 }
@@ -1365,6 +1368,14 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
     RIVE_TRY(clear(ctx, ctx->pathCanvas.ptr, 0xff, (size_t)(pathCount + 1) * 4));
     path_canvas_kernel<<<canvasCount, 256, 0, ctx->stream>>>(P<CanvasDev>(ctx->canvasTable),
                                                              P<uint32_t>(ctx->pathCanvas));
+    RIVE_TRY(ensure(ctx, ctx->pathRaster, (size_t)(pathCount + 1) * sizeof(PathRaster)));
+    RIVE_TRY(ensure(ctx, ctx->pathPaint, (size_t)(pathCount + 1) * sizeof(PathPaint)));
+    RIVE_TRY(ensure(ctx, ctx->clipFirst, ((size_t)pathCount / 64 + 1) * 4));
+    path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
+        paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, gradRows, P<PathRaster>(ctx->pathRaster),
+        P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->clipFirst));
+    RIVE_TRY(ensure(ctx, ctx->tileCover, (size_t)std::max<uint32_t>(tileTotal, 1) * 4));
+    RIVE_TRY(clear(ctx, ctx->tileCover.ptr, 0, (size_t)tileTotal * 4));
     RIVE_TRY(ensure(ctx, ctx->cells, (size_t)(pathCount + 1) * sizeof(PathCells)));
     cells_init_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(P<PathCells>(ctx->cells),
                                                                              pathCount + 1);
@@ -1459,11 +1470,13 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
     {
         bin_count_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
             P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
-            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins));
+            P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), P<CanvasDev>(ctx->canvasTable),
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
         if (largeCells > smallCells)
             bin_count_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
                 P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
-                largeCells, P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins));
+                largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), P<CanvasDev>(ctx->canvasTable),
+                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
     }
     if (bin && shared)
     {
@@ -1496,22 +1509,21 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
     {
         bin_scatter_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
             P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
-            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+            P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), P<CanvasDev>(ctx->canvasTable),
+            P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
+            P<uint32_t>(ctx->binned));
         if (largeCells > smallCells)
             bin_scatter_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
                 P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
-                largeCells, P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+                largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), P<CanvasDev>(ctx->canvasTable),
+                P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
+                P<uint32_t>(ctx->binned));
     }
     if (bin && shared)
         shared_scatter_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
             P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws),
             P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->cellCursor),
             P<uint32_t>(ctx->binned));
-    RIVE_TRY(ensure(ctx, ctx->pathRaster, (size_t)(pathCount + 1) * sizeof(PathRaster)));
-    RIVE_TRY(ensure(ctx, ctx->pathPaint, (size_t)(pathCount + 1) * sizeof(PathPaint)));
-    path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
-        paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, gradRows, P<PathRaster>(ctx->pathRaster),
-        P<PathPaint>(ctx->pathPaint));
     HIP_TRY(hipGetLastError());
     RIVE_TRY(mark(ctx, ctx->ev[4]));
 
@@ -1536,7 +1548,7 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
             RIVE_TRY(ensure(ctx, ctx->tileOrder, (size_t)tileTotal * 4));
             tile_cost_kernel<<<(tileTotal + 3) / 4, 256, 0, ctx->stream>>>(
                 P<PathCells>(ctx->cells), P<uint2>(ctx->cellPacked), P<CanvasDev>(ctx->canvasTable), canvasCount,
-                tileTotal, P<uint32_t>(ctx->tileClass), queue);
+                tileTotal, P<uint32_t>(ctx->tileCover), P<uint32_t>(ctx->tileClass), queue);
             tile_order_kernel<<<(tileTotal + 255) / 256, 256, 0, ctx->stream>>>(
                 P<uint32_t>(ctx->tileClass), queue, queue + kCostClasses, tileTotal, P<uint32_t>(ctx->tileOrder));
             order = P<uint32_t>(ctx->tileOrder);
@@ -1551,7 +1563,7 @@ int raster_pipeline(rive_hip_context* ctx, const rive_hip_flush_desc* d, const S
             P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
             P<uint32_t>(ctx->binned), P<Prim>(ctx->prims),
             P<uint32_t>(ctx->ramps), gradRows, P<ImageDesc>(ctx->imageTable), P<CanvasDev>(ctx->canvasTable),
-            canvasCount, d->dither, ctx->featherTables, order, tileTotal, queue + 2 * kCostClasses);
+            canvasCount, P<uint32_t>(ctx->tileCover), P<uint32_t>(ctx->clipFirst), d->dither, ctx->featherTables, order, tileTotal, queue + 2 * kCostClasses);
     }
     HIP_TRY(hipGetLastError());
     RIVE_TRY(mark(ctx, ctx->ev[5]));
