@@ -400,9 +400,12 @@ int rive_hip_last_frame(rive_hip_context* ctx, rive_hip_flush_desc* out, uint32_
  * DRAW records follow each other (descs[k].first_draw = descs[k-1].first_draw
  * + descs[k-1].draw_count, at most 64 flushes), their curve counting, layout
  * scans, record emission and span writing run once for the whole frame --
- * each flush still laid out on its own from location 8 and contour ID 1 --
- * and only the per-flush passes (tessellation, binning, raster) run per
- * flush.  Replaces the per-logical-flush RenderContextImpl::flush calls of
+ * each flush still laid out on its own from location 8 and contour ID 1.
+ * Where their other records follow each other too (as the reference and the
+ * front end write them) and the later flushes load the target, all passes run
+ * once for the whole frame, in device buffers of up to 32 GiB beside the
+ * bins; a larger frame, or one that does not get the memory, runs them for
+ * parts of it or flush by flush.  Replaces the per-logical-flush RenderContextImpl::flush calls of
  * one RenderContext::flush (render_context.cpp:971-1018).
  * rive_hip_pass_times then sums over the frame's flushes. */
 int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n);
@@ -487,8 +490,7 @@ uint32_t rive_hip_get_interior_triangulation(const rive_hip_context* ctx);
  * `trials` (1..64) times under each of RIVE_HIP_RASTER_CANDIDATES raster
  * configs -- tile_order x persistent x waves_per_simd, in the order
  * {0,0,6} {0,0,5} {0,1,6} {0,1,5} {1,0,6} {1,0,5} {1,1,6} {1,1,5} -- times
- * each flush's raster pass with the context's HIP events (a trial runs the
- * flushes one by one), and keeps the config of the
+ * the frame's raster passes with the context's HIP events, and keeps the config of the
  * smallest median on the context.  The frame's targets are saved before and
  * restored after, so their pixels are as they were.  out (may be null) gets
  * the chosen config, times_ms (may be null, RIVE_HIP_RASTER_CANDIDATES

@@ -992,10 +992,21 @@ __global__ void frame_padding_kernel(SpanV* __restrict__ spans, const FrameBound
 
 namespace
 {
+// One logical flush's layout from the counting pass.
+struct GeoLayout
+{
+    const rivehip::SpanV* spans;
+    uint32_t spanCount;
+    const rivehip::ContourV* contours;
+    uint32_t contourCount;
+    uint32_t recordCount;
+    uint32_t texelsUsed; // incl. the 8 + 1 padding texels
+    uint32_t tessRows;
+};
+
 // GEOMETRY-mode front half: count -> scan -> emit -> spans.  Leaves spans and
 // contours in ctx scratch and the tessellation ranges in the DRAW buffer.
-int geometry_counting(rive_hip_context* ctx, const rive_hip_flush_desc* d, const rivehip::SpanV** spans,
-                      uint32_t* spanCount, const rivehip::ContourV** contours, uint32_t* tessRows)
+int geometry_counting(rive_hip_context* ctx, const rive_hip_flush_desc* d, GeoLayout* out)
 {
     using namespace rivehip;
     const uint32_t n = d->draw_count;
@@ -1086,31 +1097,19 @@ int geometry_counting(rive_hip_context* ctx, const rive_hip_flush_desc* d, const
     HIP_TRY(hipGetLastError());
     RIVE_TRY(mark(ctx, ctx->ev[1]));
     const uint32_t texelsUsed = firstLocation + tessTotal + 1u;
-    *tessRows = std::max<uint32_t>((texelsUsed + kTessTextureWidth - 1) / kTessTextureWidth, 1);
-    *spans = P<SpanV>(ctx->geoSpans);
-    *spanCount = allSpans;
-    *contours = P<ContourV>(ctx->geoContours);
-    ctx->lastContourCount = contourTotal;
-    ctx->lastRecordCount = recordTotal;
-    ctx->lastTessVertexCount = texelsUsed;
+    out->spans = P<SpanV>(ctx->geoSpans);
+    out->spanCount = allSpans;
+    out->contours = P<ContourV>(ctx->geoContours);
+    out->contourCount = contourTotal;
+    out->recordCount = recordTotal;
+    out->texelsUsed = texelsUsed;
+    out->tessRows = std::max<uint32_t>((texelsUsed + kTessTextureWidth - 1) / kTessTextureWidth, 1);
     return RIVE_HIP_OK;
 }
 } // namespace
 
 namespace
 {
-// One logical flush's layout from a frame's counting pass.
-struct GeoLayout
-{
-    const rivehip::SpanV* spans;
-    uint32_t spanCount;
-    const rivehip::ContourV* contours;
-    uint32_t contourCount;
-    uint32_t recordCount;
-    uint32_t texelsUsed; // incl. the 8 + 1 padding texels
-    uint32_t tessRows;
-};
-
 // GEOMETRY-mode front half for several logical flushes whose draws are
 // contiguous in the DRAW buffer (descs[k].first_draw follow each other):
 // one counting launch, frame-wide scans, one emission launch and one span

@@ -160,7 +160,8 @@ struct PathCells
     int32_t tx0, ty0, tx1, ty1; // [tx0, tx1) x [ty0, ty1); empty if tx0 >= tx1
     uint32_t base;              // first cell index
     uint32_t width;             // tx1 - tx0
-    uint32_t pad[2];
+    uint32_t flushStart;        // the reserved record of a launch's second or later flush
+    uint32_t pad;
 };
 
 // One canvas of a flush: its target, tile grid and path range.  Tiles of all
@@ -176,12 +177,28 @@ struct CanvasDev
 };
 static_assert(sizeof(CanvasDev) == 48, "CanvasDev layout");
 
+// One logical flush of a launch.  A frame's flushes run together (each pass
+// once for all of them): their records follow each other in the mapped
+// buffers, path p of the launch is path ID p - pathBase of its flush, and
+// everything a flush numbers on its own (texels, contours, ramp rows, images)
+// starts at its bases here.  A launch of one flush has all bases zero.
+struct FlushDev
+{
+    uint32_t texBase, texels;           // tessellation texels, whole rows
+    uint32_t contourBase, contourCount; // ContourData records
+    uint32_t pathBase, pathCount;       // the flush's reserved record 0; live path IDs 1..pathCount
+    uint32_t gradRowBase, gradRows;     // ramp rows
+    uint32_t imageBase, imageCount;     // image table entries
+    uint32_t spanBase, drawBase, gradSpanBase;
+    uint32_t pad;
+};
+
 // One draw's tessellation range (the reference's DrawBatch, gpu.hpp).
 struct DrawTess
 {
     uint32_t pathID;
     uint32_t tessLocation;    // first texel of the draw's allocation
-    uint32_t tessVertexCount; // both directions
+    uint32_t flush;           // index into the launch's FlushDev table
     uint32_t dirs;            // ContourDirections
     uint32_t isStroke;
     uint32_t forwardBase;     // first forward texel

@@ -41,21 +41,38 @@ __device__ __forceinline__ int32_t clamp_thr(int64_t t)
     return (int32_t)(t < -lim ? -lim : (t > lim ? lim : t));
 }
 
+// The flush owning record i: the last one whose field `first` is at or before i.
+template <uint32_t FlushDev::* FIRST>
+__device__ __forceinline__ uint32_t flush_of(const FlushDev* __restrict__ flushes, uint32_t n, uint32_t i)
+{
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1)
+    {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (flushes[mid].*FIRST <= i)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
 // ---------------------------------------------------------------------------
 // Color ramps (color_ramp.glsl:40-106).  One block per GradientSpan.
 // ---------------------------------------------------------------------------
-__global__ void ramp_kernel(const uint4* __restrict__ spans, uint32_t spanCount, uint32_t rows,
-                            uint32_t* __restrict__ ramps)
+__global__ void ramp_kernel(const uint4* __restrict__ spans, uint32_t spanCount,
+                            const FlushDev* __restrict__ flushes, uint32_t flushCount, uint32_t* __restrict__ ramps)
 {
     const uint32_t s = blockIdx.x;
     if (s >= spanCount)
         return;
+    const FlushDev fl = flushes[flush_of<&FlushDev::gradSpanBase>(flushes, flushCount, s)];
     uint4 gs = spans[s];
     float x0 = float(gs.x & 0xffffu) * (1.f / 65536.f);
     float x1 = float(gs.x >> 16) * (1.f / 65536.f);
     uint32_t yflags = gs.y;
     uint32_t y = yflags & ~GRAD_SPAN_FLAGS_MASK;
-    if (y >= rows)
+    if (y >= fl.gradRows)
         return;
     float left = x0, right = x1;
     if (yflags & GRAD_SPAN_FLAG_LEFT_BORDER)
@@ -102,7 +119,7 @@ __global__ void ramp_kernel(const uint4* __restrict__ spans, uint32_t spanCount,
             float v = fminf(fmaxf(c[k], 0.f), 1.f);
             px |= (uint32_t)floorf(v * 255.f + .5f) << (8 * k);
         }
-        ramps[(size_t)y * kGradWidth + x] = px;
+        ramps[(size_t)(fl.gradRowBase + y) * kGradWidth + x] = px;
     }
 }
 
@@ -130,7 +147,8 @@ __device__ __forceinline__ void span_first_rect(const SpanV& s, int32_t* lo, int
 }
 
 __global__ void span_texel_count_kernel(const SpanV* __restrict__ spans, uint32_t n,
-                                        uint32_t rows, uint32_t* __restrict__ counts)
+                                        const FlushDev* __restrict__ flushes, uint32_t flushCount,
+                                        uint32_t* __restrict__ counts)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
@@ -138,6 +156,7 @@ __global__ void span_texel_count_kernel(const SpanV* __restrict__ spans, uint32_
     SpanV s = spans[i];
     int32_t lo, hi, x0, x1;
     span_first_rect(s, &lo, &hi, &x0, &x1);
+    const uint32_t rows = flushes[flush_of<&FlushDev::spanBase>(flushes, flushCount, i)].texels / kTessTextureWidth;
     uint32_t c = 0;
     if (s.y >= 0.f && s.y < float(rows) && hi > lo)
         c = (uint32_t)(hi - lo);
@@ -287,8 +306,8 @@ __device__ void soften_feathered_cubic(F2 p0, F2* p1, F2* p2, F2 p3, float feath
 __global__ void tessellate_kernel(const SpanV* __restrict__ spans, uint32_t spanCount,
                                   const uint32_t* __restrict__ texelOffsets, uint32_t totalTexels,
                                   TessTexel* __restrict__ tex, const uint4* __restrict__ contours,
-                                  uint32_t contourCount, const float* __restrict__ pathData, uint32_t pathCount,
-                                  const float* __restrict__ featherTables)
+                                  const float* __restrict__ pathData, const FlushDev* __restrict__ flushes,
+                                  uint32_t flushCount, const float* __restrict__ featherTables)
 {
     constexpr float PI_ = 3.14159265359f;
     constexpr float TWO_PI = 6.28318530718f;
@@ -306,6 +325,10 @@ __global__ void tessellate_kernel(const SpanV* __restrict__ spans, uint32_t span
             hi = mid;
     }
     const SpanV s = spans[lo];
+    const FlushDev fl = flushes[flush_of<&FlushDev::spanBase>(flushes, flushCount, lo)];
+    contours += fl.contourBase;
+    pathData += (size_t)fl.pathBase * 16;
+    const uint32_t contourCount = fl.contourCount, pathCount = fl.pathCount;
     int32_t rlo, rhi, x0, x1;
     span_first_rect(s, &rlo, &rhi, &x0, &x1);
     const int32_t x = rlo + (int32_t)(g - texelOffsets[lo]);
@@ -497,7 +520,7 @@ __global__ void tessellate_kernel(const SpanV* __restrict__ spans, uint32_t span
     else
         o.z = f2u(theta - TWO_PI * floorf(theta / TWO_PI));
     o.w = cf;
-    tex[(size_t)row * kTessTextureWidth + (uint32_t)x] = o;
+    tex[fl.texBase + (size_t)row * kTessTextureWidth + (uint32_t)x] = o;
 }
 
 // ---------------------------------------------------------------------------
@@ -896,15 +919,18 @@ __device__ __forceinline__ uint32_t find_draw_block(const DrawTess* __restrict__
 
 // Vertex stage once per forward texel (draw_path_common.glsl:275-789); the
 // segment between texel i and next(i) reuses both ends.
-__global__ void vertex_kernel(const TessTexel* __restrict__ tex, int texels, const PathDataV* __restrict__ paths,
-                              const DrawTess* __restrict__ draws, uint32_t drawCount, uint32_t totalPrims,
-                              VtxPair* __restrict__ verts)
+__global__ void vertex_kernel(const TessTexel* __restrict__ tex, const FlushDev* __restrict__ flushes,
+                              const PathDataV* __restrict__ paths, const DrawTess* __restrict__ draws, uint32_t drawCount,
+                              uint32_t totalPrims, VtxPair* __restrict__ verts)
 {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t di = find_draw_block(draws, drawCount, g);
     if (g >= totalPrims)
         return;
     const DrawTess d = draws[di];
+    const FlushDev fl = flushes[d.flush];
+    tex += fl.texBase;
+    const int texels = (int)fl.texels;
     const int i = min((int)(d.forwardBase + (g - d.primBase)), texels - 2);
     const PathDataV pd = paths[d.pathID];
     if (pd.featherRadius != 0.f && pd.strokeRadius == 0.f)
@@ -1206,8 +1232,8 @@ __global__ void piece_draws_kernel(const DrawTess* __restrict__ draws, uint32_t 
     out[drawCount + i] = d;
 }
 
-__global__ void expand_kernel(const TessTexel* __restrict__ tex, int texels, const VtxPair* __restrict__ verts,
-                              const ContourV* __restrict__ contours, uint32_t contourCount,
+__global__ void expand_kernel(const TessTexel* __restrict__ tex, const FlushDev* __restrict__ flushes,
+                              const VtxPair* __restrict__ verts, const ContourV* __restrict__ contours,
                               const PathDataV* __restrict__ paths, const DrawTess* __restrict__ draws,
                               uint32_t drawCount, uint32_t totalPrims, Prim* __restrict__ prims,
                               PathCells* __restrict__ cells, uint32_t* __restrict__ badContours,
@@ -1218,6 +1244,11 @@ __global__ void expand_kernel(const TessTexel* __restrict__ tex, int texels, con
     if (g >= totalPrims)
         return;
     const DrawTess d = draws[di];
+    const FlushDev fl = flushes[d.flush];
+    tex += fl.texBase;
+    contours += fl.contourBase;
+    const int texels = (int)fl.texels;
+    const uint32_t contourCount = fl.contourCount;
     // A reverse-only draw (a feathered fill through the atlas under a
     // left-handed matrix) holds its contours back to front: read it from the
     // end, so each segment is its forward one.
@@ -1454,9 +1485,9 @@ __global__ void expand_kernel(const TessTexel* __restrict__ tex, int texels, con
 // moves to the contour's midpoint, its fan triangles being dropped), and a
 // primitive still leaving the box is counted for its pieces.  Its path's
 // bounds take the primitive clamped onto the box.
-__global__ void special_prims_kernel(const TessTexel* __restrict__ tex, int texels,
-                                     const ContourV* __restrict__ contours, uint32_t contourCount,
-                                     const PathDataV* __restrict__ paths, const DrawTess* __restrict__ draws,
+__global__ void special_prims_kernel(const TessTexel* __restrict__ tex, const FlushDev* __restrict__ flushes,
+                                     const ContourV* __restrict__ contours, const PathDataV* __restrict__ paths,
+                                     const DrawTess* __restrict__ draws,
                                      uint32_t drawCount, Prim* __restrict__ prims, PathCells* __restrict__ cells,
                                      const uint32_t* __restrict__ specialList,
                                      const uint32_t* __restrict__ specialCount, uint32_t* __restrict__ farList,
@@ -1477,10 +1508,11 @@ __global__ void special_prims_kernel(const TessTexel* __restrict__ tex, int texe
             anyBad |= out.p[c] == kSnapInvalid;
         if (anyBad && !stroke && !(flags & kPrimNoEdge))
         {
+            const FlushDev fl = flushes[d.flush];
             const int i = d.dirs == 1u ? max((int)(d.forwardBase + d.forwardCount - 1u - (g - d.primBase)), 1)
-                                       : min((int)(d.forwardBase + (g - d.primBase)), texels - 2);
-            const uint32_t cid = min(max(tex[i].w & CONTOUR_ID_MASK, 1u), max(contourCount, 1u));
-            const ContourV cd = contours[cid - 1];
+                                       : min((int)(d.forwardBase + (g - d.primBase)), (int)fl.texels - 2);
+            const uint32_t cid = min(max(tex[fl.texBase + i].w & CONTOUR_ID_MASK, 1u), max(fl.contourCount, 1u));
+            const ContourV cd = contours[fl.contourBase + cid - 1];
             const PathDataV pd = paths[d.pathID];
             const float fx = (pd.m[0] * cd.mx + pd.m[2] * cd.my) + 0.f + pd.m[4];
             const float fy = (pd.m[1] * cd.mx + pd.m[3] * cd.my) + 0.f + pd.m[5];
@@ -1535,7 +1567,8 @@ __global__ void special_prims_kernel(const TessTexel* __restrict__ tex, int texe
 // ---------------------------------------------------------------------------
 // Per-path cell grids.
 // ---------------------------------------------------------------------------
-__global__ void cells_init_kernel(PathCells* __restrict__ cells, uint32_t n)
+__global__ void cells_init_kernel(PathCells* __restrict__ cells, uint32_t n, const FlushDev* __restrict__ flushes,
+                                  uint32_t flushCount)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
@@ -1545,7 +1578,9 @@ __global__ void cells_init_kernel(PathCells* __restrict__ cells, uint32_t n)
     c.tx1 = c.ty1 = -0x7fffffff;
     c.base = 0;
     c.width = 0;
-    c.pad[0] = c.pad[1] = 0;
+    // the reserved record of a flush after the launch's first marks its start
+    c.flushStart = i != 0u && flushes[flush_of<&FlushDev::pathBase>(flushes, flushCount, i)].pathBase == i ? 1u : 0u;
+    c.pad = 0;
     cells[i] = c;
 }
 
@@ -1638,6 +1673,9 @@ constexpr uint32_t kPaintNoOp = 1u << 22;
 // A kPaintPlain fill of alpha 1: where its coverage is 1 the pixel becomes its
 // color whatever was drawn before.
 constexpr uint32_t kPaintOpaque = 1u << 23;
+// The reserved record of a flush after the launch's first: the clip buffer
+// starts empty there, since each flush numbers its clip IDs from 1.
+constexpr uint32_t kPaintFlushStart = 1u << 24;
 
 // Coverage of a winding count under the path's fill rule (draw_path.frag
 // fill-rule resolution): clockwise clamps the signed count to [0, 1], nonzero
@@ -3050,8 +3088,7 @@ __device__ __forceinline__ uint32_t pack_unorm8x4(const float* v)
 
 // Gradient paint color, unpremultiplied, 0..255 scale (draw_path.vert:285-331,450-476).
 __device__ __forceinline__ void sample_gradient255(const PathRaster& pr, int px, int py,
-                                                   const uint32_t* __restrict__ ramps, uint32_t gradHeight,
-                                                   float* src)
+                                                   const uint32_t* __restrict__ ramps, float* src)
 {
     const float fx = float(px) + .5f, fy = float(py) + .5f;
     const float pcx = pr.paintMatrix[0] * fx + pr.paintMatrix[2] * fy + pr.paintMatrix[4];
@@ -3063,7 +3100,7 @@ __device__ __forceinline__ void sample_gradient255(const PathRaster& pr, int px,
     const int i0 = (int)floorf(tc);
     const float fr = tc - (float)i0;
     const int ia = min(max(i0, 0), 511), ib = min(max(i0 + 1, 0), 511);
-    const uint32_t* rowp = ramps + (size_t)min(pr.gradRow, gradHeight - 1) * kGradWidth;
+    const uint32_t* rowp = ramps + (size_t)pr.gradRow * kGradWidth;
     const uint32_t ta = rowp[ia], tb = rowp[ib];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -3078,7 +3115,7 @@ __device__ __forceinline__ void sample_gradient255(const PathRaster& pr, int px,
 // draw_raster_order_path.frag:191-204), in 0..1 scale.
 __device__ __noinline__ uint32_t resolve_general(const PathRaster* __restrict__ prp, float coverage, int px,
                                                  int py, float noise255, const uint32_t* __restrict__ ramps,
-                                                 uint32_t gradHeight, const ImageDesc* __restrict__ images,
+                                                 const ImageDesc* __restrict__ images,
                                                  uint32_t colPacked)
 {
     const PathRaster pr = *prp;
@@ -3103,7 +3140,7 @@ __device__ __noinline__ uint32_t resolve_general(const PathRaster* __restrict__ 
     }
     else
     {
-        sample_gradient255(pr, px, py, ramps, gradHeight, src);
+        sample_gradient255(pr, px, py, ramps, src);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             src[k] *= 1.f / 255.f;
@@ -3189,7 +3226,7 @@ __device__ __forceinline__ float clip_rect_coverage(const float* m, int px, int 
 
 __device__ __forceinline__ void resolve_pixel(const PathPaint& pp, const PathRaster* __restrict__ prp,
                                               float coverage, int px, int py, float noise255,
-                                              const uint32_t* __restrict__ ramps, uint32_t gradHeight,
+                                              const uint32_t* __restrict__ ramps,
                                               const ImageDesc* __restrict__ images, uint32_t& colPacked,
                                               uint32_t& clip)
 {
@@ -3209,7 +3246,7 @@ __device__ __forceinline__ void resolve_pixel(const PathPaint& pp, const PathRas
         coverage = fminf(fmaxf(clip_rect_coverage(prp->clipRect, px, py), 0.f), coverage);
     if ((flags & 0xf00u) != 0u || (pp.kind & kPaintImage))
     {
-        colPacked = resolve_general(prp, coverage, px, py, noise255, ramps, gradHeight, images, colPacked);
+        colPacked = resolve_general(prp, coverage, px, py, noise255, ramps, images, colPacked);
         return;
     }
     float src[4], a;
@@ -3222,7 +3259,7 @@ __device__ __forceinline__ void resolve_pixel(const PathPaint& pp, const PathRas
     }
     else
     {
-        sample_gradient255(*prp, px, py, ramps, gradHeight, src);
+        sample_gradient255(*prp, px, py, ramps, src);
         src[3] *= coverage;
         a = src[3] * (1.f / 255.f);
         src[0] *= a;
@@ -3400,7 +3437,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
     const PathCells* __restrict__ cells, const PathRaster* __restrict__ raster,
     const PathPaint* __restrict__ pathPaint, const uint2* __restrict__ cellPacked,
     const uint32_t* __restrict__ pathBase, const uint32_t* __restrict__ binned, const Prim* __restrict__ prims,
-    const uint32_t* __restrict__ ramps, uint32_t gradHeight, const ImageDesc* __restrict__ images,
+    const uint32_t* __restrict__ ramps, const ImageDesc* __restrict__ images,
     const CanvasDev* __restrict__ canvases, uint32_t canvasCount, const uint32_t* __restrict__ tileCover,
     const uint32_t* __restrict__ clipFirst, uint32_t dither, const float* __restrict__ featherTable, const uint32_t* __restrict__ tileOrder, uint32_t tileTotal,
     uint32_t* __restrict__ queueHead)
@@ -3500,6 +3537,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
             if (t < kWindow && p < pathEnd && (p >= cover || (pathPaint[p].kind & 8u)))
             {
                 const PathCells c = cells[p];
+                listed = c.flushStart != 0u;
                 if (tx >= c.tx0 && tx < c.tx1 && ty >= c.ty0 && ty < c.ty1)
                 {
                     const uint32_t cell = c.base + (uint32_t)(ty - c.ty0) * c.width + (uint32_t)(tx - c.tx0);
@@ -3711,8 +3749,10 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                         // winding's coverage is 1 under every fill rule.
                         if (pr.kind & kPaintPlain)
                             resolve_plain_full(pr, noise255, col);
+                        else if (pr.kind & kPaintFlushStart)
+                            clip = 0u;
                         else if (!(pr.kind & kPaintNoOp))
-                            resolve_pixel(pr, raster + path, 1.f, px, py, noise255, ramps, gradHeight, images, col,
+                            resolve_pixel(pr, raster + path, 1.f, px, py, noise255, ramps, images, col,
                                           clip);
                         continue;
                     }
@@ -3744,7 +3784,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                         }
                     }
                     if ((cov != 0.f && !(pr.kind & kPaintNoOp)) || (prFlags & 8u))
-                        resolve_pixel(pr, raster + path, cov, px, py, noise255, ramps, gradHeight, images, col, clip);
+                        resolve_pixel(pr, raster + path, cov, px, py, noise255, ramps, images, col, clip);
                 }
                 __syncthreads(); // every wave has read sLeft
                 (&sLeft[0][0])[t] = 0;
@@ -3763,7 +3803,8 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
 // draw_path.vert:431-545).
 __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const uint2* __restrict__ paints,
                                    const float* __restrict__ aux, const uint32_t* __restrict__ pathImage,
-                                   uint32_t pathCount, uint32_t gradHeight, PathRaster* __restrict__ out,
+                                   uint32_t pathCount, const FlushDev* __restrict__ flushes, uint32_t flushCount,
+                                   PathRaster* __restrict__ out,
                                    PathPaint* __restrict__ outPaint, uint32_t* __restrict__ clipFirst)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3777,6 +3818,7 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
     if (i > pathCount)
         return;
     PathRaster r;
+    const FlushDev fl = flushes[flush_of<&FlushDev::pathBase>(flushes, flushCount, i)];
     const PathDataV pd = paths[i];
     const uint2 paint = paints[i];
     const float* ax = aux + (size_t)i * 32;
@@ -3826,7 +3868,7 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
     }
     float span0 = ax[6], span1 = ax[7];
     r.gradSpan = span0 > .9f ? 2.f : span1;
-    r.gradRow = (uint32_t)(u2f(paint.y) * (float)gradHeight);
+    r.gradRow = fl.gradRowBase + min((uint32_t)(u2f(paint.y) * (float)fl.gradRows), fl.gradRows - 1u);
     // Image paints (gpu.cpp:1006-1034): image matrix and a constant LOD.
     const uint32_t img = pathImage[i];
     r.image = img & 0xffffu;
@@ -3854,6 +3896,8 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
         pp.kind |= r.alpha != 0.f ? kPaintPlain : kPaintNoOp;
     if (plain && pp.oneMinusAlpha == 0.f && !(flags & 1u))
         pp.kind |= kPaintOpaque;
+    if (i != 0u && fl.pathBase == i)
+        pp.kind = kPaintFlushStart | 8u;
     outPaint[i] = pp;
 }
 
