@@ -1364,14 +1364,12 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(ensure(ctx, ctx->pathRaster, (size_t)(pathCount + 1) * sizeof(PathRaster)));
     RIVE_TRY(ensure(ctx, ctx->pathPaint, (size_t)(pathCount + 1) * sizeof(PathPaint)));
     RIVE_TRY(ensure(ctx, ctx->clipFirst, ((size_t)pathCount / 64 + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->cells, (size_t)(pathCount + 1) * sizeof(PathCells)));
     path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
         paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, g.flushes, g.n, P<PathRaster>(ctx->pathRaster),
-        P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->clipFirst));
+        P<PathPaint>(ctx->pathPaint), P<PathCells>(ctx->cells), P<uint32_t>(ctx->clipFirst));
     RIVE_TRY(ensure(ctx, ctx->tileCover, (size_t)std::max<uint32_t>(tileTotal, 1) * 4));
     RIVE_TRY(clear(ctx, ctx->tileCover.ptr, 0, (size_t)tileTotal * 4));
-    RIVE_TRY(ensure(ctx, ctx->cells, (size_t)(pathCount + 1) * sizeof(PathCells)));
-    cells_init_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(P<PathCells>(ctx->cells),
-                                                                             pathCount + 1, g.flushes, g.n);
     RIVE_TRY(ensure(ctx, ctx->prims, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(Prim)));
     RIVE_TRY(ensure(ctx, ctx->verts, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(VtxPair)));
     if (totalPrims > 0)

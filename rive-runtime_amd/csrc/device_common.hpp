@@ -160,9 +160,12 @@ struct PathCells
     int32_t tx0, ty0, tx1, ty1; // [tx0, tx1) x [ty0, ty1); empty if tx0 >= tx1
     uint32_t base;              // first cell index
     uint32_t width;             // tx1 - tx0
-    uint32_t flushStart;        // the reserved record of a launch's second or later flush
+    uint32_t flags;             // kCell*: what the raster's listing and resolve branch on
     uint32_t pad;
 };
+constexpr uint32_t kCellStroke = 1u, kCellEvenOdd = 2u, kCellClockwise = 4u, kCellClipUpdate = 8u; // as PathRaster::flags
+constexpr uint32_t kCellPlain = 16u, kCellNoOp = 32u; // PathPaint's kPaintPlain, kPaintNoOp
+constexpr uint32_t kCellFlushStart = 64u;             // the reserved record of a launch's second or later flush
 
 // One canvas of a flush: its target, tile grid and path range.  Tiles of all
 // canvases form one launch; canvas c owns tiles [tileBase, tileBase + tilesX*tilesY).

@@ -1567,23 +1567,6 @@ __global__ void special_prims_kernel(const TessTexel* __restrict__ tex, const Fl
 // ---------------------------------------------------------------------------
 // Per-path cell grids.
 // ---------------------------------------------------------------------------
-__global__ void cells_init_kernel(PathCells* __restrict__ cells, uint32_t n, const FlushDev* __restrict__ flushes,
-                                  uint32_t flushCount)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n)
-        return;
-    PathCells c;
-    c.tx0 = c.ty0 = 0x7fffffff;
-    c.tx1 = c.ty1 = -0x7fffffff;
-    c.base = 0;
-    c.width = 0;
-    // the reserved record of a flush after the launch's first marks its start
-    c.flushStart = i != 0u && flushes[flush_of<&FlushDev::pathBase>(flushes, flushCount, i)].pathBase == i ? 1u : 0u;
-    c.pad = 0;
-    cells[i] = c;
-}
-
 // The canvas of each path (0xffffffff for paths outside every canvas): one
 // block per canvas.
 __global__ void path_canvas_kernel(const CanvasDev* __restrict__ canvases, uint32_t* __restrict__ pathCanvas)
@@ -1673,9 +1656,6 @@ constexpr uint32_t kPaintNoOp = 1u << 22;
 // A kPaintPlain fill of alpha 1: where its coverage is 1 the pixel becomes its
 // color whatever was drawn before.
 constexpr uint32_t kPaintOpaque = 1u << 23;
-// The reserved record of a flush after the launch's first: the clip buffer
-// starts empty there, since each flush numbers its clip IDs from 1.
-constexpr uint32_t kPaintFlushStart = 1u << 24;
 
 // Coverage of a winding count under the path's fill rule (draw_path.frag
 // fill-rule resolution): clockwise clamps the signed count to [0, 1], nonzero
@@ -2251,52 +2231,6 @@ __device__ __forceinline__ EdgeT make_edge(int32_t ax, int32_t ay, int32_t bx, i
     e.D0 = (int64_t)dx * (int64_t)(Y0 - ay) - (int64_t)dy * (int64_t)(X0 - ax);
     return e;
 }
-// Width-generic forms of the edge helpers for the per-row work (instantiated
-// for int64).
-template <typename I> struct EdgeTI
-{
-    int32_t A, B; // -dy, dx
-    I D0;
-};
-template <typename I>
-__device__ __forceinline__ EdgeTI<I> make_edge_t(int32_t ax, int32_t ay, int32_t bx, int32_t by, int32_t X0,
-                                                 int32_t Y0)
-{
-    EdgeTI<I> e;
-    const int32_t dx = bx - ax, dy = by - ay;
-    e.A = -dy;
-    e.B = dx;
-    e.D0 = (I)dx * (I)(Y0 - ay) - (I)dy * (I)(X0 - ax);
-    return e;
-}
-template <typename I> __device__ __forceinline__ int32_t clamp_thr_t(I t)
-{
-    const I lim = (I)1 << 30;
-    return (int32_t)(t < -lim ? -lim : (t > lim ? lim : t));
-}
-template <> __device__ __forceinline__ int32_t clamp_thr_t<double>(double t)
-{
-    return (int32_t)fmin(fmax(t, -1073741824.0), 1073741824.0);
-}
-template <typename I> __device__ __forceinline__ I ceil_div128_t(I a) { return -((-a) >> 7); }
-template <typename I> __device__ __forceinline__ I floor_div128_t(I a) { return a >> 7; }
-// Edge functions in double: coordinates lie in [-2^23, 2^23) (1/256 px), so
-// every product is below 2^49 and every sum below 2^50 -- exact, as are the
-// divisions by 128 and their floor and ceiling.
-template <> __device__ __forceinline__ double ceil_div128_t<double>(double a) { return ceil(a * (1.0 / 128.0)); }
-template <> __device__ __forceinline__ double floor_div128_t<double>(double a) { return floor(a * (1.0 / 128.0)); }
-template <typename I> __device__ __forceinline__ int32_t inside_threshold_t(const EdgeTI<I>& e, int o)
-{
-    const int pert = e.A != 0 ? (e.A > 0 ? 1 : -1) : (e.B > 0 ? 1 : (e.B < 0 ? -1 : 0));
-    const I oD0 = o > 0 ? e.D0 : -e.D0;
-    const I t = (o * pert > 0) ? ceil_div128_t<I>(-oD0) : floor_div128_t<I>(-oD0) + 1;
-    return clamp_thr_t<I>(t);
-}
-template <typename I>
-__device__ __forceinline__ I orient_t(int32_t ax, int32_t ay, int32_t bx, int32_t by, int32_t qx, int32_t qy)
-{
-    return (I)(bx - ax) * (I)(qy - ay) - (I)(by - ay) * (I)(qx - ax);
-}
 __device__ __forceinline__ float dither_noise(int x, int y)
 {
     // common.glsl:269-274, scale 1/256, bias -1/512 (gpu.cpp:822-824).
@@ -2332,7 +2266,9 @@ __device__ __forceinline__ float dither_noise(int x, int y)
 // workgroup, fills before strokes.  Every thread then resolves its pixel for
 // each path of the batch, turning the path's accumulators into coverage on
 // the way (prefix of the left-edge deltas and of the row's crossings, fill
-// rule).  The integer predicates are those of a per-pixel evaluation:
+// rule).  A batch takes three barriers: every wave resolves its own pixels and
+// clears what only it reads, and what the next batch shares is written after
+// that batch's first barrier.  The integer predicates are those of a per-pixel evaluation:
 // crossing columns solve the same threshold inequality, and a triangle's
 // pixels on a row are the candidates of a float span estimate (widened by its
 // error bound) that pass the exact three-edge test.
@@ -2348,72 +2284,6 @@ struct TileGeom
 {
     int32_t X0, Y0;
 };
-
-__device__ __forceinline__ void tri_row_candidates(int32_t ax, int32_t ay, int32_t bx, int32_t by, int32_t cx,
-                                                   int32_t cy, int32_t yq, int32_t X0, int* ilo, int* ihi)
-{
-    // Tile-relative x-range of the triangle on the row's sample line, as a
-    // float estimate widened by its error bound (an fdividef of relative
-    // error < 2^-21 scaled by the edge's width, plus rounding of the ends).
-    float xl = INFINITY, xr = -INFINITY, eps = 8.f;
-    const int32_t vx[3] = {ax - X0, bx - X0, cx - X0}, vy[3] = {ay, by, cy};
-#pragma unroll
-    for (int e = 0; e < 3; ++e)
-    {
-        const int32_t x0 = vx[e], y0 = vy[e], x1 = vx[(e + 1) % 3], y1 = vy[(e + 1) % 3];
-        if ((y0 <= yq && yq <= y1) || (y1 <= yq && yq <= y0))
-        {
-            if (y0 == y1)
-            {
-                xl = fminf(xl, (float)min(x0, x1));
-                xr = fmaxf(xr, (float)max(x0, x1));
-            }
-            else
-            {
-                const float dx = (float)(x1 - x0);
-                const float t = __fdividef((float)(yq - y0), (float)(y1 - y0));
-                const float x = (float)x0 + t * dx;
-                xl = fminf(xl, x);
-                xr = fmaxf(xr, x);
-                eps = fmaxf(eps, fabsf(dx) * (1.f / (1 << 18)) + fabsf(x) * (1.f / (1 << 20)));
-            }
-        }
-    }
-    if (!(xl <= xr))
-    {
-        *ilo = 1;
-        *ihi = 0;
-        return;
-    }
-    // pixel i's sample x is 256 i + 128 (tile-relative): the pixels whose
-    // samples fall in [xl - eps, xr + eps]
-    const float lo = (xl - eps - 128.f) * (1.f / 256.f);
-    const float hi = (xr + eps - 128.f) * (1.f / 256.f);
-    *ilo = (int)fmaxf(ceilf(lo), 0.f);
-    *ihi = (int)fminf(floorf(hi), (float)(kTile - 1));
-}
-
-// A border triangle's barycentric coverage at a pixel inside it, in
-// 1/65536 fixed point, clamped to [0, 1] (it leaves that range only by
-// rounding), so that a sum over 127 triangles stays below 2^23.
-__device__ __forceinline__ int32_t border_fixed(float cv)
-{
-    return __float2int_rn(fminf(fmaxf(cv, 0.f), 1.f) * 65536.f);
-}
-
-// Exact "inside" test of an edge against pixel (i2, j2) with orientation o.
-struct EdgeK
-{
-    int32_t A, B, thr; // o-premultiplied: inside iff A*i2 + B*j2 >= thr
-};
-template <typename I> __device__ __forceinline__ EdgeK edge_k(const EdgeTI<I>& e, int o)
-{
-    EdgeK k;
-    k.A = o * e.A;
-    k.B = o * e.B;
-    k.thr = inside_threshold_t<I>(e, o);
-    return k;
-}
 
 // Sample rows [*r0, *r1] of the tile that a primitive can touch inside the
 // tile's columns.  The per-row work looks at sample points with x in
@@ -2477,13 +2347,14 @@ __device__ __forceinline__ void prim_rows(const Prim& p, const TileGeom& g, int*
 
 // Left-edge winding of a fill primitive's inner edge I0 -> I1: the change of
 // the winding number from the tile's corner down to each row's sample line,
-// which is 0 above some row and a constant +-1 from it on.
-__device__ void fill_prim_left(const Prim& p, const TileGeom& g, int32_t* __restrict__ sLeft)
+// which is 0 above some row (*row) and a constant +-1 (returned; 0 when the
+// whole column is on the corner's side) from it on.
+__device__ __forceinline__ int32_t fill_prim_left(const Prim& p, const TileGeom& g, int* row)
 {
     const int32_t X0 = g.X0, Y0 = g.Y0;
     const int32_t xmin = min(p.p[0], p.p[4]), xmax = max(p.p[0], p.p[4]);
     if (!(xmin <= X0 && X0 < xmax) || (p.flags & kPrimNoEdge))
-        return;
+        return 0;
     const int neg = (p.flags & kPrimNegate) ? -1 : 1;
     if (p.p[1] != p.p[5])
     {
@@ -2498,128 +2369,326 @@ __device__ void fill_prim_left(const Prim& p, const TileGeom& g, int32_t* __rest
 #pragma unroll
         for (int j = 0; j < kTile; ++j)
             flipped |= (uint32_t)((s * (e.B * (2 * j + 1)) >= T) != Rcorner) << j;
-        if (flipped != 0)
-            atomicAdd(&sLeft[__builtin_ctz(flipped)], neg * s * (Rcorner ? -1 : 1));
+        *row = flipped != 0 ? __builtin_ctz(flipped) : 0;
+        return flipped != 0 ? neg * s * (Rcorner ? -1 : 1) : 0;
     }
-    else if (p.p[0] != p.p[4])
+    if (p.p[0] == p.p[4])
+        return 0;
+    // A horizontal edge never meets a sample line, but where it crosses
+    // the tile's left edge the winding below it steps by sign(dx).
+    const int32_t h = p.p[1];
+    if (Y0 >= h)
+        return 0;
+    const int32_t v = h - Y0 - (1 << (kSubpixelLog2 - 1));
+    *row = max(-((-v) >> kSubpixelLog2), 0); // first row with yq >= h
+    return *row < kTile ? neg * (p.p[4] > p.p[0] ? 1 : -1) : 0;
+}
+
+// A border triangle's barycentric coverage at a pixel inside it, in
+// 1/65536 fixed point, clamped to [0, 1] (it leaves that range only by
+// rounding), so that a sum over 127 triangles stays below 2^23.
+__device__ __forceinline__ int32_t border_fixed(float cv)
+{
+    return __float2int_rn(fminf(fmaxf(cv, 0.f), 1.f) * 65536.f);
+}
+
+// ---- one sample row of a primitive
+//
+// Along a row an edge function D(q) = dx (qy - ay) - dy (qx - ax) is linear in
+// the column, D(i) = r + s i with s = -256 dy, so a triangle's pixels are the
+// columns where its three edge values, less one where the tie rule excludes
+// zero, are all nonnegative.  The columns to look at come from -r / s of each
+// edge (five edges serve both triangles and the crossing of the inner edge): a
+// float quotient within 2^-15 of the true one wherever it decides a column,
+// widened by 1/64 for that and for the tie rule's 1 / |s| <= 1/256.  The test
+// in the loop is exact.
+//
+// Arithmetic I: a primitive whose vertices all lie within 64 px of the tile's
+// corner (every segment of a curve, in practice) takes int32.  With coordinates
+// c' = c - tile corner + 2^14 in [0, 2^15) the differences to a pixel of the
+// tile stay below 20480, each product below 2^29.4 and D below 2^30.4: exact,
+// formed by 24-bit multiplies, and the three tests are the sign of a bitwise
+// or.  Other primitives take double, exact for coordinates in [-2^23, 2^23):
+// every product is below 2^49.  The rows are VALU-bound; the form they replace
+// recomputed seven (fills) or five (strokes) double thresholds with their
+// floors and ceilings and two candidate searches per row.  Measured on MI355X,
+// raster pass with the batch's six barriers cut to three beside it: 1080p frame
+// 10.0 -> 9.0 ms, 48 canvases 8.1 -> 6.6 ms, feathered 961x541 frame 11.4 -> 9.6
+// ms (in double alone the feathered rows took 16.3 ms).
+constexpr int32_t kNearSub = 1 << 14;
+template <typename I> struct RowMath;
+template <> struct RowMath<int32_t>
+{
+    static constexpr int32_t org = kNearSub; // the tile corner's coordinate
+    static __device__ __forceinline__ int32_t mul(int32_t a, int32_t b) { return __mul24(a, b); }
+    static __device__ __forceinline__ int32_t flip(int32_t v, int32_t m) { return (v ^ m) - m; }
+    static __device__ __forceinline__ bool inside(int32_t a, int32_t b, int32_t c) { return (a | b | c) >= 0; }
+};
+template <> struct RowMath<double>
+{
+    static constexpr int32_t org = 0;
+    static __device__ __forceinline__ double mul(double a, double b) { return a * b; }
+    static __device__ __forceinline__ double flip(double v, int32_t m) { return m ? -v : v; }
+    static __device__ __forceinline__ bool inside(double a, double b, double c)
     {
-        // A horizontal edge never meets a sample line, but where it crosses
-        // the tile's left edge the winding below it steps by sign(dx).
-        const int32_t h = p.p[1];
-        if (Y0 < h)
+        return a >= 0. && b >= 0. && c >= 0.;
+    }
+};
+
+// A primitive's four vertices relative to the tile.
+template <typename I> struct TilePrim
+{
+    I x[4], y[4];
+};
+// False when a vertex is not near the tile (the int32 form then does not hold).
+__device__ __forceinline__ bool near_prim(const Prim& p, const TileGeom& g, TilePrim<int32_t>* n)
+{
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        n->x[k] = p.p[2 * k] - (g.X0 - kNearSub);
+        n->y[k] = p.p[2 * k + 1] - (g.Y0 - kNearSub);
+        m |= (uint32_t)n->x[k] | (uint32_t)n->y[k];
+    }
+    return m < 2u * (uint32_t)kNearSub;
+}
+__device__ __forceinline__ TilePrim<double> far_prim(const Prim& p, const TileGeom& g)
+{
+    TilePrim<double> n;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        n.x[k] = (double)(p.p[2 * k] - g.X0);
+        n.y[k] = (double)(p.p[2 * k + 1] - g.Y0);
+    }
+    return n;
+}
+
+// An edge a -> b along the sample row at yq: D at column i is r + s i.
+template <typename I> struct RowEdge
+{
+    I dx, dy, r, s;
+    float q; // -r / s
+};
+template <typename I>
+__device__ __forceinline__ RowEdge<I> row_edge(I ax, I ay, I bx, I by, int32_t yq)
+{
+    using M = RowMath<I>;
+    RowEdge<I> e;
+    e.dx = bx - ax;
+    e.dy = by - ay;
+    e.r = M::mul(e.dx, (I)yq - ay) - M::mul(e.dy, (I)(M::org + 128) - ax);
+    e.s = e.dy * (I)-256;
+    e.q = -(float)e.r * __builtin_amdgcn_rcpf((float)e.s);
+    return e;
+}
+template <typename I>
+__device__ __forceinline__ RowEdge<I> row_edge(const TilePrim<I>& n, int a, int b, int32_t yq)
+{
+    return row_edge<I>(n.x[a], n.y[a], n.x[b], n.y[b], yq);
+}
+template <typename I> __device__ __forceinline__ RowEdge<I> reversed(const RowEdge<I>& e)
+{
+    return RowEdge<I>{-e.dx, -e.dy, -e.r, -e.s, e.q};
+}
+// The edge as a side of a triangle of orientation 1 (m = 0) or -1 (m = -1):
+// inside at column i iff u + step i >= 0; narrows the column range [lo, hi].
+template <typename I> struct RowSide
+{
+    I u, step;
+    __device__ __forceinline__ I at(int i) const { return u + RowMath<I>::mul(step, (I)i); }
+};
+template <typename I>
+__device__ __forceinline__ RowSide<I> row_side(const RowEdge<I>& e, int32_t m, float* lo, float* hi)
+{
+    using M = RowMath<I>;
+    RowSide<I> k;
+    const I pert = e.dy != (I)0 ? -e.dy : e.dx;
+    k.step = M::flip(e.s, m);
+    k.u = M::flip(e.r, m) - (M::flip(pert, m) > (I)0 ? (I)0 : (I)1);
+    if (k.step > (I)0)
+        *lo = fmaxf(*lo, e.q);
+    else if (k.step < (I)0)
+        *hi = fminf(*hi, e.q);
+    else if (k.u < (I)0)
+        *hi = -1.f;
+    return k;
+}
+template <typename I> __device__ __forceinline__ I tri_area(I ax, I ay, I bx, I by, I cx, I cy)
+{
+    return RowMath<I>::mul(bx - ax, cy - ay) - RowMath<I>::mul(by - ay, cx - ax);
+}
+template <typename I> __device__ __forceinline__ I tri_area(const TilePrim<I>& n, int a, int b, int c)
+{
+    return tri_area<I>(n.x[a], n.y[a], n.x[b], n.y[b], n.x[c], n.y[c]);
+}
+__device__ __forceinline__ void column_range(float lo, float hi, bool draws, int* i0, int* i1)
+{
+    *i0 = (int)ceilf(fmaxf(lo - 1.f / 64.f, 0.f));
+    *i1 = (int)floorf(fminf(hi + 1.f / 64.f, (float)(kTile - 1)));
+    if (!draws || *i0 > *i1)
+    {
+        *i0 = kTile;
+        *i1 = -1;
+    }
+}
+__device__ __forceinline__ int32_t row_y(int32_t org, int j)
+{
+    return org + (j << kSubpixelLog2) + (1 << (kSubpixelLog2 - 1));
+}
+
+// The inner edge's crossing: +-1 at the first column right of it, if that is
+// not left of the tile -- the smallest i >= 0 with sg (r + s i) >= 0, sg s > 0.
+template <typename I>
+__device__ __forceinline__ void edge_crossing(const TilePrim<I>& n, const RowEdge<I>& e, int32_t yq, int neg, int j,
+                                              int32_t* __restrict__ sDelta, int32_t deltaUnit)
+{
+    const I y0 = n.y[0], y1 = n.y[2];
+    if (!((y0 <= (I)yq && (I)yq < y1) || (y1 <= (I)yq && (I)yq < y0)))
+        return;
+    const int32_t m = e.dy < (I)0 ? 0 : -1; // sg = 1 upward, -1 downward
+    const I r = RowMath<I>::flip(e.r, m), s = RowMath<I>::flip(e.s, m);
+    if (!(r < s / (I)2)) // the tile's left edge, half a column before column 0, is right of it
+        return;
+    int q = (int)fminf(fmaxf(ceilf(e.q), 0.f), (float)kTile);
+    q -= q > 0 && r + RowMath<I>::mul(s, (I)(q - 1)) >= (I)0 ? 1 : 0;
+    q += r + RowMath<I>::mul(s, (I)q) < (I)0 ? 1 : 0;
+    if (q < kTile)
+        atomicAdd(&sDelta[j * kTile + q], (m == 0 ? neg : -neg) * deltaUnit);
+}
+
+// A fill's row: the inner edge's crossing column and the two border triangles
+// T1 = (I0, O0, I1), coverage 1 - lambda(O0), and T2 = (I1, O0, O1), coverage
+// lambda(I1).  FLAT: a feathered quad without join ends, whose coverage is
+// FEATHER(half of that).
+template <typename I, bool FLAT = false>
+__device__ __forceinline__ void fill_row(const TilePrim<I>& n, uint32_t flags, int j, int32_t* __restrict__ sDelta,
+                                         int32_t* __restrict__ sBorder, int32_t deltaUnit,
+                                         const float* __restrict__ table = nullptr)
+{
+    const int32_t yq = row_y(RowMath<I>::org, j);
+    const int neg = (flags & kPrimNegate) ? -1 : 1;
+    const RowEdge<I> e = row_edge(n, 0, 2, yq), a = row_edge(n, 0, 1, yq), b = row_edge(n, 1, 2, yq);
+    const RowEdge<I> c = row_edge(n, 1, 3, yq), d = row_edge(n, 3, 2, yq);
+    if (!(flags & kPrimNoEdge))
+        edge_crossing(n, e, yq, neg, j, sDelta, deltaUnit);
+    const I A1 = (flags & kPrimNoT1) ? (I)0 : tri_area(n, 0, 1, 2);
+    const I A2 = (flags & kPrimNoT2) ? (I)0 : tri_area(n, 2, 1, 3);
+    const int32_t m1 = A1 < (I)0 ? -1 : 0, m2 = A2 < (I)0 ? -1 : 0;
+    float lo1 = 0.f, hi1 = (float)(kTile - 1), lo2 = 0.f, hi2 = (float)(kTile - 1);
+    const RowSide<I> a1 = row_side(a, m1, &lo1, &hi1), b1 = row_side(b, m1, &lo1, &hi1);
+    const RowSide<I> e1 = row_side(reversed(e), m1, &lo1, &hi1), b2 = row_side(reversed(b), m2, &lo2, &hi2);
+    const RowSide<I> c2 = row_side(c, m2, &lo2, &hi2), d2 = row_side(d, m2, &lo2, &hi2);
+    int i1, j1, i2, j2;
+    column_range(lo1, hi1, A1 != (I)0, &i1, &j1);
+    column_range(lo2, hi2, A2 != (I)0, &i2, &j2);
+    const float inv1 = __builtin_amdgcn_rcpf((float)A1), inv2 = __builtin_amdgcn_rcpf((float)A2);
+    const int32_t g1 = (neg ^ m1) - m1, g2 = (neg ^ m2) - m2; // neg * orientation
+    auto value = [&](float cv) {
+        return FLAT ? __float2int_rn(feather_table(table, .5f * cv) * 65536.f) : border_fixed(cv);
+    };
+    const int last = max(j1, j2);
+    int i = min(i1, i2);
+    I va = a1.at(i), vb = b1.at(i), ve = e1.at(i), wb = b2.at(i), wc = c2.at(i), wd = d2.at(i);
+    I De = e.r + RowMath<I>::mul(e.s, (I)i), Dc = c.r + RowMath<I>::mul(c.s, (I)i);
+    for (; i <= last; ++i)
+    {
+        const bool in1 = A1 != (I)0 && RowMath<I>::inside(va, vb, ve);
+        const bool in2 = A2 != (I)0 && RowMath<I>::inside(wb, wc, wd);
+        if (in1 || in2)
         {
-            const int32_t v = h - Y0 - (1 << (kSubpixelLog2 - 1));
-            const int jstar = max(-((-v) >> kSubpixelLog2), 0); // first row with yq >= h
-            if (jstar < kTile)
-                atomicAdd(&sLeft[jstar], neg * (p.p[4] > p.p[0] ? 1 : -1));
+            const int32_t f1 = in1 ? g1 * value(1.f + (float)De * inv1) : 0;
+            const int32_t f2 = in2 ? g2 * value((float)Dc * inv2) : 0;
+            atomicAdd(&sBorder[j * kTile + i], f1 + f2);
         }
+        va += a1.step;
+        vb += b1.step;
+        ve += e1.step;
+        wb += b2.step;
+        wc += c2.step;
+        wd += d2.step;
+        De += e.s;
+        Dc += c.s;
     }
 }
 
-// One sample row of a fill primitive: the inner edge's crossing column and
-// the two AA border triangles.
-template <typename I>
-__device__ void fill_prim_row(const Prim& p, int j, const TileGeom& g, int32_t* __restrict__ sDelta,
-                              int32_t* __restrict__ sBorder, int32_t deltaUnit)
+// find_stroke_coverage (draw_path.vert:500-508): min(x, y), or for a
+// feathered stroke (x biased below -1.5) 1 - FEATHER(1 - x) - FEATHER(1 - y)
+// (eval_feathered_stroke, draw_path_common.glsl:242-258).
+template <bool FEATHER>
+__device__ __forceinline__ float stroke_coverage(float cx, float cy, const float* __restrict__ table)
 {
-    const int32_t X0 = g.X0, Y0 = g.Y0;
-    const int32_t j2 = 2 * j + 1;
-    const int32_t yq = Y0 + (j << kSubpixelLog2) + (1 << (kSubpixelLog2 - 1));
-    const int neg = (p.flags & kPrimNegate) ? -1 : 1;
-    const EdgeTI<I> e = make_edge_t<I>(p.p[0], p.p[1], p.p[4], p.p[5], X0, Y0);
-    if (p.p[1] != p.p[5] && !(p.flags & kPrimNoEdge))
+    if (FEATHER && cx < -1.5f)
+        return 1.f - feather_table(table, 3.f + cx) - feather_table(table, 1.f - cy);
+    return fminf(cx, cy);
+}
+
+// A stroke's row: clockwise triangles T1 = (P0-, P0+, P1-) and T2 = (P1-, P0+,
+// P1+) only (so the two lie on either side of their common edge, and a pixel is
+// in one at most), the largest of the interpolated coverages.
+template <typename I, bool FEATHER = false>
+__device__ __forceinline__ void stroke_row(const TilePrim<I>& n, uint32_t flags, const float* __restrict__ cov, int j,
+                                           uint32_t* __restrict__ sMax, const float* __restrict__ table = nullptr)
+{
+    const int32_t yq = row_y(RowMath<I>::org, j);
+    const RowEdge<I> a = row_edge(n, 0, 1, yq), b = row_edge(n, 1, 2, yq), e = row_edge(n, 2, 0, yq);
+    const RowEdge<I> c = row_edge(n, 1, 3, yq), d = row_edge(n, 3, 2, yq);
+    const I A1 = (flags & kPrimNoT1) ? (I)0 : tri_area(n, 0, 1, 2);
+    const I A2 = (flags & kPrimNoT2) ? (I)0 : tri_area(n, 2, 1, 3);
+    float lo1 = 0.f, hi1 = (float)(kTile - 1), lo2 = 0.f, hi2 = (float)(kTile - 1);
+    const RowSide<I> a1 = row_side(a, 0, &lo1, &hi1), b1 = row_side(b, 0, &lo1, &hi1);
+    const RowSide<I> e1 = row_side(e, 0, &lo1, &hi1), b2 = row_side(reversed(b), 0, &lo2, &hi2);
+    const RowSide<I> c2 = row_side(c, 0, &lo2, &hi2), d2 = row_side(d, 0, &lo2, &hi2);
+    int i1, j1, i2, j2;
+    column_range(lo1, hi1, A1 > (I)0, &i1, &j1);
+    column_range(lo2, hi2, A2 > (I)0, &i2, &j2);
+    const int last = max(j1, j2);
+    int i = min(i1, i2);
+    const float inv1 = __builtin_amdgcn_rcpf((float)A1), inv2 = __builtin_amdgcn_rcpf((float)A2);
+    I va = a1.at(i), vb = b1.at(i), ve = e1.at(i), wb = b2.at(i), wc = c2.at(i), wd = d2.at(i);
+    // the edge values less the tie rule's 0 or 1, which each triangle's sides
+    // carry, are the barycentrics' numerators
+    const I ta = a.r - a1.u, tb = b.r - b1.u, te = e.r - e1.u, tc = c.r - c2.u, td = d.r - d2.u;
+    for (; i <= last; ++i)
     {
-        const int32_t ymin = min(p.p[1], p.p[5]), ymax = max(p.p[1], p.p[5]);
-        if (ymin <= yq && yq < ymax)
+        const bool in1 = A1 > (I)0 && RowMath<I>::inside(va, vb, ve);
+        const bool in2 = A2 > (I)0 && RowMath<I>::inside(wb, wc, wd);
+        if (in1 || in2)
         {
-            const int s = p.p[5] < p.p[1] ? 1 : -1;
-            const int32_t T = clamp_thr_t<I>(ceil_div128_t<I>(s > 0 ? -e.D0 : e.D0));
-            const int32_t krow = e.B * j2;
-            if (!(s * krow >= T))
-            {
-                // Smallest i with s*(A*(2i+1) + krow) >= T, where s*A = |dy|:
-                // 2|dy| i >= T - |dy| - s*krow.  The quotient is exact in
-                // double wherever it decides a column inside the tile.
-                const int64_t sa2 = 2 * (int64_t)(s * e.A);
-                const int64_t r = (int64_t)T - sa2 / 2 - (int64_t)s * krow;
-                if (r <= sa2 * (kTile - 1))
-                {
-                    // ceil(r / sa2) in [0, kTile): a float estimate, then exact
-                    int q = r <= 0 ? 0 : (int)ceilf(__fdividef((float)r, (float)sa2));
-                    q = min(max(q, 0), kTile - 1);
-                    while (q > 0 && sa2 * (q - 1) >= r)
-                        --q;
-                    while (sa2 * q < r)
-                        ++q;
-                    atomicAdd(&sDelta[j * kTile + q], neg * s * deltaUnit);
-                }
-            }
+            const float fb = (float)(vb + tb);
+            const float l0 = in1 ? fb * inv1 : (float)(wc + tc) * inv2;              // P0- of T1, P1- of T2
+            const float l1 = in1 ? (float)(ve + te) * inv1 : (float)(wd + td) * inv2; // P0+ of both
+            const float l2 = in1 ? (float)(va + ta) * inv1 : -fb * inv2;             // P1- of T1, P1+ of T2
+            const float cx = l0 * (in1 ? cov[0] : cov[4]) + l1 * cov[2] + l2 * (in1 ? cov[4] : cov[6]);
+            const float cy = l0 * (in1 ? cov[1] : cov[5]) + l1 * cov[3] + l2 * (in1 ? cov[5] : cov[7]);
+            const float v = stroke_coverage<FEATHER>(cx, cy, table);
+            if (v > 0.f)
+                atomicMax(&sMax[j * kTile + i], __float_as_uint(v));
         }
+        va += a1.step;
+        vb += b1.step;
+        ve += e1.step;
+        wb += b2.step;
+        wc += c2.step;
+        wd += d2.step;
     }
-    // Border triangle T1 = (I0, O0, I1), coverage 1 - lambda(O0).
-    const I A1 = (p.flags & kPrimNoT1) ? (I)0 : orient_t<I>(p.p[0], p.p[1], p.p[2], p.p[3], p.p[4], p.p[5]);
-    if (A1 != 0)
-    {
-        int ilo, ihi;
-        tri_row_candidates(p.p[0], p.p[1], p.p[2], p.p[3], p.p[4], p.p[5], yq, X0, &ilo, &ihi);
-        if (ilo <= ihi)
-        {
-            const int o = A1 > 0 ? 1 : -1;
-            const EdgeK k01 = edge_k<I>(make_edge_t<I>(p.p[0], p.p[1], p.p[2], p.p[3], X0, Y0), o);
-            const EdgeK k12 = edge_k<I>(make_edge_t<I>(p.p[2], p.p[3], p.p[4], p.p[5], X0, Y0), o);
-            const EdgeK k20 = edge_k<I>(make_edge_t<I>(p.p[4], p.p[5], p.p[0], p.p[1], X0, Y0), o);
-            const float inv = __builtin_amdgcn_rcpf((float)A1);
-            // edge values at pixel ilo, stepped exactly by 2A per pixel
-            const int32_t i2 = 2 * ilo + 1;
-            int32_t v01 = k01.A * i2 + k01.B * j2, v12 = k12.A * i2 + k12.B * j2, v20 = k20.A * i2 + k20.B * j2;
-            int32_t ke = e.A * i2 + e.B * j2;
-            const float D0 = (float)e.D0;
-            for (int i = ilo; i <= ihi; ++i)
-            {
-                if (v01 >= k01.thr && v12 >= k12.thr && v20 >= k20.thr)
-                {
-                    const float De = D0 + 128.f * (float)ke;
-                    atomicAdd(&sBorder[j * kTile + i], neg * o * border_fixed(1.f + De * inv));
-                }
-                v01 += 2 * k01.A;
-                v12 += 2 * k12.A;
-                v20 += 2 * k20.A;
-                ke += 2 * e.A;
-            }
-        }
-    }
-    // Border triangle T2 = (I1, O0, O1), coverage lambda(I1).
-    const I A2 = (p.flags & kPrimNoT2) ? (I)0 : orient_t<I>(p.p[4], p.p[5], p.p[2], p.p[3], p.p[6], p.p[7]);
-    if (A2 != 0)
-    {
-        int ilo, ihi;
-        tri_row_candidates(p.p[4], p.p[5], p.p[2], p.p[3], p.p[6], p.p[7], yq, X0, &ilo, &ihi);
-        if (ilo <= ihi)
-        {
-            const int o = A2 > 0 ? 1 : -1;
-            const EdgeK f01 = edge_k<I>(make_edge_t<I>(p.p[4], p.p[5], p.p[2], p.p[3], X0, Y0), o);
-            const EdgeTI<I> f12e = make_edge_t<I>(p.p[2], p.p[3], p.p[6], p.p[7], X0, Y0);
-            const EdgeK f12 = edge_k(f12e, o);
-            const EdgeK f20 = edge_k<I>(make_edge_t<I>(p.p[6], p.p[7], p.p[4], p.p[5], X0, Y0), o);
-            const float inv = __builtin_amdgcn_rcpf((float)A2);
-            const int32_t i2 = 2 * ilo + 1;
-            int32_t v01 = f01.A * i2 + f01.B * j2, v12 = f12.A * i2 + f12.B * j2, v20 = f20.A * i2 + f20.B * j2;
-            int32_t k12 = f12e.A * i2 + f12e.B * j2;
-            const float D0 = (float)f12e.D0;
-            for (int i = ilo; i <= ihi; ++i)
-            {
-                if (v01 >= f01.thr && v12 >= f12.thr && v20 >= f20.thr)
-                {
-                    const float D12 = D0 + 128.f * (float)k12;
-                    atomicAdd(&sBorder[j * kTile + i], neg * o * border_fixed(D12 * inv));
-                }
-                v01 += 2 * f01.A;
-                v12 += 2 * f12.A;
-                v20 += 2 * f20.A;
-                k12 += 2 * f12e.A;
-            }
-        }
-    }
+}
+
+// Rows of primitives that are not near, out of line so that the near rows keep
+// their registers.
+__device__ __noinline__ void fill_far_row(const Prim* __restrict__ prims, uint32_t idx, int j, int32_t X0, int32_t Y0,
+                                          int32_t* __restrict__ sDelta, int32_t* __restrict__ sBorder,
+                                          int32_t deltaUnit)
+{
+    const Prim p = prims[idx];
+    fill_row<double>(far_prim(p, TileGeom{X0, Y0}), p.flags, j, sDelta, sBorder, deltaUnit);
+}
+__device__ __noinline__ void stroke_far_row(const Prim* __restrict__ prims, uint32_t idx, int j, int32_t X0,
+                                            int32_t Y0, uint32_t* __restrict__ sMax)
+{
+    const Prim p = prims[idx];
+    stroke_row<double>(far_prim(p, TileGeom{X0, Y0}), p.flags, p.cov, j, sMax);
 }
 
 // eval_feathered_fill (draw_path_common.glsl:153-240): the feather above y0
@@ -2650,76 +2719,79 @@ __device__ __forceinline__ float eval_feathered_fill(const float* c, const float
     return cov * signf_(c[0]);
 }
 
-// One sample row of one triangle of a feathered segment: the coverage
-// vectors interpolated at each pixel inside it, evaluated, and added with the
-// triangle's orientation (the fixed-point border units of the fill rows).
-__device__ __forceinline__ void feather_tri_row(int32_t ax, int32_t ay, int32_t bx, int32_t by, int32_t cx,
-                                                int32_t cy, const float* ca, const float* cb, const float* cc,
-                                                int neg, int j, const TileGeom& g, int32_t* __restrict__ sBorder,
+// One sample row of one triangle of a feathered segment with a join end: the
+// coverage vectors interpolated at each pixel inside it, evaluated, and added
+// with the triangle's orientation (the fixed-point border units of the fill
+// rows).
+template <typename I>
+__device__ __forceinline__ void feather_tri_row(I ax, I ay, I bx, I by, I cx, I cy, const float* ca, const float* cb,
+                                                const float* cc, int neg, int j, int32_t* __restrict__ sBorder,
                                                 const float* __restrict__ table)
 {
-    typedef double I;
-    const I A = orient_t<I>(ax, ay, bx, by, cx, cy);
-    if (A == 0)
+    const I A = tri_area<I>(ax, ay, bx, by, cx, cy);
+    if (A == (I)0)
         return;
-    const int32_t X0 = g.X0, Y0 = g.Y0;
-    const int32_t j2 = 2 * j + 1;
-    const int32_t yq = Y0 + (j << kSubpixelLog2) + (1 << (kSubpixelLog2 - 1));
-    int ilo, ihi;
-    tri_row_candidates(ax, ay, bx, by, cx, cy, yq, X0, &ilo, &ihi);
-    if (ilo > ihi)
-        return;
-    const int o = A > 0 ? 1 : -1;
-    const EdgeTI<I> eab = make_edge_t<I>(ax, ay, bx, by, X0, Y0);
-    const EdgeTI<I> ebc = make_edge_t<I>(bx, by, cx, cy, X0, Y0);
-    const EdgeTI<I> eca = make_edge_t<I>(cx, cy, ax, ay, X0, Y0);
-    const EdgeK kab = edge_k<I>(eab, o), kbc = edge_k<I>(ebc, o), kca = edge_k<I>(eca, o);
+    const int32_t yq = row_y(RowMath<I>::org, j), m = A < (I)0 ? -1 : 0;
+    const RowEdge<I> eab = row_edge<I>(ax, ay, bx, by, yq), ebc = row_edge<I>(bx, by, cx, cy, yq);
+    const RowEdge<I> eca = row_edge<I>(cx, cy, ax, ay, yq);
+    float lo = 0.f, hi = (float)(kTile - 1);
+    const RowSide<I> sab = row_side(eab, m, &lo, &hi), sbc = row_side(ebc, m, &lo, &hi);
+    const RowSide<I> sca = row_side(eca, m, &lo, &hi);
+    int i, last;
+    column_range(lo, hi, true, &i, &last);
     const float inv = 1.f / (float)A;
-    const int32_t i2 = 2 * ilo + 1;
-    int32_t vab = kab.A * i2 + kab.B * j2, vbc = kbc.A * i2 + kbc.B * j2, vca = kca.A * i2 + kca.B * j2;
-    int32_t wab = eab.A * i2 + eab.B * j2, wbc = ebc.A * i2 + ebc.B * j2, wca = eca.A * i2 + eca.B * j2;
-    const float dab = (float)eab.D0, dbc = (float)ebc.D0, dca = (float)eca.D0;
-    for (int i = ilo; i <= ihi; ++i)
+    I vab = sab.at(i), vbc = sbc.at(i), vca = sca.at(i);
+    I Dab = eab.r + RowMath<I>::mul(eab.s, (I)i), Dbc = ebc.r + RowMath<I>::mul(ebc.s, (I)i);
+    I Dca = eca.r + RowMath<I>::mul(eca.s, (I)i);
+    const int32_t sign = (neg ^ m) - m;
+    for (; i <= last; ++i)
     {
-        if (vab >= kab.thr && vbc >= kbc.thr && vca >= kca.thr)
+        if (RowMath<I>::inside(vab, vbc, vca))
         {
             // barycentrics: the edge opposite each vertex over the area
-            const float la = (dbc + 128.f * (float)wbc) * inv;
-            const float lb = (dca + 128.f * (float)wca) * inv;
-            const float lc = (dab + 128.f * (float)wab) * inv;
+            const float la = (float)Dbc * inv, lb = (float)Dca * inv, lc = (float)Dab * inv;
             float c4[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 c4[q] = la * ca[q] + lb * cb[q] + lc * cc[q];
             const float v = fminf(fmaxf(eval_feathered_fill(c4, table), -1.f), 1.f);
-            atomicAdd(&sBorder[j * kTile + i], neg * o * __float2int_rn(v * 65536.f));
+            atomicAdd(&sBorder[j * kTile + i], sign * __float2int_rn(v * 65536.f));
         }
-        vab += 2 * kab.A;
-        vbc += 2 * kbc.A;
-        vca += 2 * kca.A;
-        wab += 2 * eab.A;
-        wbc += 2 * ebc.A;
-        wca += 2 * eca.A;
+        vab += sab.step;
+        vbc += sbc.step;
+        vca += sca.step;
+        Dab += eab.s;
+        Dbc += ebc.s;
+        Dca += eca.s;
     }
 }
 
 // One sample row of a feathered segment [E0, T0, E1, T1]: the edge's crossing
-// column and its four border triangles (the inner points are 2E - T).  Kept
-// out of line, reading the primitive itself, so the fill and stroke rows keep
-// their registers.
-__device__ __noinline__ void feather_prim_row(const Prim* __restrict__ prims, uint32_t idx, int j, int32_t X0,
-                                              int32_t Y0, int32_t* __restrict__ sDelta,
-                                              int32_t* __restrict__ sBorder, int32_t deltaUnit,
-                                              const float* __restrict__ table)
+// column and its four border triangles, those of the quad and of its mirror
+// [E0, B0, E1, B1] (B = 2E - T).  A segment without join ends has coverage
+// vectors (y, -2, 1e6, y) with y half the plain border's coverage, whose
+// feathered value is FEATHER(y): its quads are filled like a plain fill's.
+// Segments with a join end interpolate and evaluate the whole vectors.
+template <typename I, bool JOIN>
+__device__ __forceinline__ void feather_rows(const Prim& p, const TilePrim<I>& n, int j, int32_t* __restrict__ sDelta,
+                                             int32_t* __restrict__ sBorder, int32_t deltaUnit,
+                                             const float* __restrict__ table)
 {
-    Prim p = prims[idx];
-    const TileGeom g{X0, Y0};
+    TilePrim<I> mirror = n;
+    mirror.x[1] = n.x[0] + n.x[0] - n.x[1];
+    mirror.y[1] = n.y[0] + n.y[0] - n.y[1];
+    mirror.x[3] = n.x[2] + n.x[2] - n.x[3];
+    mirror.y[3] = n.y[2] + n.y[2] - n.y[3];
+    if (!JOIN)
     {
-        Prim edge = p;
-        edge.flags |= kPrimNoT1 | kPrimNoT2;
-        fill_prim_row<double>(edge, j, g, sDelta, sBorder, deltaUnit);
+        fill_row<I, true>(n, p.flags, j, sDelta, sBorder, deltaUnit, table);
+        fill_row<I, true>(mirror, p.flags | kPrimNoEdge, j, sDelta, sBorder, deltaUnit, table);
+        return;
     }
     const int neg = (p.flags & kPrimNegate) ? -1 : 1;
+    const int32_t yq = row_y(RowMath<I>::org, j);
+    if (!(p.flags & kPrimNoEdge))
+        edge_crossing(n, row_edge(n, 0, 2, yq), yq, neg, j, sDelta, deltaUnit);
     float cE0[4] = {.5f, -2.f, 1e6f, .5f}, cT0[4] = {0.f, -2.f, 1e6f, 0.f};
     float cE1[4] = {.5f, -2.f, 1e6f, .5f}, cT1[4] = {0.f, -2.f, 1e6f, 0.f};
     if (p.flags & kPrimJoin0)
@@ -2742,118 +2814,65 @@ __device__ __noinline__ void feather_prim_row(const Prim* __restrict__ prims, ui
         cE1[2] = cT1[2];
         cE1[3] = u2f(p.pad[1]);
     }
-    const int32_t e0x = p.p[0], e0y = p.p[1], t0x = p.p[2], t0y = p.p[3];
-    const int32_t e1x = p.p[4], e1y = p.p[5], t1x = p.p[6], t1y = p.p[7];
-    const int32_t b0x = 2 * e0x - t0x, b0y = 2 * e0y - t0y, b1x = 2 * e1x - t1x, b1y = 2 * e1y - t1y;
-    feather_tri_row(e0x, e0y, t0x, t0y, e1x, e1y, cE0, cT0, cE1, neg, j, g, sBorder, table);
-    feather_tri_row(e1x, e1y, t0x, t0y, t1x, t1y, cE1, cT0, cT1, neg, j, g, sBorder, table);
-    feather_tri_row(e0x, e0y, b0x, b0y, e1x, e1y, cE0, cT0, cE1, neg, j, g, sBorder, table);
-    feather_tri_row(e1x, e1y, b0x, b0y, b1x, b1y, cE1, cT0, cT1, neg, j, g, sBorder, table);
+#pragma unroll 1
+    for (int k = 0; k < 2; ++k)
+    {
+        const I x1 = k == 0 ? n.x[1] : mirror.x[1], y1 = k == 0 ? n.y[1] : mirror.y[1];
+        const I x3 = k == 0 ? n.x[3] : mirror.x[3], y3 = k == 0 ? n.y[3] : mirror.y[3];
+        feather_tri_row<I>(n.x[0], n.y[0], x1, y1, n.x[2], n.y[2], cE0, cT0, cE1, neg, j, sBorder, table);
+        feather_tri_row<I>(n.x[2], n.y[2], x1, y1, x3, y3, cE1, cT0, cT1, neg, j, sBorder, table);
+    }
 }
 
-// find_stroke_coverage (draw_path.vert:500-508): min(x, y), or for a
-// feathered stroke (x biased below -1.5) 1 - FEATHER(1 - x) - FEATHER(1 - y)
-// (eval_feathered_stroke, draw_path_common.glsl:242-258).
-template <bool FEATHER>
-__device__ __forceinline__ float stroke_coverage(float cx, float cy, const float* __restrict__ table)
+// The int32 form for a feathered segment, whose outer points lie up to a
+// feather's radius away: with every vertex of both quads within 128 px of the
+// tile's corner and no edge over kNearEdge along an axis, the differences to a
+// pixel of the tile or the column after it stay below 2^15 + 2^12 + 2^8, each
+// product below 9.7e8 and D below 1.94e9 < 2^31.
+constexpr int32_t kNearEdge = 26000; // 101 px
+__device__ __forceinline__ bool near_feather(const TilePrim<int32_t>& n)
 {
-    if (FEATHER && cx < -1.5f)
-        return 1.f - feather_table(table, 3.f + cx) - feather_table(table, 1.f - cy);
-    return fminf(cx, cy);
+    const int32_t bx0 = 2 * n.x[0] - n.x[1], by0 = 2 * n.y[0] - n.y[1];
+    const int32_t bx1 = 2 * n.x[2] - n.x[3], by1 = 2 * n.y[2] - n.y[3];
+    auto span = [](int32_t a, int32_t b, int32_t c, int32_t d) {
+        return max(max(a, b), max(c, d)) - min(min(a, b), min(c, d));
+    };
+    auto far = [](int32_t v) { return (uint32_t)(v + kNearSub) >= 4u * (uint32_t)kNearSub; };
+    bool bad = far(bx0) || far(by0) || far(bx1) || far(by1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        bad = bad || far(n.x[k]) || far(n.y[k]);
+    const int32_t w = max(span(n.x[0], n.x[1], n.x[2], n.x[3]), span(n.x[0], bx0, n.x[2], bx1));
+    const int32_t h = max(span(n.y[0], n.y[1], n.y[2], n.y[3]), span(n.y[0], by0, n.y[2], by1));
+    return !bad && max(w, h) < kNearEdge;
 }
 
-template <typename I, bool FEATHER = false>
-__device__ void stroke_prim_row(const Prim& p, int j, const TileGeom& g, uint32_t* __restrict__ sMax,
-                                const float* __restrict__ table = nullptr)
+// Kept out of line, reading the primitive itself, so the fill and stroke rows
+// keep their registers; JOIN: a segment with a join end.
+__device__ __noinline__ void feather_far_row(const Prim* __restrict__ prims, uint32_t idx, int j, int32_t X0,
+                                             int32_t Y0, int32_t* __restrict__ sDelta, int32_t* __restrict__ sBorder,
+                                             int32_t deltaUnit, const float* __restrict__ table)
 {
-    const int32_t X0 = g.X0, Y0 = g.Y0;
-    const int32_t j2 = 2 * j + 1;
-    const int32_t yq = Y0 + (j << kSubpixelLog2) + (1 << (kSubpixelLog2 - 1));
-    // T1 = (P0-, P0+, P1-): vertices 0, 1, 2; T2 = (P1-, P0+, P1+): 2, 1, 3.
-    // Only clockwise triangles draw.
-    const I A1 = (p.flags & kPrimNoT1) ? (I)0 : orient_t<I>(p.p[0], p.p[1], p.p[2], p.p[3], p.p[4], p.p[5]);
-    const I A2 = (p.flags & kPrimNoT2) ? (I)0 : orient_t<I>(p.p[4], p.p[5], p.p[2], p.p[3], p.p[6], p.p[7]);
-    const EdgeTI<I> e12 = make_edge_t<I>(p.p[2], p.p[3], p.p[4], p.p[5], X0, Y0);
-    if (A1 > 0)
-    {
-        int ilo, ihi;
-        tri_row_candidates(p.p[0], p.p[1], p.p[2], p.p[3], p.p[4], p.p[5], yq, X0, &ilo, &ihi);
-        if (ilo <= ihi)
-        {
-            const EdgeTI<I> e01 = make_edge_t<I>(p.p[0], p.p[1], p.p[2], p.p[3], X0, Y0);
-            const EdgeTI<I> e20 = make_edge_t<I>(p.p[4], p.p[5], p.p[0], p.p[1], X0, Y0);
-            const int32_t t01 = inside_threshold_t<I>(e01, 1), t12 = inside_threshold_t<I>(e12, 1),
-                          t20 = inside_threshold_t<I>(e20, 1);
-            const float inv = __builtin_amdgcn_rcpf((float)A1);
-            // Edge values at pixel ilo, stepped exactly by 2A per pixel; the
-            // interpolated coverages are linear in the column too and step by
-            // float adds (within 16 ulp of a direct evaluation).
-            const int32_t i2 = 2 * ilo + 1;
-            int32_t k01 = e01.A * i2 + e01.B * j2, k12 = e12.A * i2 + e12.B * j2, k20 = e20.A * i2 + e20.B * j2;
-            const float l0 = ((float)e12.D0 + 128.f * (float)k12) * inv;
-            const float l1 = ((float)e20.D0 + 128.f * (float)k20) * inv;
-            const float l2 = ((float)e01.D0 + 128.f * (float)k01) * inv;
-            const float s0 = 256.f * (float)e12.A * inv, s1 = 256.f * (float)e20.A * inv,
-                        s2 = 256.f * (float)e01.A * inv;
-            float cx = l0 * p.cov[0] + l1 * p.cov[2] + l2 * p.cov[4];
-            float cy = l0 * p.cov[1] + l1 * p.cov[3] + l2 * p.cov[5];
-            const float dcx = s0 * p.cov[0] + s1 * p.cov[2] + s2 * p.cov[4];
-            const float dcy = s0 * p.cov[1] + s1 * p.cov[3] + s2 * p.cov[5];
-            for (int i = ilo; i <= ihi; ++i)
-            {
-                if (k01 >= t01 && k12 >= t12 && k20 >= t20)
-                {
-                    const float v = stroke_coverage<FEATHER>(cx, cy, table);
-                    if (v > 0.f)
-                        atomicMax(&sMax[j * kTile + i], __float_as_uint(v));
-                }
-                k01 += 2 * e01.A;
-                k12 += 2 * e12.A;
-                k20 += 2 * e20.A;
-                cx += dcx;
-                cy += dcy;
-            }
-        }
-    }
-    if (A2 > 0)
-    {
-        int ilo, ihi;
-        tri_row_candidates(p.p[4], p.p[5], p.p[2], p.p[3], p.p[6], p.p[7], yq, X0, &ilo, &ihi);
-        if (ilo <= ihi)
-        {
-            // T2 edges: P1- -> P0+ is the reverse of e12.
-            const EdgeTI<I> e13 = make_edge_t<I>(p.p[2], p.p[3], p.p[6], p.p[7], X0, Y0);
-            const EdgeTI<I> e32 = make_edge_t<I>(p.p[6], p.p[7], p.p[4], p.p[5], X0, Y0);
-            const int32_t t21 = inside_threshold_t<I>(EdgeTI<I>{-e12.A, -e12.B, -e12.D0}, 1);
-            const int32_t t13 = inside_threshold_t<I>(e13, 1), t32 = inside_threshold_t<I>(e32, 1);
-            const float inv = __builtin_amdgcn_rcpf((float)A2);
-            const int32_t i2 = 2 * ilo + 1;
-            int32_t k12 = e12.A * i2 + e12.B * j2, k13 = e13.A * i2 + e13.B * j2, k32 = e32.A * i2 + e32.B * j2;
-            const float l0 = ((float)e13.D0 + 128.f * (float)k13) * inv;  // P1-
-            const float l1 = ((float)e32.D0 + 128.f * (float)k32) * inv;  // P0+
-            const float l2 = -((float)e12.D0 + 128.f * (float)k12) * inv; // P1+
-            const float s0 = 256.f * (float)e13.A * inv, s1 = 256.f * (float)e32.A * inv,
-                        s2 = -256.f * (float)e12.A * inv;
-            float cx = l0 * p.cov[4] + l1 * p.cov[2] + l2 * p.cov[6];
-            float cy = l0 * p.cov[5] + l1 * p.cov[3] + l2 * p.cov[7];
-            const float dcx = s0 * p.cov[4] + s1 * p.cov[2] + s2 * p.cov[6];
-            const float dcy = s0 * p.cov[5] + s1 * p.cov[3] + s2 * p.cov[7];
-            for (int i = ilo; i <= ihi; ++i)
-            {
-                if (-k12 >= t21 && k13 >= t13 && k32 >= t32)
-                {
-                    const float v = stroke_coverage<FEATHER>(cx, cy, table);
-                    if (v > 0.f)
-                        atomicMax(&sMax[j * kTile + i], __float_as_uint(v));
-                }
-                k12 += 2 * e12.A;
-                k13 += 2 * e13.A;
-                k32 += 2 * e32.A;
-                cx += dcx;
-                cy += dcy;
-            }
-        }
-    }
+    const Prim p = prims[idx];
+    const TilePrim<double> n = far_prim(p, TileGeom{X0, Y0});
+    if (p.flags & (kPrimJoin0 | kPrimJoin1))
+        feather_rows<double, true>(p, n, j, sDelta, sBorder, deltaUnit, table);
+    else
+        feather_rows<double, false>(p, n, j, sDelta, sBorder, deltaUnit, table);
+}
+template <bool JOIN>
+__device__ __noinline__ void feather_prim_row(const Prim* __restrict__ prims, uint32_t idx, int j, int32_t X0,
+                                              int32_t Y0, int32_t* __restrict__ sDelta,
+                                              int32_t* __restrict__ sBorder, int32_t deltaUnit,
+                                              const float* __restrict__ table)
+{
+    const Prim p = prims[idx];
+    TilePrim<int32_t> n;
+    (void)near_prim(p, TileGeom{X0, Y0}, &n);
+    if (near_feather(n))
+        feather_rows<int32_t, JOIN>(p, n, j, sDelta, sBorder, deltaUnit, table);
+    else
+        feather_far_row(prims, idx, j, X0, Y0, sDelta, sBorder, deltaUnit, table);
 }
 
 // A feathered stroke's sample row, out of line like feather_prim_row.
@@ -2862,7 +2881,12 @@ __device__ __noinline__ void feather_stroke_prim_row(const Prim* __restrict__ pr
                                                      const float* __restrict__ table)
 {
     const Prim p = prims[idx];
-    stroke_prim_row<double, true>(p, j, TileGeom{X0, Y0}, sMax, table);
+    const TileGeom g{X0, Y0};
+    TilePrim<int32_t> n;
+    if (near_prim(p, g, &n))
+        stroke_row<int32_t, true>(n, p.flags, p.cov, j, sMax, table);
+    else
+        stroke_row<double, true>(far_prim(p, g), p.flags, p.cov, j, sMax, table);
 }
 
 // Image sampling with the reference's sampler state (pipeline_manager_vulkan.cpp:
@@ -3444,17 +3468,19 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
 {
     __shared__ __align__(16) int32_t sAcc[kAccArrays][kTile * kTile];
     __shared__ int32_t sLeft[kAccArrays][kTile];
-    // The listed paths of the current window of 256 paths, in order, with
+    // The listed paths of the current window of kWindow paths, in order, with
     // exclusive prefixes of their primitive counts and of slot_arrays().
-    // sRel[q] = (path, primitive count n, corner winding C, slot/array
-    // prefix) -- one 16-byte read per entry in the resolve; sRelB[q] = (bin
-    // offset, primitive prefix).
+    // sRel[q] = (path, primitive count n, corner winding C, slot/array prefix
+    // (below 2^24: at most 127 entries of two arrays come before one) | the
+    // path's kCell flags << 24) -- one 16-byte read per entry in the resolve;
+    // sRelB[q] = (bin offset, primitive prefix).
+    constexpr uint32_t kPrefixMask = 0xffffffu;
     __shared__ uint4 sRel[kWindow];
     __shared__ uint2 sRelB[kWindow];
     __shared__ uint32_t sWave[3][kWgThreads / 64];
     __shared__ uint8_t sOwner[kMaxItems];
     __shared__ uint32_t sItemPrim[kWgThreads];
-    __shared__ uint32_t sItemInfo[kWgThreads]; // array | wide << 4 | stroke << 5 | row0 << 8 | item0 << 16
+    __shared__ uint32_t sItemInfo[kWgThreads]; // array | wide << 4 | class << 5 | row0 << 8 | item0 << 16
 
     __shared__ uint32_t sTake;
 
@@ -3534,11 +3560,13 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
             uint32_t off = 0, n = 0;
             int32_t C = 0;
             bool listed = false;
-            if (t < kWindow && p < pathEnd && (p >= cover || (pathPaint[p].kind & 8u)))
+            uint32_t flags = 0;
+            if (t < kWindow && p < pathEnd)
             {
                 const PathCells c = cells[p];
-                listed = c.flushStart != 0u;
-                if (tx >= c.tx0 && tx < c.tx1 && ty >= c.ty0 && ty < c.ty1)
+                flags = c.flags;
+                listed = (flags & kCellFlushStart) != 0u;
+                if ((p >= cover || (flags & kCellClipUpdate)) && tx >= c.tx0 && tx < c.tx1 && ty >= c.ty0 && ty < c.ty1)
                 {
                     const uint32_t cell = c.base + (uint32_t)(ty - c.ty0) * c.width + (uint32_t)(tx - c.tx0);
                     const uint2 here = cellPacked[cell];
@@ -3551,10 +3579,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                     // (every clip draw has a fresh ID), so it is not listed.
                     listed = n != 0;
                     if (n == 0 && C != 0)
-                    {
-                        const uint32_t flags = pathPaint[p].kind & 0xffffu;
-                        listed = !(flags & 1u) && fill_rule_coverage((float)C, flags) != 0.f;
-                    }
+                        listed = !(flags & kCellStroke) && fill_rule_coverage((float)C, flags) != 0.f;
                 }
             }
             const uint32_t vSA = slot_arrays(n);
@@ -3594,7 +3619,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
             if (listed)
             {
                 const uint32_t q = preL + posInWave;
-                sRel[q] = make_uint4(p, n, (uint32_t)C, preSA + iSA - vSA);
+                sRel[q] = make_uint4(p, n, (uint32_t)C, (preSA + iSA - vSA) | (flags << 24));
                 sRelB[q] = make_uint2(off, preP + iP - n);
             }
             __syncthreads();
@@ -3602,7 +3627,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
             for (uint32_t s = 0; s < nRel;)
             {
                 // ---- the batch: entries s .. s+len-1, cut where a limit breaks
-                const uint32_t baseP = uniform_u32(sRelB[s].y), baseSA = uniform_u32(sRel[s].w);
+                const uint32_t baseP = uniform_u32(sRelB[s].y), baseSA = uniform_u32(sRel[s].w & kPrefixMask);
                 uint32_t len;
                 {
                     const uint32_t i = s + (uint32_t)lane;
@@ -3610,7 +3635,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                     if (i < nRel)
                     {
                         const uint32_t ni = sRel[i].y;
-                        const uint32_t sa = sRel[i].w + slot_arrays(ni) - baseSA;
+                        const uint32_t sa = (sRel[i].w & kPrefixMask) + slot_arrays(ni) - baseSA;
                         const uint32_t primsIncl = sRelB[i].y + ni - baseP;
                         stop = (sa >> 16) > (uint32_t)kAccArrays || (primsIncl > kBatchPrims && (sa & 0xffffu) > 1u);
                     }
@@ -3619,17 +3644,21 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                 }
                 const uint32_t last = s + len - 1;
                 const uint32_t nPrim = uniform_u32(sRelB[last].y + sRel[last].y - baseP);
-                const uint32_t arraysUsed = uniform_u32((sRel[last].w + slot_arrays(sRel[last].y) - baseSA) >> 16);
+                const uint32_t arraysUsed = uniform_u32(((sRel[last].w & kPrefixMask) + slot_arrays(sRel[last].y) - baseSA) >> 16);
 
                 if (arraysUsed != 0)
                 {
                     // (the arrays and sLeft are clear: set at the start and
-                    // cleared again after the previous batch's resolve)
+                    // cleared again by the previous batch's resolve)
                     for (uint32_t c0 = 0; c0 < nPrim; c0 += kBatchPrims)
                     {
                         // ---- one primitive per thread
                         const uint32_t f = c0 + (uint32_t)t;
-                        uint32_t rowsF = 0, rowsS = 0, info = 0, primIdx = 0;
+                        // rows by item class: fills, feathered segments without and
+                        // with a join end, strokes (waves then rarely mix classes)
+                        uint32_t rowsA = 0, rowsB = 0, cls = 0, info = 0, primIdx = 0;
+                        int32_t left = 0; // its left-edge winding step ...
+                        int leftRow = 0;  // ... from this row on
                         if (f < nPrim)
                         {
                             // owning entry: the last one whose first primitive is at or
@@ -3645,53 +3674,84 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                             }
                             const uint4 r = sRel[lo];
                             const uint2 rb = sRelB[lo];
-                            const uint32_t a = (r.w - baseSA) >> 16;
+                            const uint32_t a = ((r.w & kPrefixMask) - baseSA) >> 16;
                             const bool wide = r.y > kPackedPrims;
-                            const bool stroke = pathPaint[r.x].kind & 1u;
+                            const bool stroke = ((r.w >> 24) & kCellStroke) != 0u;
                             primIdx = binned[rb.x + (f - (rb.y - baseP))];
                             const Prim pm = prims[primIdx];
                             int r0, r1;
                             prim_rows(pm, g, &r0, &r1);
                             const uint32_t rows = (uint32_t)max(r1 - r0 + 1, 0);
+                            if (!stroke)
+                                left = fill_prim_left(pm, g, &leftRow);
                             if (stroke)
-                                rowsS = rows;
-                            else
-                            {
-                                rowsF = rows;
-                                fill_prim_left(pm, g, sLeft[a]);
-                            }
-                            info = a | (wide ? 16u : 0u) | (stroke ? 32u : 0u) | ((uint32_t)min(r0, kTile - 1) << 8);
+                                cls = 3;
+                            else if (FEATHER && (pm.flags & kPrimFeather))
+                                cls = (pm.flags & (kPrimJoin0 | kPrimJoin1)) ? 2 : 1;
+                            rowsA = cls < 2 ? rows << (16 * cls) : 0;
+                            rowsB = cls < 2 ? 0 : rows << (16 * (cls - 2));
+                            info = a | (wide ? 16u : 0u) | (cls << 5) | ((uint32_t)min(r0, kTile - 1) << 8);
                         }
-                        // exclusive prefix of the row counts, fills then strokes
-                        const uint32_t v = rowsF | (rowsS << 16);
-                        uint32_t inc = v;
+                        // exclusive prefix of the row counts, class after class (without
+                        // feathers only classes 0 and 3, in one word)
+                        const uint32_t vA = FEATHER ? rowsA : rowsA | rowsB, vB = rowsB;
+                        uint32_t incA = vA, incB = vB;
     #pragma unroll
                         for (int d = 1; d < 64; d <<= 1)
                         {
-                            const uint32_t a0 = (uint32_t)__shfl_up((int)inc, d);
+                            const uint32_t a0 = (uint32_t)__shfl_up((int)incA, d);
+                            const uint32_t b0 = FEATHER ? (uint32_t)__shfl_up((int)incB, d) : 0u;
                             if (lane >= d)
-                                inc += a0;
+                            {
+                                incA += a0;
+                                incB += b0;
+                            }
                         }
                         if (lane == 63)
-                            sWave[0][wave] = inc;
+                        {
+                            sWave[0][wave] = incA;
+                            if (FEATHER)
+                                sWave[1][wave] = incB;
+                        }
                         __syncthreads();
-                        uint32_t pre = 0, tot = 0;
+                        uint32_t preA = 0, totA = 0, preB = 0, totB = 0;
     #pragma unroll
                         for (int w = 0; w < kWgThreads / 64; ++w)
                         {
-                            const uint32_t x = sWave[0][w];
+                            const uint32_t x = sWave[0][w], y = FEATHER ? sWave[1][w] : 0u;
                             if (w < wave)
-                                pre += x;
-                            tot += x;
+                            {
+                                preA += x;
+                                preB += y;
+                            }
+                            totA += x;
+                            totB += y;
                         }
-                        const uint32_t ex = pre + inc - v;
-                        const uint32_t totF = tot & 0xffffu, total = uniform_u32(totF + (tot >> 16));
-                        const uint32_t item0 = rowsS != 0 ? totF + (ex >> 16) : (ex & 0xffffu);
-                        for (uint32_t k = 0; k < rowsF + rowsS; ++k)
+                        const uint32_t exA = preA + incA - vA, exB = preB + incB - vB;
+                        const uint32_t tot01 = (totA & 0xffffu) + (totA >> 16);
+                        const uint32_t total = uniform_u32(tot01 + (totB & 0xffffu) + (totB >> 16));
+                        uint32_t item0;
+                        if (!FEATHER)
+                            item0 = cls != 0 ? (totA & 0xffffu) + (exA >> 16) : (exA & 0xffffu);
+                        else if (cls < 2)
+                            item0 = cls == 0 ? (exA & 0xffffu) : (totA & 0xffffu) + (exA >> 16);
+                        else
+                            item0 = tot01 + (cls == 2 ? (exB & 0xffffu) : (totB & 0xffffu) + (exB >> 16));
+                        const uint32_t rowsAll = (vA & 0xffffu) + (vA >> 16) + (FEATHER ? (vB & 0xffffu) + (vB >> 16) : 0u);
+                        for (uint32_t k = 0; k < rowsAll; ++k)
                             sOwner[item0 + k] = (uint8_t)t;
                         sItemPrim[t] = primIdx;
                         sItemInfo[t] = info | (item0 << 16);
+                        // (every wave is past the previous batch's resolve, which
+                        // leaves sLeft clear)
+                        if (left != 0)
+                            atomicAdd(&sLeft[info & 15u][leftRow], left);
                         __syncthreads();
+                        // left-edge deltas -> prefix over rows, in place, once the
+                        // batch's last primitives are in: thread t holds array
+                        // t / 16, row t % 16, and a DPP row is one array
+                        if (c0 + kBatchPrims >= nPrim)
+                            (&sLeft[0][0])[t] = row_scan16((&sLeft[0][0])[t]);
 
                         // ---- (primitive, row) items
                         for (uint32_t it = (uint32_t)t; it < total; it += kWgThreads)
@@ -3702,27 +3762,30 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                             const int row = (int)((inf >> 8) & 15u) + (int)(it - (inf >> 16));
                             const uint32_t pIdx = sItemPrim[owner];
                             const Prim pm = prims[pIdx];
-                            if (inf & 32u)
+                            TilePrim<int32_t> np;
+                            const bool near = near_prim(pm, g, &np);
+                            int32_t* border = sAcc[a + (int)((inf >> 4) & 1u)];
+                            const int32_t unit = (inf & 16u) ? 1 : (1 << 24);
+                            if ((inf & 0x60u) == 0x60u)
                             {
+                                uint32_t* sMax = reinterpret_cast<uint32_t*>(sAcc[a]);
                                 if (FEATHER && (pm.flags & kPrimFeatherStroke))
-                                    feather_stroke_prim_row(prims, pIdx, row, g.X0, g.Y0,
-                                                            reinterpret_cast<uint32_t*>(sAcc[a]), featherTable);
+                                    feather_stroke_prim_row(prims, pIdx, row, g.X0, g.Y0, sMax, featherTable);
+                                else if (near)
+                                    stroke_row<int32_t>(np, pm.flags, pm.cov, row, sMax);
                                 else
-                                    stroke_prim_row<double>(pm, row, g, reinterpret_cast<uint32_t*>(sAcc[a]));
+                                    stroke_far_row(prims, pIdx, row, g.X0, g.Y0, sMax);
                             }
-                            else if (FEATHER && (pm.flags & kPrimFeather))
-                                feather_prim_row(prims, pIdx, row, g.X0, g.Y0, sAcc[a], sAcc[a + ((inf >> 4) & 1u)],
-                                                 (inf & 16u) ? 1 : (1 << 24), featherTable);
-                            else if (inf & 16u)
-                                fill_prim_row<double>(pm, row, g, sAcc[a], sAcc[a + 1], 1);
+                            else if (FEATHER && (inf & 0x60u) == 0x20u)
+                                feather_prim_row<false>(prims, pIdx, row, g.X0, g.Y0, sAcc[a], border, unit, featherTable);
+                            else if (FEATHER && (inf & 0x60u) == 0x40u)
+                                feather_prim_row<true>(prims, pIdx, row, g.X0, g.Y0, sAcc[a], border, unit, featherTable);
+                            else if (near)
+                                fill_row<int32_t>(np, pm.flags, row, sAcc[a], border, unit);
                             else
-                                fill_prim_row<double>(pm, row, g, sAcc[a], sAcc[a], 1 << 24);
+                                fill_far_row(prims, pIdx, row, g.X0, g.Y0, sAcc[a], border, unit);
                         }
-                        __syncthreads();
                     }
-                    // left-edge deltas -> prefix over rows, in place: thread t
-                    // holds array t / 16, row t % 16, and a DPP row is one array
-                    (&sLeft[0][0])[t] = row_scan16((&sLeft[0][0])[t]);
                     __syncthreads();
                 }
 
@@ -3740,28 +3803,27 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                     const uint32_t path = uniform_u32(rel.x);
                     const uint32_t ni = uniform_u32(rel.y);
                     const int32_t C = (int32_t)uniform_u32(rel.z);
+                    const uint32_t w = uniform_u32(rel.w), prFlags = w >> 24;
                     const PathPaint pr = pathPaint[path];
-                    const uint32_t prFlags = pr.kind & 0xffffu;
                     if (ni == 0)
                     {
                         // No primitives here: the listing keeps such a path only
                         // where its corner winding gives coverage, and an integer
                         // winding's coverage is 1 under every fill rule.
-                        if (pr.kind & kPaintPlain)
+                        if (prFlags & kCellPlain)
                             resolve_plain_full(pr, noise255, col);
-                        else if (pr.kind & kPaintFlushStart)
+                        else if (prFlags & kCellFlushStart)
                             clip = 0u;
-                        else if (!(pr.kind & kPaintNoOp))
-                            resolve_pixel(pr, raster + path, 1.f, px, py, noise255, ramps, images, col,
-                                          clip);
+                        else if (!(prFlags & kCellNoOp))
+                            resolve_pixel(pr, raster + path, 1.f, px, py, noise255, ramps, images, col, clip);
                         continue;
                     }
                     float cov;
                     {
-                        const uint32_t a = uniform_u32((rel.w - baseSA) >> 16);
+                        const uint32_t a = ((w & kPrefixMask) - baseSA) >> 16;
                         const int32_t v = sAcc[a][t];
                         sAcc[a][t] = 0;
-                        if (prFlags & 1u)
+                        if (prFlags & kCellStroke)
                             cov = fminf(__int_as_float(v), 1.f);
                         else
                         {
@@ -3779,16 +3841,17 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                                 b = (int32_t)((uint32_t)v << 8) >> 8;
                             }
                             const int32_t left = sLeft[a][t >> kTileLog2];
-                            const int32_t w = C + left + row_scan16(d);
-                            cov = fill_rule_coverage(fmaf((float)b, 1.f / 65536.f, (float)w), prFlags); // exact scaling
+                            const int32_t wind = C + left + row_scan16(d);
+                            cov = fill_rule_coverage(fmaf((float)b, 1.f / 65536.f, (float)wind), prFlags); // exact scaling
                         }
                     }
-                    if ((cov != 0.f && !(pr.kind & kPaintNoOp)) || (prFlags & 8u))
+                    if ((cov != 0.f && !(prFlags & kCellNoOp)) || (prFlags & kCellClipUpdate))
                         resolve_pixel(pr, raster + path, cov, px, py, noise255, ramps, images, col, clip);
                 }
-                __syncthreads(); // every wave has read sLeft
-                (&sLeft[0][0])[t] = 0;
-                __syncthreads(); // the next batch accumulates into the arrays and sLeft
+                // Each wave clears the rows of sLeft that only it reads; the next
+                // batch adds to them after a barrier that follows this.
+                if (arraysUsed != 0)
+                    sLeft[lane >> 2][wave * (kTile / 4) + (lane & 3)] = 0;
                 s += len;
             }
         }
@@ -3800,12 +3863,12 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
 }
 
 // Unpacks PathData/PaintData/PaintAux into PathRaster (gpu.cpp:859-1063,
-// draw_path.vert:431-545).
+// draw_path.vert:431-545) and starts each path's cell grid empty.
 __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const uint2* __restrict__ paints,
                                    const float* __restrict__ aux, const uint32_t* __restrict__ pathImage,
                                    uint32_t pathCount, const FlushDev* __restrict__ flushes, uint32_t flushCount,
-                                   PathRaster* __restrict__ out,
-                                   PathPaint* __restrict__ outPaint, uint32_t* __restrict__ clipFirst)
+                                   PathRaster* __restrict__ out, PathPaint* __restrict__ outPaint,
+                                   PathCells* __restrict__ cells, uint32_t* __restrict__ clipFirst)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // the earliest path the 64 paths of this wave read clip content from
@@ -3896,8 +3959,20 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
         pp.kind |= r.alpha != 0.f ? kPaintPlain : kPaintNoOp;
     if (plain && pp.oneMinusAlpha == 0.f && !(flags & 1u))
         pp.kind |= kPaintOpaque;
+    uint32_t cellFlags = (flags & 15u) | ((pp.kind & kPaintPlain) ? kCellPlain : 0u) |
+                         ((pp.kind & kPaintNoOp) ? kCellNoOp : 0u);
+    // The reserved record of a flush after the launch's first: the clip buffer
+    // starts empty there, since each flush numbers its clip IDs from 1.
     if (i != 0u && fl.pathBase == i)
-        pp.kind = kPaintFlushStart | 8u;
+        cellFlags = kCellFlushStart;
+    PathCells c;
+    c.tx0 = c.ty0 = 0x7fffffff;
+    c.tx1 = c.ty1 = -0x7fffffff;
+    c.base = 0;
+    c.width = 0;
+    c.flags = cellFlags;
+    c.pad = 0;
+    cells[i] = c;
     outPaint[i] = pp;
 }
 
