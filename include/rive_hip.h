@@ -457,7 +457,9 @@ int rive_hip_last_flush_stats(rive_hip_context* ctx, rive_hip_flush_stats* out);
 /* How the raster pass runs on this context.  No counterpart in the reference
  * (its raster is the GPU's fixed-function pipeline); these are the launch
  * choices of the tile raster, set by hand or by rive_hip_autotune_frame.
- * Every choice renders the same pixels.
+ * Every choice renders the same pixels.  A new context has {0, 0, 6, 0}, with
+ * the tile order left to the library (heaviest first where a launch has more
+ * tiles than run at once) until one is set.
  *  tile_order     0: tiles in canvas/row/column order; 1: heaviest first (a
  *                 per-tile cost estimate from the binning, two small kernels).
  *  persistent     0: one workgroup per tile; 1: a resident grid (waves_per_simd
