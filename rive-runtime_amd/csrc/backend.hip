@@ -104,7 +104,7 @@ struct rive_hip_context
     // pipeline scratch (grow-only)
     DevBuf spanTexelCounts, spanTexelOffsets, scanPartials, scalars;
     DevBuf tess, prims, cells, cellCursor, binned, cellPacked, pathDraws, pathBins, pathBase;
-    DevBuf pathRaster, pathPaint, ramps, drawTess, verts;
+    DevBuf pathRaster, pathPaint, ramps, drawTess, primFlags, primCov;
     DevBuf geoCounts, geoRecords, geoContours, geoSpans, geoSpanCounts, geoSpanOffsets;
     uint32_t lastMode = 0, lastRecordCount = 0, lastTessVertexCount = 0;
     uint32_t* hostScalars = nullptr; // pinned
@@ -199,7 +199,7 @@ struct rive_hip_context
 namespace
 {
 // The scratch buffers of a context (every DevBuf member), in one list.
-constexpr int kDevBufCount = 41;
+constexpr int kDevBufCount = 42;
 // The device scalars of a flush (totals, counters), 32 words: the pipeline
 // uses slots 0-7, device counting 8-13, guard-box pieces kFarSlot .. +3.
 constexpr size_t kScalarBytes = 128;
@@ -212,7 +212,7 @@ void devbufs(rive_hip_context* c, DevBuf** out)
                                  &c->cellCursor, &c->binned, &c->pathRaster,
                                  &c->ramps, &c->drawTess, &c->geoCounts, &c->geoRecords,
                                  &c->geoContours, &c->geoSpans, &c->geoSpanCounts, &c->geoSpanOffsets,
-                                 &c->verts, &c->imageTable, &c->pathImage, &c->launchTable,
+                                 &c->primFlags, &c->primCov, &c->imageTable, &c->pathImage, &c->launchTable,
                                  &c->pathCanvas, &c->cellPacked, &c->pathDraws, &c->pathPaint,
                                  &c->patchTable, &c->patchWork, &c->specialList, &c->farList, &c->drawPieces,
                                  &c->drawPieceOffset, &c->pieceCursor, &c->drawTessAll, &c->tileClass,
@@ -1371,25 +1371,23 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
         P<PathPaint>(ctx->pathPaint), P<PathCells>(ctx->cells), P<uint32_t>(ctx->clipFirst));
     RIVE_TRY(ensure(ctx, ctx->tileCover, (size_t)std::max<uint32_t>(tileTotal, 1) * 4));
     RIVE_TRY(clear(ctx, ctx->tileCover.ptr, 0, (size_t)tileTotal * 4));
-    RIVE_TRY(ensure(ctx, ctx->prims, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(Prim)));
-    RIVE_TRY(ensure(ctx, ctx->verts, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(VtxPair)));
-    if (totalPrims > 0)
-        vertex_kernel<<<(totalPrims + 255) / 256, 256, 0, ctx->stream>>>(
-            P<TessTexel>(ctx->tess), g.flushes, paths, drawTess, drawCount, totalPrims, P<VtxPair>(ctx->verts));
+    RIVE_TRY(ensure(ctx, ctx->prims, (size_t)std::max<uint32_t>(totalPrims, 1) * 2 * sizeof(int4)));
+    RIVE_TRY(ensure(ctx, ctx->primFlags, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->primCov, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(PrimCov)));
+    PrimStore prims{P<int4>(ctx->prims), P<uint32_t>(ctx->primFlags), P<PrimCov>(ctx->primCov)};
     RIVE_TRY(ensure(ctx, ctx->specialList, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->farList, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->drawPieces, (size_t)(drawCount + 1) * 4));
     RIVE_TRY(clear(ctx, ctx->drawPieces.ptr, 0, (size_t)(drawCount + 1) * 4));
     if (totalPrims > 0)
     {
-        expand_kernel<<<(totalPrims + 255) / 256, 256, 0, ctx->stream>>>(
-            P<TessTexel>(ctx->tess), g.flushes, P<VtxPair>(ctx->verts), contours, paths,
-            drawTess, drawCount, totalPrims, P<Prim>(ctx->prims), P<PathCells>(ctx->cells), scal + 5,
-            P<uint32_t>(ctx->specialList), scal + kFarSlot + 3);
+        expand_kernel<<<(totalPrims - 1) / kExpandPrims + 1, kExpandThreads, 0, ctx->stream>>>(
+            P<TessTexel>(ctx->tess), g.flushes, contours, paths, drawTess, drawCount, totalPrims, prims,
+            P<PathCells>(ctx->cells), scal + 5, P<uint32_t>(ctx->specialList), scal + kFarSlot + 3);
         // a grid-stride pass over the set-aside primitives (usually none)
         special_prims_kernel<<<64, 256, 0, ctx->stream>>>(
             P<TessTexel>(ctx->tess), g.flushes, contours, paths, drawTess, drawCount,
-            P<Prim>(ctx->prims), P<PathCells>(ctx->cells), P<uint32_t>(ctx->specialList), scal + kFarSlot + 3,
+            prims, P<PathCells>(ctx->cells), P<uint32_t>(ctx->specialList), scal + kFarSlot + 3,
             P<uint32_t>(ctx->farList), scal + kFarSlot, P<uint32_t>(ctx->drawPieces));
     }
     cells_layout_kernel<<<1, 1024, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
@@ -1425,8 +1423,11 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     uint32_t binDrawCount = drawCount;
     if (pieces > 0)
     {
-        RIVE_TRY(grow_keep(ctx, ctx->prims, (size_t)totalPrims * sizeof(Prim),
-                           (size_t)(totalPrims + pieces) * sizeof(Prim)));
+        const size_t all = (size_t)totalPrims + pieces;
+        RIVE_TRY(grow_keep(ctx, ctx->prims, (size_t)totalPrims * 2 * sizeof(int4), all * 2 * sizeof(int4)));
+        RIVE_TRY(grow_keep(ctx, ctx->primFlags, (size_t)totalPrims * 4, all * 4));
+        RIVE_TRY(grow_keep(ctx, ctx->primCov, (size_t)totalPrims * sizeof(PrimCov), all * sizeof(PrimCov)));
+        prims = {P<int4>(ctx->prims), P<uint32_t>(ctx->primFlags), P<PrimCov>(ctx->primCov)};
         RIVE_TRY(ensure(ctx, ctx->drawPieceOffset, (size_t)(drawCount + 1) * 4));
         RIVE_TRY(ensure(ctx, ctx->pieceCursor, (size_t)(drawCount + 1) * 4));
         RIVE_TRY(ensure(ctx, ctx->drawTessAll, (size_t)drawCount * 2 * sizeof(DrawTess)));
@@ -1436,7 +1437,7 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
         if (rc)
             return rc;
         far_pieces_kernel<<<(farPrims + 255) / 256, 256, 0, ctx->stream>>>(
-            P<Prim>(ctx->prims), P<uint32_t>(ctx->farList), scal + kFarSlot, drawTess, drawCount,
+            prims, P<uint32_t>(ctx->farList), scal + kFarSlot, drawTess, drawCount,
             P<uint32_t>(ctx->drawPieceOffset), P<uint32_t>(ctx->pieceCursor), totalPrims);
         piece_draws_kernel<<<(drawCount + 255) / 256, 256, 0, ctx->stream>>>(
             drawTess, drawCount, P<uint32_t>(ctx->drawPieces), P<uint32_t>(ctx->drawPieceOffset), totalPrims,
@@ -1463,12 +1464,12 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     if (bin)
     {
         bin_count_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
-            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
+            prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
             P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
             P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
         if (largeCells > smallCells)
             bin_count_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
-                P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
+                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
                 largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
                 P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
     }
@@ -1479,7 +1480,7 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
                                                                     P<uint32_t>(ctx->pathDraws),
                                                                     P<uint2>(ctx->cellPacked),
                                                                     P<uint32_t>(ctx->cellCursor));
-        shared_count_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(P<Prim>(ctx->prims), binDraws,
+        shared_count_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(prims, binDraws,
                                                                    P<PathCells>(ctx->cells),
                                                                    P<uint32_t>(ctx->pathDraws),
                                                                    P<uint2>(ctx->cellPacked));
@@ -1506,20 +1507,20 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     if (bin)
     {
         bin_scatter_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
-            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
+            prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
             P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
             P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
             P<uint32_t>(ctx->binned));
         if (largeCells > smallCells)
             bin_scatter_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
-                P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
+                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
                 largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
                 P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
                 P<uint32_t>(ctx->binned));
     }
     if (bin && shared)
         shared_scatter_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
-            P<Prim>(ctx->prims), binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws),
+            prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws),
             P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->cellCursor),
             P<uint32_t>(ctx->binned));
     HIP_TRY(hipGetLastError());
@@ -1566,7 +1567,7 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
         raster_fn(feathered, persistent, waves)<<<grid, kWgThreads, 0, ctx->stream>>>(
             P<PathCells>(ctx->cells), P<PathRaster>(ctx->pathRaster), P<PathPaint>(ctx->pathPaint),
             P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
-            P<uint32_t>(ctx->binned), P<Prim>(ctx->prims),
+            P<uint32_t>(ctx->binned), prims,
             P<uint32_t>(ctx->ramps), P<ImageDesc>(ctx->imageTable), canvases,
             canvasCount, P<uint32_t>(ctx->tileCover), P<uint32_t>(ctx->clipFirst), d->dither, ctx->featherTables, order, tileTotal, queue + 2 * kCostClasses);
     }
@@ -2089,7 +2090,7 @@ int flush_impl(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t
 // in the mapped buffers, the later ones loading it.  Grouping matters beyond
 // the launches it saves: an opaque fill hides what earlier flushes of the group
 // drew under it too.  The group's buffers are bounded by kGroupBytes: 16 B a
-// texel, 120 B a primitive (at most one a texel) and 8 B a (path, tile) cell
+// texel, 92 B a primitive (at most one a texel) and 8 B a (path, tile) cell
 // -- an eighth of the card's memory; a 4K frame of 20 000 draws counts 26 GB,
 // and a longer one runs in several groups.  Measured on MI355X: the 1080p
 // 5000-path frame (6 flushes) 19.4 -> 11.6 ms, the 4K 20 000-draw frame (35
@@ -2119,7 +2120,7 @@ uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs
         texels += (uint64_t)layouts[e].tessRows * kTessTextureWidth;
         paths += (uint64_t)d.path_count + 1u;
         images += d.image_count;
-        if (e > k && (texels * 136u + paths * tiles * 8u > kGroupBytes || texels > kMaxFlushTexels ||
+        if (e > k && (texels * 108u + paths * tiles * 8u > kGroupBytes || texels > kMaxFlushTexels ||
                       paths > kMaxFlushPaths || images > 0xffffu || paths * (tiles + 1u) >= 0xffffffffu))
             break;
     }

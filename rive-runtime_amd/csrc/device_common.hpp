@@ -63,11 +63,59 @@ struct Prim
 {
     int32_t p[8];
     float cov[8];
-    uint32_t path;  // 1-based path ID
-    uint32_t flags; // kPrimFill / kPrimStroke / kPrimNegate / kPrimEmpty
+    uint32_t flags; // kPrim*
     uint32_t pad[2];
 };
-static_assert(sizeof(Prim) == 80, "Prim is 80 bytes");
+// Where primitives live in device memory: the vertices and the flags, which
+// every pass reads (36 bytes a primitive), apart from the coverages, which only
+// the rows of strokes and feathered segments do.
+struct alignas(16) PrimCov
+{
+    float cov[8];
+    uint32_t pad[4];
+};
+struct PrimStore
+{
+    int4* geo; // two per primitive
+    uint32_t* flags;
+    PrimCov* cov;
+
+    __device__ __forceinline__ Prim load(uint32_t g) const
+    {
+        Prim p;
+        const int4 a = geo[2 * (size_t)g], b = geo[2 * (size_t)g + 1];
+        p.p[0] = a.x, p.p[1] = a.y, p.p[2] = a.z, p.p[3] = a.w;
+        p.p[4] = b.x, p.p[5] = b.y, p.p[6] = b.z, p.p[7] = b.w;
+        p.flags = flags[g];
+        return p;
+    }
+    __device__ __forceinline__ void load_cov(uint32_t g, Prim* p) const
+    {
+        const PrimCov c = cov[g];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            p->cov[k] = c.cov[k];
+        p->pad[0] = c.pad[0];
+        p->pad[1] = c.pad[1];
+    }
+    __device__ __forceinline__ void store(uint32_t g, const Prim& p) const
+    {
+        geo[2 * (size_t)g] = make_int4(p.p[0], p.p[1], p.p[2], p.p[3]);
+        geo[2 * (size_t)g + 1] = make_int4(p.p[4], p.p[5], p.p[6], p.p[7]);
+        flags[g] = p.flags;
+    }
+    __device__ __forceinline__ void store_cov(uint32_t g, const Prim& p) const
+    {
+        PrimCov c;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            c.cov[k] = p.cov[k];
+        c.pad[0] = p.pad[0];
+        c.pad[1] = p.pad[1];
+        c.pad[2] = c.pad[3] = 0u;
+        cov[g] = c;
+    }
+};
 constexpr uint32_t kPrimFill = 1u;
 constexpr uint32_t kPrimStroke = 2u;
 constexpr uint32_t kPrimNegate = 4u;
