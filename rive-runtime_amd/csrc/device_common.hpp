@@ -1,6 +1,7 @@
 // Shared device-side definitions of the gfx950 backend.
 #pragma once
 
+#include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -167,6 +168,25 @@ __device__ __forceinline__ float feather_table(const float* __restrict__ t, floa
     const int l = max(r - 1, 0);
     const float w = fminf(fmaxf(u - (float)l, 0.f), 1.f);
     return t[l] * (1.f - w) + t[r] * w;
+}
+
+// The table as the raster holds it in LDS: word r is the texel pair (r - 1, r)
+// in fp16, which is what the texels are, so a sample is one 32-bit read; the
+// same value as feather_table's.
+__device__ __forceinline__ uint32_t feather_pair(const float* __restrict__ t, int r)
+{
+    const uint32_t lo = (uint32_t)__half_as_ushort(__float2half_rn(t[max(r - 1, 0)]));
+    return lo | ((uint32_t)__half_as_ushort(__float2half_rn(t[r])) << 16);
+}
+__device__ __forceinline__ float feather_table(const uint32_t* __restrict__ pairs, float x)
+{
+    x = fminf(fmaxf(x, 0.f), 1.f); // NaN -> 0
+    const float u = x * (float)kFeatherTableSize - .5f;
+    const int r = (int)fminf(u + 1.f, (float)(kFeatherTableSize - 1));
+    const uint32_t p = pairs[r];
+    const float w = fminf(fmaxf(u - (float)max(r - 1, 0), 0.f), 1.f);
+    return __half2float(__ushort_as_half((unsigned short)p)) * (1.f - w) +
+           __half2float(__ushort_as_half((unsigned short)(p >> 16))) * w;
 }
 
 // Per-path raster parameters, unpacked from PathData/PaintData/PaintAux.
