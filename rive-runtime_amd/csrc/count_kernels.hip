@@ -119,17 +119,7 @@ __device__ __forceinline__ void push_cubic(Emit* e, const V2d* pts, V2d jt, uint
 // triangulated ones 1.00 -> .21 ms, 700 feathered ones 1.47 -> .24 ms, 20 000
 // draws 2.2 -> .58 ms, 21 652 fills of 8-32 cubics (where the threads already
 // filled the chip) .237 -> .220 ms.
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
-{
-#pragma unroll
-    for (int k = 32; k > 0; k >>= 1)
-        v += (uint32_t)__shfl_xor((int)v, k);
-    return v;
-}
-__device__ __forceinline__ uint32_t wave_excl(uint32_t v, int lane)
-{
-    return (uint32_t)wave_scan_add((int32_t)v, lane) - v;
-}
+__device__ __forceinline__ uint32_t wave_excl(uint32_t v) { return (uint32_t)wave_scan_add((int32_t)v) - v; }
 __device__ __forceinline__ V2d shfl_v2(V2d v, int lane) { return V2d{__shfl(v.x, lane), __shfl(v.y, lane)}; }
 // The highest lane below this one in the mask, -1 if none.
 __device__ __forceinline__ int lane_before(uint64_t mask, int lane)
@@ -172,7 +162,7 @@ __device__ DrawCounts walk_outer_draw(const rive_hip_draw& d, const uint8_t* __r
     {
         const uint32_t k = k0 + (uint32_t)lane;
         const uint32_t v = k < d.verb_count ? verbs[k] : 255u;
-        const uint32_t np = verb_points(v), pi = pointBase + wave_excl(np, lane);
+        const uint32_t np = verb_points(v), pi = pointBase + wave_excl(np);
         const uint64_t moves = __ballot(v == 0u);
         // the contour this verb closes (a move) or belongs to: its index from 1
         // and its first point
@@ -192,7 +182,7 @@ __device__ DrawCounts walk_outer_draw(const rive_hip_draw& d, const uint8_t* __r
             n = (uint32_t)sclamp(ceilf(w * (1.f / kSpan)), 1.f, (float)kMaxSubdivisions);
             recs = n == 1u ? 1u : n + (n + 1u) / 3u;
         }
-        const uint32_t rec0 = wave_excl(recs, lane);
+        const uint32_t rec0 = wave_excl(recs);
         const uint32_t chunkRecs = (uint32_t)__shfl((int)(rec0 + recs), 63);
         if (EMIT)
         {
@@ -354,7 +344,7 @@ __device__ DrawCounts walk_draw(const rive_hip_draw& d, const uint8_t* __restric
         {
             const uint32_t k = k0 + (uint32_t)lane;
             const uint32_t v = k < ce ? verbs[k] : 255u;
-            const uint32_t np = verb_points(v), q = qBase + wave_excl(np, lane);
+            const uint32_t np = verb_points(v), q = qBase + wave_excl(np);
             const bool isLine = v == 1u, isCubic = v == 4u;
             const uint64_t drawn = __ballot(isLine || isCubic);
             const V2d* cp = P + q - 1;
@@ -570,7 +560,7 @@ __device__ DrawCounts walk_draw(const rive_hip_draw& d, const uint8_t* __restric
             {
                 const uint32_t k = k0 + (uint32_t)lane;
                 const uint32_t vb = k < ce ? verbs[k] : 255u;
-                const uint32_t np = verb_points(vb), q = qb + wave_excl(np, lane);
+                const uint32_t np = verb_points(vb), q = qb + wave_excl(np);
                 const bool drawsVerb = vb == 1u || vb == 4u;
                 const uint64_t drawn = __ballot(drawsVerb);
                 const int from = lane_before(drawn, lane);
@@ -670,7 +660,7 @@ __device__ DrawCounts walk_draw(const rive_hip_draw& d, const uint8_t* __restric
                 if (drawsVerb)
                     records(&le, std::false_type());
                 const uint32_t nRec = le.rec, texels = le.fwd;
-                const uint32_t rec0 = wave_excl(nRec, lane), texel0 = wave_excl(texels, lane);
+                const uint32_t rec0 = wave_excl(nRec), texel0 = wave_excl(texels);
                 const uint32_t chunkRecs = (uint32_t)__shfl((int)(rec0 + nRec), 63);
                 const uint32_t chunkTexels = (uint32_t)__shfl((int)(texel0 + texels), 63);
                 if (drawsVerb)

@@ -1466,20 +1466,16 @@ __global__ __launch_bounds__(kExpandThreads) void expand_kernel(
         ty1 = (maxy >> (kSubpixelLog2 + kTileLog2)) + 1;
     }
     const int lane = threadIdx.x & 63;
-    const uint32_t wavePath = (uint32_t)__shfl((int)d.pathID, 0);
+    const uint32_t wavePath = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.pathID);
     const bool same = !makes || d.pathID == wavePath;
     const uint64_t sameMask = __ballot(same);
     if (sameMask == ~0ull)
     {
         // the whole wave (all 64 lanes active) belongs to one path
-#pragma unroll
-        for (int k = 32; k > 0; k >>= 1)
-        {
-            tx0 = min(tx0, __shfl_xor(tx0, k));
-            ty0 = min(ty0, __shfl_xor(ty0, k));
-            tx1 = max(tx1, __shfl_xor(tx1, k));
-            ty1 = max(ty1, __shfl_xor(ty1, k));
-        }
+        tx0 = wave_min(tx0);
+        ty0 = wave_min(ty0);
+        tx1 = -wave_min(-tx1);
+        ty1 = -wave_min(-ty1);
         if (lane == 0 && tx0 < tx1)
         {
             PathCells* pc = &cells[d.pathID];
@@ -1950,18 +1946,6 @@ __global__ void path_draws_kernel(const DrawTess* __restrict__ draws, uint32_t d
         *anyShared = 1u; // every writer stores the same value
 }
 
-__device__ __forceinline__ int32_t wave_scan_add(int32_t v, int lane)
-{
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1)
-    {
-        const int32_t t = __shfl_up(v, d);
-        if (lane >= d)
-            v += t;
-    }
-    return v;
-}
-
 // One workgroup per draw of a solo path whose grid has [minCells, maxCells]
 // cells (LDS: one word per cell).  The word holds the primitive count in its
 // low 16 bits and the corner-crossing sum, two's complement, in the high 16: a
@@ -2019,14 +2003,14 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
         {
             const uint32_t x = x0 + (uint32_t)lane;
             const uint32_t w = x < c.width ? sCell[r * c.width + x] : 0u;
-            const int32_t v = wave_scan_add((int32_t)w >> 16, lane) + carry;
+            const int32_t v = wave_scan_add((int32_t)w >> 16) + carry;
             if (x < c.width)
             {
                 sCell[r * c.width + x] = (w & 0xffffu) | ((uint32_t)v << 16);
                 if (opaque && (w & 0xffffu) == 0u && v != 0 && fill_rule_coverage((float)v, kind) != 0.f)
                     atomicMax(&cover[r * coverStride + x], d.pathID);
             }
-            carry = __shfl(v, 63);
+            carry = wave_last(v);
         }
     }
     __syncthreads();
@@ -2037,9 +2021,7 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
     uint32_t sum = 0;
     for (uint32_t i = first + (uint32_t)lane; i < end; i += 64u)
         sum += sCell[i] & 0xffffu;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1)
-        sum += (uint32_t)__shfl_xor((int)sum, s);
+    sum = wave_sum(sum);
     if (lane == 0)
         sWaveSum[wave] = sum;
     __syncthreads();
@@ -2053,10 +2035,10 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
     {
         const uint32_t i = i0 + (uint32_t)lane;
         const uint32_t w = i < end ? sCell[i] : 0u;
-        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)(w & 0xffffu), lane);
+        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)(w & 0xffffu));
         if (i < end)
             packed[c.base + i] = make_uint2(carry + incl - (w & 0xffffu), (uint32_t)((int32_t)w >> 16));
-        carry += (uint32_t)__shfl((int)incl, 63);
+        carry += (uint32_t)wave_last((int32_t)incl);
     }
     if (threadIdx.x == 0)
     {
@@ -2167,10 +2149,10 @@ __global__ __launch_bounds__(256) void shared_layout_kernel(const PathCells* __r
         for (uint32_t x0 = 0; x0 < c.width; x0 += 64)
         {
             const uint32_t x = x0 + (uint32_t)lane;
-            const int32_t v = wave_scan_add(x < c.width ? (int32_t)grid[r * c.width + x].y : 0, lane) + carry;
+            const int32_t v = wave_scan_add(x < c.width ? (int32_t)grid[r * c.width + x].y : 0) + carry;
             if (x < c.width)
                 grid[r * c.width + x].y = (uint32_t)v;
-            carry = __shfl(v, 63);
+            carry = wave_last(v);
         }
     }
     // counts -> offsets, 256 cells per step; a total beyond 2^32-1 saturates
@@ -2180,7 +2162,7 @@ __global__ __launch_bounds__(256) void shared_layout_kernel(const PathCells* __r
     {
         const uint32_t i = i0 + threadIdx.x;
         const uint32_t v = i < nCells ? grid[i].x : 0u;
-        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)v, lane);
+        const uint32_t incl = (uint32_t)wave_scan_add((int32_t)v);
         if (lane == 63)
             sWaveSum[wave] = incl;
         __syncthreads();
@@ -3349,17 +3331,6 @@ __device__ __forceinline__ uint32_t uniform_u32(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-// Inclusive prefix sum within each DPP row of 16 lanes (row_shr:1, 2, 4, 8;
-// lanes shifted in from outside the row read 0).  All 64 lanes must be active.
-__device__ __forceinline__ int32_t row_scan16(int32_t x)
-{
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
-    return x;
-}
-
 // Accumulator arrays a path with n primitives in the tile needs, packed with
 // a slot count of one: slots | arrays << 16.
 __device__ __forceinline__ uint32_t slot_arrays(uint32_t n)
@@ -3423,9 +3394,7 @@ __global__ __launch_bounds__(256) void tile_cost_kernel(const PathCells* __restr
             cost += n != 0 ? 4u + n : (here.y != 0 ? 4u : 0u);
         }
     }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1)
-        cost += (uint32_t)__shfl_xor((int)cost, d);
+    cost = wave_sum(cost);
     if (lane == 0)
     {
         const uint32_t cls = cost_class(cost);
@@ -3573,10 +3542,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
             uint32_t reach = cover;
             for (uint32_t q = (cover >> 6) + (uint32_t)lane; q <= (pathEnd - 1u) >> 6; q += 64u)
                 reach = min(reach, clipFirst[q]);
-    #pragma unroll
-            for (int k = 32; k > 0; k >>= 1)
-                reach = min(reach, (uint32_t)__shfl_xor((int)reach, k));
-            begin = max(uniform_u32(reach), pathBegin);
+            begin = max((uint32_t)wave_min((int32_t)min(reach, 0x7fffffffu)), pathBegin);
         }
         for (uint32_t base = begin; base < pathEnd; base += kWindow)
         {
@@ -3608,17 +3574,7 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                 }
             }
             const uint32_t vSA = slot_arrays(n);
-            uint32_t iSA = vSA, iP = n;
-    #pragma unroll
-            for (int d = 1; d < 64; d <<= 1)
-            {
-                const uint32_t a0 = (uint32_t)__shfl_up((int)iSA, d), a1 = (uint32_t)__shfl_up((int)iP, d);
-                if (lane >= d)
-                {
-                    iSA += a0;
-                    iP += a1;
-                }
-            }
+            const uint32_t iSA = (uint32_t)wave_scan_add((int32_t)vSA), iP = (uint32_t)wave_scan_add((int32_t)n);
             const uint64_t bal = __ballot(listed);
             const uint32_t posInWave = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
             if (lane == 63)
@@ -3720,18 +3676,8 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
                         // exclusive prefix of the row counts, class after class (without
                         // feathers only classes 0 and 3, in one word)
                         const uint32_t vA = FEATHER ? rowsA : rowsA | rowsB, vB = rowsB;
-                        uint32_t incA = vA, incB = vB;
-    #pragma unroll
-                        for (int d = 1; d < 64; d <<= 1)
-                        {
-                            const uint32_t a0 = (uint32_t)__shfl_up((int)incA, d);
-                            const uint32_t b0 = FEATHER ? (uint32_t)__shfl_up((int)incB, d) : 0u;
-                            if (lane >= d)
-                            {
-                                incA += a0;
-                                incB += b0;
-                            }
-                        }
+                        const uint32_t incA = (uint32_t)wave_scan_add((int32_t)vA);
+                        const uint32_t incB = FEATHER ? (uint32_t)wave_scan_add((int32_t)vB) : vB;
                         if (lane == 63)
                         {
                             sWave[0][wave] = incA;
@@ -3913,9 +3859,7 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // the earliest path the 64 paths of this wave read clip content from
     uint32_t reach = i <= pathCount ? clip_reach(paints, i) : 0xffffffffu;
-#pragma unroll
-    for (int k = 32; k > 0; k >>= 1)
-        reach = min(reach, (uint32_t)__shfl_xor((int)reach, k));
+    reach = (uint32_t)wave_min((int32_t)min(reach, 0x7fffffffu));
     if ((threadIdx.x & 63) == 0 && i <= pathCount)
         clipFirst[i >> 6] = reach;
     if (i > pathCount)
