@@ -1457,22 +1457,43 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(ensure(ctx, ctx->pathBins, (size_t)(pathCount + 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->pathBase, (size_t)(pathCount + 2) * 4));
     RIVE_TRY(clear(ctx, ctx->pathBins.ptr, 0, (size_t)(pathCount + 1) * 4));
-    // The solo kernels' LDS: as many words as the largest canvas has tiles,
-    // up to the small limit; a second launch takes the larger grids.
+    // The solo kernels' LDS: as many words as the largest canvas has tiles, up to
+    // the small limit; a second launch takes the larger grids.  A CU holds 32
+    // waves: 8 workgroups of 256 threads, or fewer of 512 or 1024 where the draws
+    // or the LDS allow no more.  Measured on MI355X, both kernels, 256 threads
+    // against the form taken here: 5000 draws of up to 8160 cells 1.11 -> .83 ms
+    // (512), 722 draws .24 -> .13 ms (512), 200 draws .157 -> .107 ms (1024).
     const bool bin = totalPrims > 0 && drawCount > 0 && totalCells > 0;
-    const uint32_t smallCells = std::min(maxTiles, kBinSmallCells), largeCells = std::min(maxTiles, kBinLargeCells);
-    if (bin)
-    {
-        bin_count_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
-            prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
-            P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
-            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
+    const uint32_t largeCells = std::min(maxTiles, kBinLargeCells);
+    const uint32_t cus = (uint32_t)std::max(ctx->cuCount, 1);
+    const uint32_t smallCells = binDrawCount > 2u * cus ? std::min(maxTiles, kBinSmallCells) : 0u;
+    const auto solo = [&](auto&& launch256, auto&& launch512, auto&& launch1024) {
+        if (smallCells > kBinFewCells || (smallCells != 0 && binDrawCount <= 8u * cus))
+            launch512(binDrawCount, 512u, smallCells * 4u, 1u, smallCells);
+        else if (smallCells != 0)
+            launch256(binDrawCount, 256u, smallCells * 4u, 1u, smallCells);
         if (largeCells > smallCells)
-            bin_count_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
-                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
-                largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
-                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
-    }
+            launch1024(binDrawCount, 1024u, largeCells * 4u, smallCells + 1u, largeCells);
+    };
+    const auto count = [&](auto kernel) {
+        return [&, kernel](uint32_t blocks, uint32_t threads, uint32_t lds, uint32_t minCells, uint32_t maxCells) {
+            kernel<<<blocks, threads, lds, ctx->stream>>>(
+                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), minCells, maxCells,
+                P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases, P<uint2>(ctx->cellPacked),
+                P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
+        };
+    };
+    const auto scatter = [&](auto kernel) {
+        return [&, kernel](uint32_t blocks, uint32_t threads, uint32_t lds, uint32_t minCells, uint32_t maxCells) {
+            kernel<<<blocks, threads, lds, ctx->stream>>>(
+                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), minCells, maxCells,
+                P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases, P<uint32_t>(ctx->tileCover),
+                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+        };
+    };
+    if (bin)
+        solo(count(&bin_count_solo_kernel<256>), count(&bin_count_solo_kernel<512>),
+             count(&bin_count_solo_kernel<1024>));
     if (bin && shared)
     {
         RIVE_TRY(ensure(ctx, ctx->cellCursor, (size_t)totalCells * 4));
@@ -1505,19 +1526,8 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     ctx->stats.tile_count = tileTotal;
     RIVE_TRY(ensure(ctx, ctx->binned, (size_t)std::max<uint32_t>(totalPairs, 1) * 4));
     if (bin)
-    {
-        bin_scatter_solo_kernel<256><<<binDrawCount, 256, smallCells * 4, ctx->stream>>>(
-            prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), 1u, smallCells,
-            P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
-            P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
-            P<uint32_t>(ctx->binned));
-        if (largeCells > smallCells)
-            bin_scatter_solo_kernel<1024><<<binDrawCount, 1024, largeCells * 4, ctx->stream>>>(
-                prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), smallCells + 1u,
-                largeCells, P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases,
-                P<uint32_t>(ctx->tileCover), P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase),
-                P<uint32_t>(ctx->binned));
-    }
+        solo(scatter(&bin_scatter_solo_kernel<256>), scatter(&bin_scatter_solo_kernel<512>),
+             scatter(&bin_scatter_solo_kernel<1024>));
     if (bin && shared)
         shared_scatter_kernel<<<binDrawCount, 256, 0, ctx->stream>>>(
             prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws),

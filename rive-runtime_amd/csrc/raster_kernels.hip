@@ -1788,15 +1788,6 @@ __device__ __forceinline__ bool slab_extent(const float (&u)[4], const float (&v
     return rlo <= rhi;
 }
 
-// "q right of edge a->b" for the ray-left crossing rule, with the sample point
-// perturbed by (+e, +e^2): s*D(q) >= 0 where s = +1 for upward edges.
-__device__ __forceinline__ bool right_of(int32_t ax, int32_t ay, int32_t bx, int32_t by, int64_t qx,
-                                         int64_t qy)
-{
-    int64_t D = (int64_t)(bx - ax) * (qy - ay) - (int64_t)(by - ay) * (qx - ax);
-    return by < ay ? D >= 0 : D <= 0;
-}
-
 // The cells of a path's grid that primitive p can touch (row-major,
 // grid-local index), passed to visit(cell).  The raster reads a tile's
 // primitives at the points of [X0, X0 + 3968] x [Y0, Y0 + 3968] (subpixels:
@@ -1859,37 +1850,121 @@ __device__ __forceinline__ void for_prim_cells(const Prim& p, const PathCells& c
     }
 }
 
+// The first tile-row line of the grid that a fill primitive's inner edge
+// I0->I1 crosses (ymin <= Y < ymax), c.ty1 if it crosses none.
+__device__ __forceinline__ int first_crossing(const Prim& p, const PathCells& c)
+{
+    if (!(p.flags & kPrimFill) || (p.flags & kPrimNoEdge))
+        return c.ty1;
+    const int32_t ymin = min(p.p[1], p.p[5]), ymax = max(p.p[1], p.p[5]);
+    const int unit = 1 << (kSubpixelLog2 + kTileLog2);
+    const int ty = max(c.ty0, (ymin + unit - 1) >> (kSubpixelLog2 + kTileLog2));
+    return ty < c.ty1 && ty * unit < ymax ? ty : c.ty1;
+}
+
 // Corner crossings of a fill primitive's inner edge I0->I1 on tile-row lines:
-// visit(cell, +-1) at the first corner of each crossed row right of the edge.
+// visit(cell, +-1) at the first corner of each crossed row right of the edge
+// (the ray-left crossing rule, with the sample point perturbed by (+e, +e^2):
+// s*D(q) >= 0, s = +1 for upward edges).  The column comes from a float
+// quotient, within a few subpixels of the true crossing, and is settled by D in
+// double, exact for coordinates in [-2^23, 2^23).
 template <typename F>
 __device__ __forceinline__ void for_prim_crossings(const Prim& p, const PathCells& c, F visit)
 {
-    if (!(p.flags & kPrimFill) || (p.flags & kPrimNoEdge))
+    int ty = first_crossing(p, c);
+    if (ty >= c.ty1)
         return;
+    constexpr int kShift = kSubpixelLog2 + kTileLog2;
     const int32_t ax = p.p[0], ay = p.p[1], bx = p.p[4], by = p.p[5];
-    if (ay == by)
-        return;
     // NEGATE_PATH_FILL_COVERAGE negates the whole fan, backdrop included.
     const int s = (by < ay ? 1 : -1) * ((p.flags & kPrimNegate) ? -1 : 1);
-    const int32_t ymin = min(ay, by), ymax = max(ay, by);
-    const int unit = 1 << (kSubpixelLog2 + kTileLog2);
-    const int tyA = max(c.ty0, (ymin + unit - 1) >> (kSubpixelLog2 + kTileLog2));
-    for (int ty = tyA; ty < c.ty1; ++ty)
+    const double sg = by < ay ? 1. : -1.;
+    const double dx = sg * (double)(bx - ax), dy = sg * (double)(by - ay);
+    const float slope = (float)(bx - ax) * __builtin_amdgcn_rcpf((float)(by - ay));
+    const int32_t ymax = max(ay, by);
+    for (; ty < c.ty1 && (ty << kShift) < ymax; ++ty)
     {
-        const int64_t Y = (int64_t)ty * unit;
-        if (!(ymin <= Y && Y < ymax))
-            break;
-        // Smallest column c with corner (c*unit, Y) right of the edge.
-        const double xe = ax + (double)(bx - ax) * (double)(Y - ay) / (double)(by - ay);
-        int64_t cc = (int64_t)floor(xe / unit) + 1;
-        while (right_of(ax, ay, bx, by, (cc - 1) * unit, Y))
-            --cc;
-        while (!right_of(ax, ay, bx, by, cc * unit, Y))
-            ++cc;
-        const int col = (int)max<int64_t>(cc, (int64_t)c.tx0);
+        const int32_t qy = (ty << kShift) - ay;
+        const double Dy = dx * (double)qy;
+        auto right_of = [&](int col) { return Dy - dy * (double)((col << kShift) - ax) >= 0.; };
+        // Smallest column with its corner (col << kShift, Y) right of the edge.
+        int col = (int)floorf(((float)ax + slope * (float)qy) * (1.f / (float)(1 << kShift))) + 1;
+        while (right_of(col - 1))
+            --col;
+        while (!right_of(col))
+            ++col;
+        col = max(col, c.tx0);
         if (col < c.tx1)
             visit((uint32_t)(ty - c.ty0) * c.width + (uint32_t)(col - c.tx0), s);
     }
+}
+
+// Visits the cells, and with CROSS the crossings, of a draw's primitives, 64 a
+// wave at a time.  A segment of a curve lies in one tile row or column and
+// crosses no tile line, most of the time; the few that need their cells trimmed
+// row by row or a crossing settled would make every wave take both forms, so
+// each wave puts their indices aside in its part of the queue and takes them 64
+// together.  Measured on MI355X, counting and scattering kernels (with the
+// workgroup sizes the launches choose): 1080p 5000-path frame 1.15 -> .83 ms, 48
+// canvases .59 -> .51 ms, 600 triangulated draws .24 -> .13 ms, 4K 20 000-draw frame
+// 18.6 -> 18.3 ms (there nearly every segment spans rows and columns).
+constexpr uint32_t kWalkQueue = 112; // (what the largest grids leave of the LDS)
+template <int THREADS, bool CROSS, typename C, typename X>
+__device__ __forceinline__ void walk_prims(const PrimStore& prims, const DrawTess& d, const PathCells& c,
+                                           uint16_t* __restrict__ queue, C cell, X crossing)
+{
+    const int lane = threadIdx.x & 63;
+    queue += (threadIdx.x >> 6) * kWalkQueue;
+    auto whole = [&](uint32_t k) {
+        const uint32_t g = d.primBase + k;
+        const Prim p = prims.load(g);
+        for_prim_cells(p, c, [&](uint32_t at) { cell(at, g); });
+        if (CROSS)
+            for_prim_crossings(p, c, crossing);
+    };
+    uint32_t queued = 0; // the same in every lane
+    for (uint32_t k0 = threadIdx.x & ~63u; k0 < d.forwardCount; k0 += THREADS)
+    {
+        const uint32_t k = k0 + (uint32_t)lane, g = d.primBase + k;
+        bool aside = false;
+        if (k < d.forwardCount)
+        {
+            const Prim p = prims.load(g);
+            if (!(p.flags & kPrimEmpty))
+            {
+                int tx0, ty0, tx1, ty1;
+                prim_tile_range(p, c, &tx0, &ty0, &tx1, &ty1);
+                aside = (ty1 - ty0 > 1 && tx1 - tx0 > 1) || (CROSS && first_crossing(p, c) < c.ty1);
+                if (!aside)
+                    for (int ty = ty0; ty < ty1; ++ty)
+                        for (int tx = tx0; tx < tx1; ++tx)
+                            cell((uint32_t)(ty - c.ty0) * c.width + (uint32_t)(tx - c.tx0), g);
+            }
+        }
+        const uint64_t m = __ballot(aside);
+        const uint32_t n = (uint32_t)__popcll(m);
+        if (queued + n > kWalkQueue)
+        {
+            const uint32_t take = min(queued, 64u);
+            queued -= take;
+            if ((uint32_t)lane < take)
+                whole(queue[queued + (uint32_t)lane]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (aside)
+            queue[queued + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)k;
+        queued += n;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    while (queued > 64u)
+    {
+        queued -= 64u;
+        whole(queue[queued + (uint32_t)lane]);
+    }
+    if ((uint32_t)lane < queued)
+        whole(queue[lane]);
 }
 
 // ---- binning per draw
@@ -1916,9 +1991,10 @@ __device__ __forceinline__ void for_prim_crossings(const Prim& p, const PathCell
 // Other paths (several draws, as with guard-box pieces; 32768 primitives or
 // more, which the packed LDS word cannot count; grids beyond the large LDS)
 // take the shared_* kernels with global atomics.
+constexpr uint32_t kBinFewCells = 4096;
 constexpr uint32_t kBinSmallCells = 8192;
 constexpr uint32_t kBinLargeCells = 40000;
-constexpr uint32_t kBinSoloPrims = 32768;
+constexpr uint32_t kBinSoloPrims = 32768; // (the walk's queue holds 16-bit indices too)
 
 __device__ __forceinline__ uint32_t grid_cells(const PathCells& c)
 {
@@ -1962,6 +2038,7 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
 {
     extern __shared__ uint32_t sCell[];
     __shared__ uint32_t sWaveSum[THREADS / 64];
+    __shared__ uint16_t sQueue[THREADS / 64 * kWalkQueue];
     const DrawTess d = draws[blockIdx.x];
     if (d.pathID == 0u || d.forwardCount == 0u)
         return;
@@ -1974,14 +2051,9 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
     for (uint32_t i = threadIdx.x; i < nCells; i += THREADS)
         sCell[i] = 0;
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < d.forwardCount; k += THREADS)
-    {
-        const Prim p = prims.load(d.primBase + k);
-        if (p.flags & kPrimEmpty)
-            continue;
-        for_prim_cells(p, c, [&](uint32_t cell) { atomicAdd(&sCell[cell], 1u); });
-        for_prim_crossings(p, c, [&](uint32_t cell, int v) { atomicAdd(&sCell[cell], (uint32_t)v << 16); });
-    }
+    walk_prims<THREADS, true>(
+        prims, d, c, sQueue, [&](uint32_t cell, uint32_t) { atomicAdd(&sCell[cell], 1u); },
+        [&](uint32_t cell, int v) { atomicAdd(&sCell[cell], (uint32_t)v << 16); });
     __syncthreads();
     // corner windings: a prefix along each row, one wave per row; an opaque
     // fill covers the tiles without primitives that it fills
@@ -2059,6 +2131,7 @@ __global__ __launch_bounds__(THREADS) void bin_scatter_solo_kernel(
 {
     constexpr uint32_t kHidden = 0xffffffffu; // no bin has this index: totals up to it are refused
     extern __shared__ uint32_t sCell[];
+    __shared__ uint16_t sQueue[THREADS / 64 * kWalkQueue];
     const DrawTess d = draws[blockIdx.x];
     if (d.pathID == 0u || d.forwardCount == 0u)
         return;
@@ -2077,16 +2150,13 @@ __global__ __launch_bounds__(THREADS) void bin_scatter_solo_kernel(
         sCell[i] = hidden ? kHidden : base + packed[c.base + i].x;
     }
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < d.forwardCount; k += THREADS)
-    {
-        const uint32_t g = d.primBase + k;
-        const Prim p = prims.load(g);
-        if (!(p.flags & kPrimEmpty))
-            for_prim_cells(p, c, [&](uint32_t cell) {
-                if (sCell[cell] != kHidden)
-                    binned[atomicAdd(&sCell[cell], 1u)] = g;
-            });
-    }
+    walk_prims<THREADS, false>(
+        prims, d, c, sQueue,
+        [&](uint32_t cell, uint32_t g) {
+            if (sCell[cell] != kHidden)
+                binned[atomicAdd(&sCell[cell], 1u)] = g;
+        },
+        [](uint32_t, int) {});
 }
 
 // ---- paths that are not solo: counts and crossings by global atomics on the
