@@ -662,16 +662,18 @@ hipError_t image_mips(rive_hip_context* ctx, rive_hip_image* img)
 {
     const rivehip::ImageDesc& d = img->desc;
     uint32_t* texels = const_cast<uint32_t*>(d.texels);
-    hipError_t e = hipSuccess;
-    for (uint32_t l = 0; l + 1 < d.levels && e == hipSuccess; ++l)
+    for (uint32_t l = 0; l + 1 < d.levels; l += kMipStep)
     {
-        const int sw = (int)std::max(d.width >> l, 1u), sh = (int)std::max(d.height >> l, 1u);
-        const int dw = (int)std::max(d.width >> (l + 1), 1u), dh = (int)std::max(d.height >> (l + 1), 1u);
-        mip_kernel<<<dim3((dw + 63) / 64, dh), 64, 0, ctx->stream>>>(texels, d.levelOffset[l], sw, sh,
-                                                                      d.levelOffset[l + 1], dw, dh);
-        e = hipGetLastError();
+        MipLevels m{};
+        m.w = (int)std::max(d.width >> l, 1u);
+        m.h = (int)std::max(d.height >> l, 1u);
+        m.count = (int)std::min<uint32_t>(d.levels - 1u - l, kMipStep);
+        for (int k = 0; k <= m.count; ++k)
+            m.offset[k] = d.levelOffset[l + k];
+        mip_kernel<<<dim3((m.w + kMipBlock - 1) / kMipBlock, (m.h + kMipBlock - 1) / kMipBlock), 256, 0,
+                     ctx->stream>>>(texels, m);
     }
-    return e;
+    return hipGetLastError();
 }
 
 void image_free(rive_hip_image* img)
@@ -970,6 +972,12 @@ uint32_t premul_clear(uint32_t argb)
 int device_scan(rive_hip_context* ctx, const uint32_t* in, uint32_t n, uint32_t* out,
                 uint32_t* totalSlot)
 {
+    if (n <= kScanSmall)
+    {
+        scan_small_kernel<<<1, 1024, 0, ctx->stream>>>(ScanJobs{{{in, out, totalSlot}, {}, {}}}, n);
+        HIP_TRY(hipGetLastError());
+        return RIVE_HIP_OK;
+    }
     uint32_t blocks = std::max<uint32_t>((n + kScanTile - 1) / kScanTile, 1);
     RIVE_TRY(ensure(ctx, ctx->scanPartials, (size_t)blocks * 4));
     scan_reduce_kernel<<<blocks, kScanBlock, 0, ctx->stream>>>(in, n, P<uint32_t>(ctx->scanPartials));
@@ -977,6 +985,20 @@ int device_scan(rive_hip_context* ctx, const uint32_t* in, uint32_t n, uint32_t*
     scan_apply_kernel<<<blocks, kScanBlock, 0, ctx->stream>>>(in, n, P<uint32_t>(ctx->scanPartials),
                                                                totalSlot, out);
     HIP_TRY(hipGetLastError());
+    return RIVE_HIP_OK;
+}
+
+// Three scans of n values each.
+int device_scans(rive_hip_context* ctx, const ScanJobs& jobs, uint32_t n)
+{
+    if (n <= kScanSmall)
+    {
+        scan_small_kernel<<<3, 1024, 0, ctx->stream>>>(jobs, n);
+        HIP_TRY(hipGetLastError());
+        return RIVE_HIP_OK;
+    }
+    for (const ScanJob& j : jobs.job)
+        RIVE_TRY(device_scan(ctx, j.in, n, j.out, j.total));
     return RIVE_HIP_OK;
 }
 
@@ -1048,6 +1070,22 @@ __global__ void fill_u32_kernel(uint32_t* __restrict__ p, uint32_t value, size_t
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         p[i] = value;
+}
+struct FillRanges
+{
+    struct
+    {
+        uint32_t* p;
+        uint32_t n, value;
+    } range[6];
+};
+__global__ void fill_ranges_kernel(FillRanges f)
+{
+    const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+#pragma unroll
+    for (const auto& r : f.range)
+        for (uint32_t i = first; i < r.n; i += step)
+            r.p[i] = r.value;
 }
 int clear(rive_hip_context* ctx, void* ptr, uint8_t byte, size_t bytes)
 {
@@ -1359,8 +1397,22 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(mark(ctx, ctx->ev[3]));
 
     // ---- expansion + binning
+    // (what starts at a fixed value, in one launch)
+    constexpr size_t queueWords = 2 * kCostClasses + 1;
     RIVE_TRY(ensure(ctx, ctx->pathCanvas, (size_t)(pathCount + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->pathCanvas.ptr, 0xff, (size_t)(pathCount + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->tileCover, (size_t)std::max<uint32_t>(tileTotal, 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->drawPieces, (size_t)(drawCount + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->pathDraws, (size_t)(pathCount + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->pathBins, (size_t)(pathCount + 1) * 4));
+    RIVE_TRY(ensure(ctx, ctx->tileQueue, queueWords * 4));
+    const FillRanges fills{{{P<uint32_t>(ctx->pathCanvas), pathCount + 1, 0xffffffffu},
+                            {P<uint32_t>(ctx->tileCover), tileTotal, 0u},
+                            {P<uint32_t>(ctx->drawPieces), drawCount + 1, 0u},
+                            {P<uint32_t>(ctx->pathDraws), pathCount + 1, 0u},
+                            {P<uint32_t>(ctx->pathBins), pathCount + 1, 0u},
+                            {P<uint32_t>(ctx->tileQueue), (uint32_t)queueWords, 0u}}};
+    const uint32_t longest = std::max({pathCount + 1, tileTotal, drawCount + 1, (uint32_t)queueWords});
+    fill_ranges_kernel<<<std::min((longest + 255u) / 256u, 1024u), 256, 0, ctx->stream>>>(fills);
     path_canvas_kernel<<<canvasCount, 256, 0, ctx->stream>>>(canvases, P<uint32_t>(ctx->pathCanvas));
     RIVE_TRY(ensure(ctx, ctx->pathRaster, (size_t)(pathCount + 1) * sizeof(PathRaster)));
     RIVE_TRY(ensure(ctx, ctx->pathPaint, (size_t)(pathCount + 1) * sizeof(PathPaint)));
@@ -1369,16 +1421,12 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
         paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, g.flushes, g.n, P<PathRaster>(ctx->pathRaster),
         P<PathPaint>(ctx->pathPaint), P<PathCells>(ctx->cells), P<uint32_t>(ctx->clipFirst));
-    RIVE_TRY(ensure(ctx, ctx->tileCover, (size_t)std::max<uint32_t>(tileTotal, 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->tileCover.ptr, 0, (size_t)tileTotal * 4));
     RIVE_TRY(ensure(ctx, ctx->prims, (size_t)std::max<uint32_t>(totalPrims, 1) * 2 * sizeof(int4)));
     RIVE_TRY(ensure(ctx, ctx->primFlags, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->primCov, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(PrimCov)));
     PrimStore prims{P<int4>(ctx->prims), P<uint32_t>(ctx->primFlags), P<PrimCov>(ctx->primCov)};
     RIVE_TRY(ensure(ctx, ctx->specialList, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->farList, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
-    RIVE_TRY(ensure(ctx, ctx->drawPieces, (size_t)(drawCount + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->drawPieces.ptr, 0, (size_t)(drawCount + 1) * 4));
     if (totalPrims > 0)
     {
         expand_kernel<<<(totalPrims - 1) / kExpandPrims + 1, kExpandThreads, 0, ctx->stream>>>(
@@ -1393,8 +1441,6 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     cells_layout_kernel<<<1, 1024, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
                                                      P<uint32_t>(ctx->pathCanvas), canvases,
                                                      scal + 1);
-    RIVE_TRY(ensure(ctx, ctx->pathDraws, (size_t)(pathCount + 1) * 4));
-    RIVE_TRY(clear(ctx, ctx->pathDraws.ptr, 0, (size_t)(pathCount + 1) * 4));
     if (drawCount > 0)
         path_draws_kernel<<<(drawCount + 255) / 256, 256, 0, ctx->stream>>>(
             drawTess, drawCount, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), scal + kSharedSlot);
@@ -1454,9 +1500,7 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
             RIVE_TRY(fetch(ctx, ctx->hostScalars + 1, P<uint32_t>(ctx->drawPieceOffset) + last.drawBase, 4));
     }
     RIVE_TRY(ensure(ctx, ctx->cellPacked, (size_t)std::max<uint32_t>(totalCells, 1) * sizeof(uint2)));
-    RIVE_TRY(ensure(ctx, ctx->pathBins, (size_t)(pathCount + 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->pathBase, (size_t)(pathCount + 2) * 4));
-    RIVE_TRY(clear(ctx, ctx->pathBins.ptr, 0, (size_t)(pathCount + 1) * 4));
     // The solo kernels' LDS: as many words as the largest canvas has tiles, up to
     // the small limit; a second launch takes the larger grids.  A CU holds 32
     // waves: 8 workgroups of 256 threads, or fewer of 512 or 1024 where the draws
@@ -1546,9 +1590,6 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
             feathered = ctx->in.pathsHost[i].feather_radius != 0.f;
         const rive_hip_raster_config& rc = ctx->rasterConfig;
         const bool persistent = rc.persistent != 0;
-        const size_t queueBytes = (2 * kCostClasses + 1) * 4;
-        RIVE_TRY(ensure(ctx, ctx->tileQueue, queueBytes));
-        RIVE_TRY(clear(ctx, ctx->tileQueue.ptr, 0, queueBytes));
         uint32_t* queue = P<uint32_t>(ctx->tileQueue);
         const uint32_t* order = nullptr;
         // Until a config is set: heaviest tiles first wherever the launch has

@@ -1119,13 +1119,10 @@ int geometry_counting(rive_hip_context* ctx, const rive_hip_flush_desc* d, GeoLa
             ctx->bufs[RIVE_HIP_BUFFER_POINT].size / sizeof(V2d), scal + 12, tessCounts, contourCounts,
             recordCounts);
     HIP_TRY(hipGetLastError());
-    int rc = device_scan(ctx, tessCounts, n, tessOffsets, scal + 8);
-    if (rc)
-        return rc;
-    rc = device_scan(ctx, contourCounts, n, contourOffsets, scal + 9);
-    if (rc)
-        return rc;
-    rc = device_scan(ctx, recordCounts, n, recordOffsets, scal + 10);
+    const ScanJobs jobs{{{tessCounts, tessOffsets, scal + 8},
+                         {contourCounts, contourOffsets, scal + 9},
+                         {recordCounts, recordOffsets, scal + 10}}};
+    int rc = device_scans(ctx, jobs, n);
     if (rc)
         return rc;
     RIVE_TRY(fetch(ctx, ctx->hostScalars, scal + 8, 20));
@@ -1244,9 +1241,10 @@ int geometry_counting_frame(rive_hip_context* ctx, const rive_hip_flush_desc* de
             ctx->bufs[RIVE_HIP_BUFFER_POINT].size / sizeof(V2d), scal + 12, tessCounts, contourCounts,
             recordCounts);
     HIP_TRY(hipGetLastError());
-    RIVE_TRY(device_scan(ctx, tessCounts, n, tessOffsets, scal + 8));
-    RIVE_TRY(device_scan(ctx, contourCounts, n, contourOffsets, scal + 9));
-    RIVE_TRY(device_scan(ctx, recordCounts, n, recordOffsets, scal + 10));
+    const ScanJobs jobs{{{tessCounts, tessOffsets, scal + 8},
+                         {contourCounts, contourOffsets, scal + 9},
+                         {recordCounts, recordOffsets, scal + 10}}};
+    RIVE_TRY(device_scans(ctx, jobs, n));
     frame_bounds_kernel<<<1, kMaxFrameFlushes + 1, 0, ctx->stream>>>(drawBounds, tessOffsets, contourOffsets,
                                                                      recordOffsets, boundVals);
     HIP_TRY(hipGetLastError());
