@@ -1077,7 +1077,7 @@ struct FillRanges
     {
         uint32_t* p;
         uint32_t n, value;
-    } range[6];
+    } range[7];
 };
 __global__ void fill_ranges_kernel(FillRanges f)
 {
@@ -1405,12 +1405,27 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(ensure(ctx, ctx->pathDraws, (size_t)(pathCount + 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->pathBins, (size_t)(pathCount + 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->tileQueue, queueWords * 4));
+    // Until a config is set: heaviest tiles first wherever the launch has more
+    // tiles than run at once, so that long tiles do not trail (the order costs
+    // two kernels, ~15 us).  Measured on MI355X, raster pass with the order's
+    // kernels: 1080p frame 9.0 -> 7.35 ms, 48 canvases 6.6 -> 4.4 ms, 24 served
+    // requests 7.0 -> 5.4 ms, 1024^2 200-path frame .27 ms either way.
+    const uint32_t resident =
+        (uint32_t)std::max(ctx->cuCount, 1) * (ctx->rasterConfig.waves_per_simd == 5 ? 5u : 6u);
+    const bool ordered = tileTotal > 0 && (ctx->rasterConfigSet ? ctx->rasterConfig.tile_order != 0 : tileTotal > resident);
+    if (ordered)
+    {
+        RIVE_TRY(ensure(ctx, ctx->tileClass, (size_t)tileTotal * 4));
+        RIVE_TRY(ensure(ctx, ctx->tileOrder, (size_t)tileTotal * 4));
+    }
+    uint32_t* tileClass = ordered ? P<uint32_t>(ctx->tileClass) : nullptr;
     const FillRanges fills{{{P<uint32_t>(ctx->pathCanvas), pathCount + 1, 0xffffffffu},
                             {P<uint32_t>(ctx->tileCover), tileTotal, 0u},
                             {P<uint32_t>(ctx->drawPieces), drawCount + 1, 0u},
                             {P<uint32_t>(ctx->pathDraws), pathCount + 1, 0u},
                             {P<uint32_t>(ctx->pathBins), pathCount + 1, 0u},
-                            {P<uint32_t>(ctx->tileQueue), (uint32_t)queueWords, 0u}}};
+                            {P<uint32_t>(ctx->tileQueue), (uint32_t)queueWords, 0u},
+                            {tileClass, ordered ? tileTotal : 0u, 0u}}};
     const uint32_t longest = std::max({pathCount + 1, tileTotal, drawCount + 1, (uint32_t)queueWords});
     fill_ranges_kernel<<<std::min((longest + 255u) / 256u, 1024u), 256, 0, ctx->stream>>>(fills);
     path_canvas_kernel<<<canvasCount, 256, 0, ctx->stream>>>(canvases, P<uint32_t>(ctx->pathCanvas));
@@ -1532,7 +1547,7 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
             kernel<<<blocks, threads, lds, ctx->stream>>>(
                 prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), minCells, maxCells,
                 P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases, P<uint32_t>(ctx->tileCover),
-                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned));
+                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBase), P<uint32_t>(ctx->binned), tileClass);
         };
     };
     if (bin)
@@ -1549,10 +1564,9 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
                                                                    P<PathCells>(ctx->cells),
                                                                    P<uint32_t>(ctx->pathDraws),
                                                                    P<uint2>(ctx->cellPacked));
-        shared_layout_kernel<<<pathCount + 1, 256, 0, ctx->stream>>>(P<PathCells>(ctx->cells), pathCount + 1,
-                                                                     P<uint32_t>(ctx->pathDraws),
-                                                                     P<uint2>(ctx->cellPacked),
-                                                                     P<uint32_t>(ctx->pathBins));
+        shared_layout_kernel<<<pathCount + 1, 256, 0, ctx->stream>>>(
+            P<PathCells>(ctx->cells), pathCount + 1, P<uint32_t>(ctx->pathDraws), P<uint32_t>(ctx->pathCanvas), canvases,
+            P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), tileClass);
     }
     rc = device_scan(ctx, P<uint32_t>(ctx->pathBins), pathCount + 1, P<uint32_t>(ctx->pathBase), scal + 2);
     if (rc)
@@ -1592,22 +1606,11 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
         const bool persistent = rc.persistent != 0;
         uint32_t* queue = P<uint32_t>(ctx->tileQueue);
         const uint32_t* order = nullptr;
-        // Until a config is set: heaviest tiles first wherever the launch has
-        // more tiles than run at once, so that long tiles do not trail (the
-        // order costs two kernels, ~15 us).  Measured on MI355X, raster pass
-        // with the order's kernels: 1080p frame 9.0 -> 7.35 ms, 48 canvases
-        // 6.6 -> 4.4 ms, 24 served requests 7.0 -> 5.4 ms, 1024^2 200-path
-        // frame .27 ms either way.
-        const uint32_t resident = (uint32_t)std::max(ctx->cuCount, 1) * (rc.waves_per_simd == 5 ? 5u : 6u);
-        if (ctx->rasterConfigSet ? rc.tile_order != 0 : tileTotal > resident)
+        if (ordered)
         {
-            RIVE_TRY(ensure(ctx, ctx->tileClass, (size_t)tileTotal * 4));
-            RIVE_TRY(ensure(ctx, ctx->tileOrder, (size_t)tileTotal * 4));
-            tile_cost_kernel<<<(tileTotal + 3) / 4, 256, 0, ctx->stream>>>(
-                P<PathCells>(ctx->cells), P<uint2>(ctx->cellPacked), canvases, canvasCount,
-                tileTotal, P<uint32_t>(ctx->tileCover), P<uint32_t>(ctx->tileClass), queue);
+            tile_class_kernel<<<(tileTotal + 255) / 256, 256, 0, ctx->stream>>>(tileClass, tileTotal, queue);
             tile_order_kernel<<<(tileTotal + 255) / 256, 256, 0, ctx->stream>>>(
-                P<uint32_t>(ctx->tileClass), queue, queue + kCostClasses, tileTotal, P<uint32_t>(ctx->tileOrder));
+                tileClass, queue, queue + kCostClasses, tileTotal, P<uint32_t>(ctx->tileOrder));
             order = P<uint32_t>(ctx->tileOrder);
         }
         const int waves = rc.waves_per_simd == 5 ? 5 : 6;
