@@ -2145,7 +2145,7 @@ int flush_impl(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t
 // the launches it saves: an opaque fill hides what earlier flushes of the group
 // drew under it too.  The group's buffers are bounded by kGroupBytes: 16 B a
 // texel, 92 B a primitive (at most one a texel) and 8 B a (path, tile) cell
-// -- an eighth of the card's memory; a 4K frame of 20 000 draws counts 26 GB,
+// -- an eighth of the card's memory; a 4K frame of 20 000 draws counts 22 GB,
 // and a longer one runs in several groups.  Measured on MI355X: the 1080p
 // 5000-path frame (6 flushes) 19.4 -> 11.6 ms, the 4K 20 000-draw frame (35
 // flushes) 792 -> 211 ms end to end (raster 637 -> 84 ms, binning 47 -> 25).
