@@ -33,13 +33,22 @@ int fail(int code, const std::string& msg)
     return code;
 }
 
+// Reports a failed HIP call.  The runtime keeps its error as the thread's last
+// one until it is read, whatever succeeds after it, so it is read here: the
+// check after a later launch must not take it for that launch's.
+int hip_fail(int code, const std::string& msg)
+{
+    (void)hipGetLastError();
+    return fail(code, msg);
+}
+
 #define HIP_TRY(expr)                                                                        \
     do                                                                                       \
     {                                                                                        \
         hipError_t _e = (expr);                                                              \
         if (_e != hipSuccess)                                                                \
-            return fail(RIVE_HIP_ERROR_DEVICE,                                               \
-                        std::string(#expr) + ": " + hipGetErrorString(_e));                  \
+            return hip_fail(RIVE_HIP_ERROR_DEVICE,                                           \
+                            std::string(#expr) + ": " + hipGetErrorString(_e));              \
     } while (0)
 
 struct DevBuf
@@ -251,7 +260,7 @@ int ensure(rive_hip_context* ctx, DevBuf& b, size_t bytes)
     {
         hipError_t e = hipFree(b.ptr);
         if (e != hipSuccess)
-            return fail(RIVE_HIP_ERROR_DEVICE, std::string("hipFree: ") + hipGetErrorString(e));
+            return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("hipFree: ") + hipGetErrorString(e));
         b.ptr = nullptr;
         b.cap = 0;
     }
@@ -260,8 +269,8 @@ int ensure(rive_hip_context* ctx, DevBuf& b, size_t bytes)
     if (e != hipSuccess)
     {
         b.ptr = nullptr;
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY,
-                    "scratch allocation of " + std::to_string(cap) + " bytes failed: " + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY,
+                        "scratch allocation of " + std::to_string(cap) + " bytes failed: " + hipGetErrorString(e));
     }
     b.cap = cap;
     return RIVE_HIP_OK;
@@ -411,7 +420,7 @@ int rive_hip_create(int device, rive_hip_context** out)
         return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT, "out is null");
     int n = 0;
     if (hipGetDeviceCount(&n) != hipSuccess || n <= 0)
-        return fail(RIVE_HIP_ERROR_DEVICE, "no HIP device available");
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, "no HIP device available");
     if (device < 0 || device >= n)
         return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT, "device ordinal out of range");
     HIP_TRY(hipSetDevice(device));
@@ -462,7 +471,7 @@ int rive_hip_create(int device, rive_hip_context** out)
     if (e != hipSuccess)
     {
         delete ctx;
-        return fail(RIVE_HIP_ERROR_DEVICE, std::string("context setup: ") + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("context setup: ") + hipGetErrorString(e));
     }
     *out = ctx;
     return RIVE_HIP_OK;
@@ -563,7 +572,7 @@ void* rive_hip_buffer_map(rive_hip_context* ctx, int kind, size_t bytes)
     const int next = (b.slot + 1) % kRingSlots;
     if (hipEventSynchronize(b.copied[next]) != hipSuccess)
     {
-        fail(RIVE_HIP_ERROR_DEVICE, "staging slot wait failed");
+        hip_fail(RIVE_HIP_ERROR_DEVICE, "staging slot wait failed");
         return nullptr;
     }
     b.slot = next;
@@ -600,7 +609,7 @@ int rive_hip_target_create(rive_hip_context* ctx, uint32_t width, uint32_t heigh
     if (e != hipSuccess)
     {
         delete t;
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "target allocation failed");
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "target allocation failed");
     }
     HIP_TRY(hipMemsetAsync(t->pixels, 0, (size_t)width * height * 4, ctx->stream));
     *out = t;
@@ -651,7 +660,7 @@ int image_alloc(rive_hip_context* ctx, uint32_t width, uint32_t height, uint32_t
     HIP_TRY(hipSetDevice(ctx->device));
     uint32_t* texels = nullptr;
     if (hipMalloc(&texels, (size_t)total * 4) != hipSuccess)
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "image allocation failed");
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "image allocation failed");
     desc.texels = texels;
     *out = new rive_hip_image{ctx, desc};
     return RIVE_HIP_OK;
@@ -707,7 +716,7 @@ int decode_png_level0(rive_hip_context* ctx, const std::vector<uint8_t>& rgba, r
     const size_t n = (size_t)img->desc.width * img->desc.height;
     uint32_t* staged = t.alloc<uint32_t>(n * 4);
     if (staged == nullptr)
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "image decode staging allocation failed");
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "image decode staging allocation failed");
     HIP_TRY(hipMemcpyAsync(staged, rgba.data(), n * 4, hipMemcpyHostToDevice, ctx->stream));
     premultiply_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, ctx->stream>>>(
         staged, const_cast<uint32_t*>(img->desc.texels), n);
@@ -736,7 +745,7 @@ int decode_jpeg_level0(rive_hip_context* ctx, const rivehip::image::Jpeg& j, riv
     int16_t* coef = t.alloc<int16_t>(j.coef.size() * 2);
     uint16_t* qt = t.alloc<uint16_t>(sizeof(j.qt));
     if (coef == nullptr || qt == nullptr)
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "JPEG coefficient allocation failed");
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "JPEG coefficient allocation failed");
     HIP_TRY(hipMemcpyAsync(coef, j.coef.data(), j.coef.size() * 2, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMemcpyAsync(qt, j.qt, sizeof(j.qt), hipMemcpyHostToDevice, ctx->stream));
     JpegColor color{};
@@ -758,7 +767,7 @@ int decode_jpeg_level0(rive_hip_context* ctx, const rivehip::image::Jpeg& j, riv
         p.stride = c.blocksW * 8u * c.scaleH;
         p.samples = t.alloc<uint8_t>((size_t)p.stride * c.blocksH * 8u * c.scaleV);
         if (p.samples == nullptr)
-            return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "JPEG sample plane allocation failed");
+            return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, "JPEG sample plane allocation failed");
         const uint32_t blocks = c.blocksW * c.blocksH;
         jpeg_idct_kernel<<<(blocks + 63) / 64, 64, 0, ctx->stream>>>(p);
         HIP_TRY(hipGetLastError());
@@ -798,7 +807,7 @@ int rive_hip_image_create(rive_hip_context* ctx, uint32_t width, uint32_t height
     if (e != hipSuccess)
     {
         image_free(img);
-        return fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e));
     }
     *out = img;
     return RIVE_HIP_OK;
@@ -892,7 +901,7 @@ int rive_hip_image_decode(rive_hip_context* ctx, const uint8_t* bytes, size_t n,
         // the temporaries are freed only once the stream is done with them
         const hipError_t es = hipStreamSynchronize(ctx->stream);
         if (rc == RIVE_HIP_OK && (e != hipSuccess || es != hipSuccess))
-            rc = fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e != hipSuccess ? e : es));
+            rc = hip_fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e != hipSuccess ? e : es));
     }
     if (rc != RIVE_HIP_OK)
     {
@@ -1051,7 +1060,7 @@ int settle(rive_hip_context* ctx)
     if (e != hipSuccess)
     {
         ctx->pendingReads.clear();
-        return fail(RIVE_HIP_ERROR_DEVICE, std::string("stream sync: ") + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("stream sync: ") + hipGetErrorString(e));
     }
     if (ctx->reads == rive_hip_context::Reads::record)
         for (const auto& r : ctx->pendingReads)
@@ -2272,7 +2281,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
     {
         restore();
         rive_hip_frame_graph_destroy(g.release());
-        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, std::string("frame graph records: ") + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, std::string("frame graph records: ") + hipGetErrorString(e));
     }
     // 1. an eager frame that sizes every buffer and records the totals it reads
     ctx->pendingReads.clear();
@@ -2290,7 +2299,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
     }
     ctx->reads = rive_hip_context::Reads::live;
     if (rc == RIVE_HIP_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
-        rc = fail(RIVE_HIP_ERROR_DEVICE, "frame graph: recording flush failed");
+        rc = hip_fail(RIVE_HIP_ERROR_DEVICE, "frame graph: recording flush failed");
     if (rc != RIVE_HIP_OK)
     {
         ctx->groupFlushes = true;
@@ -2320,7 +2329,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
     if (e != hipSuccess)
     {
         rive_hip_frame_graph_destroy(g.release());
-        return fail(RIVE_HIP_ERROR_DEVICE, std::string("frame capture: ") + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("frame capture: ") + hipGetErrorString(e));
     }
     if (rc != RIVE_HIP_OK || !consumed)
     {
@@ -2331,7 +2340,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
     if (e != hipSuccess)
     {
         rive_hip_frame_graph_destroy(g.release());
-        return fail(RIVE_HIP_ERROR_DEVICE, std::string("graph instantiate: ") + hipGetErrorString(e));
+        return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("graph instantiate: ") + hipGetErrorString(e));
     }
     *out = g.release();
     return RIVE_HIP_OK;
@@ -2609,7 +2618,7 @@ extern "C" int rive_hip_autotune_frame(rive_hip_context* ctx, const rive_hip_flu
     const rive_hip_raster_config before = ctx->rasterConfig;
     const bool beforeSet = ctx->rasterConfigSet;
     ctx->rasterConfigSet = true; // each candidate runs as it says
-    int rc = e == hipSuccess ? RIVE_HIP_OK : fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e));
+    int rc = e == hipSuccess ? RIVE_HIP_OK : hip_fail(RIVE_HIP_ERROR_DEVICE, hipGetErrorString(e));
     float best = INFINITY;
     int bestK = 0;
     std::vector<float> t(trials);
@@ -2650,7 +2659,7 @@ extern "C" int rive_hip_autotune_frame(rive_hip_context* ctx, const rive_hip_flu
         e = hipStreamSynchronize(ctx->stream);
     (void)hipFree(saved);
     if (rc == RIVE_HIP_OK && e != hipSuccess)
-        rc = fail(RIVE_HIP_ERROR_DEVICE, std::string("autotune: ") + hipGetErrorString(e));
+        rc = hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("autotune: ") + hipGetErrorString(e));
     if (rc != RIVE_HIP_OK)
     {
         ctx->rasterConfig = before;
