@@ -2263,7 +2263,12 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
         }
         for (int k = 0; k < RIVE_HIP_BUFFER_KIND_COUNT; ++k)
             ctx->bufs[k].dev = savedDev[k];
+        // the last flush's intermediates went with the graph's buffers: there is
+        // nothing for a readback to read
         ctx->lastSpans = ctx->lastContours = nullptr;
+        ctx->lastSpanCount = ctx->lastContourCount = ctx->lastRecordCount = ctx->lastDrawCount = 0;
+        ctx->lastTexels = ctx->lastGradRows = 0;
+        ctx->lastTexBase = ctx->lastRampBase = 0;
         ctx->in = rive_hip_context::FlushInputs{};
     };
     hipError_t e = hipSuccess;
