@@ -403,10 +403,12 @@ int rive_hip_last_frame(rive_hip_context* ctx, rive_hip_flush_desc* out, uint32_
  * each flush still laid out on its own from location 8 and contour ID 1.
  * Where their other records follow each other too (as the reference and the
  * front end write them) and the later flushes load the target, all passes run
- * once for the whole frame, in device buffers of up to 32 GiB beside the
- * bins; a larger frame, or one that does not get the memory, runs them for
- * parts of it or flush by flush.  Replaces the per-logical-flush RenderContextImpl::flush calls of
- * one RenderContext::flush (render_context.cpp:971-1018).
+ * once for the whole frame, in device buffers of up to an eighth of the card's
+ * memory (or the context's scratch limit) beside the bins; a larger frame, or
+ * one that does not get the memory, runs them for parts of it or flush by
+ * flush.  (What one flush needs is not bounded by that eighth.)  Replaces the
+ * per-logical-flush RenderContextImpl::flush calls of one
+ * RenderContext::flush (render_context.cpp:971-1018).
  * rive_hip_pass_times then sums over the frame's flushes. */
 int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n);
 
@@ -476,6 +478,15 @@ typedef struct rive_hip_raster_config
 
 int rive_hip_set_raster_config(rive_hip_context* ctx, const rive_hip_raster_config* config);
 int rive_hip_get_raster_config(rive_hip_context* ctx, rive_hip_raster_config* out);
+
+/* Bounds the device scratch a context holds between and during flushes, in
+ * bytes (0, the default: no bound).  Scratch beyond the bound is freed, frames
+ * run in launch groups that fit, and a flush that needs more is refused with
+ * RIVE_HIP_ERROR_OUT_OF_MEMORY.  A frame graph's own buffers count against the
+ * bound while it is created.  The getter returns the bytes held now.  No
+ * counterpart in the reference (its resources are sized per flush). */
+int rive_hip_set_scratch_limit(rive_hip_context* ctx, uint64_t bytes);
+uint64_t rive_hip_get_scratch_bytes(rive_hip_context* ctx);
 
 /* Interior triangulation for frames the context's front end lays out
  * (RenderContext::FrameDescriptor::triangulationThresholds,

@@ -155,6 +155,10 @@ struct rive_hip_context
     // and whether one did run out.
     bool groupFlushes = true;
     bool groupFellBack = false;
+    // What a launch group's buffers may take (group_bytes), and the caller's
+    // bound on all device scratch (0: none).
+    uint64_t groupBudget = 0;
+    uint64_t scratchLimit = 0;
     uint32_t lastGradRows = 0;
     rive_hip_flush_stats stats = {};
     std::vector<rive_hip_canvas> flushCanvases; // the current flush's canvas table (capacity kept)
@@ -230,6 +234,40 @@ void devbufs(rive_hip_context* c, DevBuf** out)
         out[i] = all[i];
 }
 
+// The device scratch a context holds.
+uint64_t scratch_bytes(rive_hip_context* ctx)
+{
+    DevBuf* all[kDevBufCount];
+    devbufs(ctx, all);
+    uint64_t sum = 0;
+    for (const DevBuf* b : all)
+        sum += b->carved ? 0 : b->cap;
+    return sum;
+}
+
+// Frees a scratch buffer that no enqueued work uses.
+int release(DevBuf& b)
+{
+    if (b.ptr != nullptr && !b.carved)
+    {
+        const hipError_t e = hipFree(b.ptr);
+        if (e != hipSuccess)
+            return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("hipFree: ") + hipGetErrorString(e));
+    }
+    b = DevBuf{};
+    return RIVE_HIP_OK;
+}
+
+// The last flush's intermediates are gone: there is nothing to read back.
+void forget_intermediates(rive_hip_context* ctx)
+{
+    ctx->lastSpans = ctx->lastContours = nullptr;
+    ctx->lastSpanCount = ctx->lastContourCount = ctx->lastRecordCount = ctx->lastDrawCount = 0;
+    ctx->lastTexels = ctx->lastGradRows = 0;
+    ctx->lastTexBase = ctx->lastRampBase = 0;
+    ctx->in = rive_hip_context::FlushInputs{};
+}
+
 // Grows a scratch buffer to at least `bytes` (grow-only, 1.25x headroom).
 // Inside a no-alloc flush it carves the buffer from the device's scratch
 // array instead and never calls the allocator.
@@ -256,15 +294,17 @@ int ensure(rive_hip_context* ctx, DevBuf& b, size_t bytes)
         return RIVE_HIP_OK;
     if (ctx->capturing)
         return fail(RIVE_HIP_ERROR_DEVICE, "a captured frame needs a buffer its recording did not size");
+    const size_t cap = std::max<size_t>(bytes + bytes / 4, 256);
+    if (ctx->scratchLimit != 0 && scratch_bytes(ctx) - b.cap + cap > ctx->scratchLimit)
+        return fail(RIVE_HIP_ERROR_OUT_OF_MEMORY,
+                    "scratch allocation of " + std::to_string(cap) + " bytes beyond the scratch limit of " +
+                        std::to_string(ctx->scratchLimit));
     if (b.ptr != nullptr)
     {
-        hipError_t e = hipFree(b.ptr);
-        if (e != hipSuccess)
-            return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("hipFree: ") + hipGetErrorString(e));
-        b.ptr = nullptr;
-        b.cap = 0;
+        const int rc = release(b);
+        if (rc != RIVE_HIP_OK)
+            return rc;
     }
-    size_t cap = std::max<size_t>(bytes + bytes / 4, 256);
     hipError_t e = hipMalloc(&b.ptr, cap);
     if (e != hipSuccess)
     {
@@ -454,6 +494,12 @@ int rive_hip_create(int device, rive_hip_context** out)
         std::vector<float> tables(2 * kFeatherTableSize);
         feather_tables_host(tables.data());
         e = hipMemcpy(ctx->featherTables, tables.data(), sizeof(float) * tables.size(), hipMemcpyHostToDevice);
+    }
+    if (e == hipSuccess)
+    {
+        size_t freeBytes = 0, totalBytes = 0;
+        e = hipMemGetInfo(&freeBytes, &totalBytes);
+        ctx->groupBudget = totalBytes / 8;
     }
     // the binning of large grids takes more LDS than a launch may by default
     if (e == hipSuccess)
@@ -1391,9 +1437,9 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
                 spans, spanCount, P<uint32_t>(ctx->spanTexelOffsets), used, P<TessTexel>(ctx->tess),
                 reinterpret_cast<const uint4*>(contours), reinterpret_cast<const float*>(paths), g.flushes, g.n,
                 ctx->featherTables);
-        ctx->lastTexels = last.texels;
-        ctx->lastTexBase = last.texBase;
     }
+    ctx->lastTexels = last.texels;
+    ctx->lastTexBase = last.texBase;
     HIP_TRY(hipGetLastError());
     if (d->mode == RIVE_HIP_FLUSH_SPANS && d->patch_batch_count > 0)
     {
@@ -2148,22 +2194,36 @@ int flush_impl(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t
     return RIVE_HIP_OK;
 }
 
+// What a launch group of so many texels and (path, tile) cells reserves, with
+// the headroom ensure() adds: 16 B a texel, 92 B a primitive (at most one a
+// texel), 8 B a cell and 4 B for the cursor of a cell that several draws bin
+// into.  The bins come on top.
+uint64_t group_bytes(uint64_t texels, uint64_t cells)
+{
+    const uint64_t bytes = texels * 108u + cells * 12u;
+    return bytes + bytes / 4;
+}
+
 // One past the last flush that may run in the same launch group as flush k:
 // consecutive GEOMETRY flushes of one target whose records follow each other
 // in the mapped buffers, the later ones loading it.  Grouping matters beyond
 // the launches it saves: an opaque fill hides what earlier flushes of the group
-// drew under it too.  The group's buffers are bounded by kGroupBytes: 16 B a
-// texel, 92 B a primitive (at most one a texel) and 8 B a (path, tile) cell
-// -- an eighth of the card's memory; a 4K frame of 20 000 draws counts 22 GB,
-// and a longer one runs in several groups.  Measured on MI355X: the 1080p
-// 5000-path frame (6 flushes) 19.4 -> 11.6 ms, the 4K 20 000-draw frame (35
-// flushes) 792 -> 211 ms end to end (raster 637 -> 84 ms, binning 47 -> 25).
-constexpr uint64_t kGroupBytes = (uint64_t)32 << 30;
+// drew under it too.  What joins a group beyond its first flush is bounded by
+// groupBudget -- an eighth of the card's memory, 36 GiB of 288 -- and half of a
+// caller's scratch limit, which leaves the other half for bins and records.  A
+// 4K frame of 20 000 draws counts 30 GB; a longer one runs in several groups.
+// (The memory free at the moment does not count: a captured frame must form the
+// groups its recording did.)  Measured on MI355X when flushes were first
+// joined: the 1080p 5000-path frame (6 flushes) 19.4 -> 11.6 ms, the 4K
+// 20 000-draw frame (35 flushes) 792 -> 211 ms end to end (raster 637 -> 84 ms,
+// binning 47 -> 25).
 uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n,
                    const GeoLayout* layouts, uint32_t k)
 {
     if (!ctx->groupFlushes || descs[k].target == nullptr)
         return k + 1;
+    const uint64_t budget =
+        ctx->scratchLimit != 0 ? std::min(ctx->groupBudget, ctx->scratchLimit / 2) : ctx->groupBudget;
     const uint64_t tiles = (uint64_t)((descs[k].target->width + kTile - 1) / kTile) *
                            ((descs[k].target->height + kTile - 1) / kTile);
     uint64_t texels = 0, paths = 0, images = 0;
@@ -2183,7 +2243,7 @@ uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs
         texels += (uint64_t)layouts[e].tessRows * kTessTextureWidth;
         paths += (uint64_t)d.path_count + 1u;
         images += d.image_count;
-        if (e > k && (texels * 108u + paths * tiles * 8u > kGroupBytes || texels > kMaxFlushTexels ||
+        if (e > k && (group_bytes(texels, paths * tiles) > budget || texels > kMaxFlushTexels ||
                       paths > kMaxFlushPaths || images > 0xffffu || paths * (tiles + 1u) >= 0xffffffffu))
             break;
     }
@@ -2263,13 +2323,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
         }
         for (int k = 0; k < RIVE_HIP_BUFFER_KIND_COUNT; ++k)
             ctx->bufs[k].dev = savedDev[k];
-        // the last flush's intermediates went with the graph's buffers: there is
-        // nothing for a readback to read
-        ctx->lastSpans = ctx->lastContours = nullptr;
-        ctx->lastSpanCount = ctx->lastContourCount = ctx->lastRecordCount = ctx->lastDrawCount = 0;
-        ctx->lastTexels = ctx->lastGradRows = 0;
-        ctx->lastTexBase = ctx->lastRampBase = 0;
-        ctx->in = rive_hip_context::FlushInputs{};
+        forget_intermediates(ctx); // they went with the graph's buffers
     };
     hipError_t e = hipSuccess;
     for (int k = 0; k < RIVE_HIP_BUFFER_KIND_COUNT && e == hipSuccess; ++k)
@@ -2769,6 +2823,30 @@ extern "C" int rive_hip_set_raster_config(rive_hip_context* ctx, const rive_hip_
     ctx->rasterConfig = *config;
     ctx->rasterConfigSet = true;
     return RIVE_HIP_OK;
+}
+
+extern "C" int rive_hip_set_scratch_limit(rive_hip_context* ctx, uint64_t bytes)
+{
+    if (ctx == nullptr)
+        return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT, "null context");
+    if (bytes != 0 && scratch_bytes(ctx) > bytes)
+    {
+        // what is held goes; the next flush takes what it needs within the limit
+        HIP_TRY(hipSetDevice(ctx->device));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        DevBuf* all[kDevBufCount];
+        devbufs(ctx, all);
+        for (DevBuf* b : all)
+            RIVE_TRY(release(*b));
+        forget_intermediates(ctx);
+    }
+    ctx->scratchLimit = bytes;
+    return RIVE_HIP_OK;
+}
+
+extern "C" uint64_t rive_hip_get_scratch_bytes(rive_hip_context* ctx)
+{
+    return ctx != nullptr ? scratch_bytes(ctx) : 0;
 }
 
 extern "C" int rive_hip_set_interior_triangulation(rive_hip_context* ctx, uint32_t enabled)

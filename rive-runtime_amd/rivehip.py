@@ -148,6 +148,7 @@ class RasterConfig(ctypes.Structure):
 
 EXPORTED = [
     "rive_hip_set_interior_triangulation", "rive_hip_get_interior_triangulation",
+    "rive_hip_set_scratch_limit", "rive_hip_get_scratch_bytes",
     "rive_hip_last_error", "rive_hip_create", "rive_hip_destroy", "rive_hip_buffer_resize",
     "rive_hip_buffer_map", "rive_hip_buffer_unmap", "rive_hip_target_create",
     "rive_hip_target_destroy", "rive_hip_flush", "rive_hip_sync", "rive_hip_read_pixels",
@@ -218,6 +219,9 @@ def lib():
     L.rive_hip_image_read.argtypes = [vp, u32, vp, ctypes.c_size_t, ctypes.POINTER(u32), ctypes.POINTER(u32)]
     L.rive_hip_set_raster_config.argtypes = [vp, ctypes.POINTER(RasterConfig)]
     L.rive_hip_get_raster_config.argtypes = [vp, ctypes.POINTER(RasterConfig)]
+    L.rive_hip_set_scratch_limit.argtypes = [vp, ctypes.c_uint64]
+    L.rive_hip_get_scratch_bytes.argtypes = [vp]
+    L.rive_hip_get_scratch_bytes.restype = ctypes.c_uint64
     L.rive_hip_set_interior_triangulation.argtypes = [vp, ctypes.c_uint32]
     L.rive_hip_get_interior_triangulation.argtypes = [vp]
     L.rive_hip_get_interior_triangulation.restype = ctypes.c_uint32
@@ -573,6 +577,14 @@ class Context:
         """Whether the front end lays large plain fills out as outer-cubic
         patches (interior triangulation); off by default."""
         check(self.L.rive_hip_set_interior_triangulation(self.h, 1 if enabled else 0))
+
+    def set_scratch_limit(self, nbytes):
+        """Bounds the device scratch the context holds (0: no bound)."""
+        check(self.L.rive_hip_set_scratch_limit(self.h, int(nbytes)))
+
+    def scratch_bytes(self):
+        """Bytes of device scratch the context holds now."""
+        return int(self.L.rive_hip_get_scratch_bytes(self.h))
 
     def interior_triangulation(self):
         return bool(self.L.rive_hip_get_interior_triangulation(self.h))
