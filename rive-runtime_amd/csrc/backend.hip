@@ -150,14 +150,15 @@ struct rive_hip_context
     const void* lastSpans = nullptr;    // the last flush's TessVertexSpans (device)
     const void* lastContours = nullptr; // and ContourData
     size_t lastTexBase = 0, lastRampBase = 0; // its first texel and ramp row
-    // Whether a frame's flushes may run in launch groups (false after a group
-    // ran out of memory, until the frame or the graph recording it is done),
-    // and whether one did run out.
-    bool groupFlushes = true;
+    // How many flushes a launch group may join (fewer after a group was
+    // refused, until the frame or the graph recording it is done), and whether
+    // one was refused.
+    uint32_t groupMost = 0xffffffffu;
     bool groupFellBack = false;
-    // What a launch group's buffers may take (group_bytes), and the caller's
-    // bound on all device scratch (0: none).
-    uint64_t groupBudget = 0;
+    // What a launch group's buffers may take (group_bytes), at most and after
+    // groups that did not get their memory, and the caller's bound on all
+    // device scratch (0: none).
+    uint64_t groupBudgetMost = 0, groupBudget = 0;
     uint64_t scratchLimit = 0;
     uint32_t lastGradRows = 0;
     rive_hip_flush_stats stats = {};
@@ -255,6 +256,25 @@ int release(DevBuf& b)
             return hip_fail(RIVE_HIP_ERROR_DEVICE, std::string("hipFree: ") + hipGetErrorString(e));
     }
     b = DevBuf{};
+    return RIVE_HIP_OK;
+}
+
+// Frees what a refused launch group grew: every scratch buffer but the frame's
+// layout (the counting pass's contours and spans, which its flushes still read).
+int release_flush_buffers(rive_hip_context* ctx)
+{
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    DevBuf* all[kDevBufCount];
+    devbufs(ctx, all);
+    for (DevBuf* b : all)
+    {
+        if (b == &ctx->geoCounts || b == &ctx->geoRecords || b == &ctx->geoContours || b == &ctx->geoSpans ||
+            b == &ctx->geoSpanCounts || b == &ctx->geoSpanOffsets)
+            continue;
+        const int rc = release(*b);
+        if (rc != RIVE_HIP_OK)
+            return rc;
+    }
     return RIVE_HIP_OK;
 }
 
@@ -499,7 +519,7 @@ int rive_hip_create(int device, rive_hip_context** out)
     {
         size_t freeBytes = 0, totalBytes = 0;
         e = hipMemGetInfo(&freeBytes, &totalBytes);
-        ctx->groupBudget = totalBytes / 8;
+        ctx->groupBudgetMost = ctx->groupBudget = totalBytes / 8;
     }
     // the binning of large grids takes more LDS than a launch may by default
     if (e == hipSuccess)
@@ -2217,10 +2237,12 @@ uint64_t group_bytes(uint64_t texels, uint64_t cells)
 // joined: the 1080p 5000-path frame (6 flushes) 19.4 -> 11.6 ms, the 4K
 // 20 000-draw frame (35 flushes) 792 -> 211 ms end to end (raster 637 -> 84 ms,
 // binning 47 -> 25).
+// *bytes gets what the group counts.
 uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n,
-                   const GeoLayout* layouts, uint32_t k)
+                   const GeoLayout* layouts, uint32_t k, uint64_t* bytes)
 {
-    if (!ctx->groupFlushes || descs[k].target == nullptr)
+    *bytes = 0;
+    if (descs[k].target == nullptr)
         return k + 1;
     const uint64_t budget =
         ctx->scratchLimit != 0 ? std::min(ctx->groupBudget, ctx->scratchLimit / 2) : ctx->groupBudget;
@@ -2228,7 +2250,7 @@ uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs
                            ((descs[k].target->height + kTile - 1) / kTile);
     uint64_t texels = 0, paths = 0, images = 0;
     uint32_t e = k;
-    for (; e < n; ++e)
+    for (; e < n && e - k < ctx->groupMost; ++e)
     {
         const rive_hip_flush_desc& d = descs[e];
         if (e > k)
@@ -2243,11 +2265,74 @@ uint32_t group_end(const rive_hip_context* ctx, const rive_hip_flush_desc* descs
         texels += (uint64_t)layouts[e].tessRows * kTessTextureWidth;
         paths += (uint64_t)d.path_count + 1u;
         images += d.image_count;
-        if (e > k && (group_bytes(texels, paths * tiles) > budget || texels > kMaxFlushTexels ||
-                      paths > kMaxFlushPaths || images > 0xffffu || paths * (tiles + 1u) >= 0xffffffffu))
+        const uint64_t count = group_bytes(texels, paths * tiles);
+        if (e > k && (count > budget || texels > kMaxFlushTexels || paths > kMaxFlushPaths || images > 0xffffu ||
+                      paths * (tiles + 1u) >= 0xffffffffu))
             break;
+        *bytes = count;
     }
     return std::max(e, k + 1);
+}
+} // namespace
+
+namespace
+{
+// Copies of targets' pixels, to put them back as they were.
+struct SavedTargets
+{
+    std::vector<rive_hip_target*> targets;
+    unsigned char* copy = nullptr;
+
+    ~SavedTargets()
+    {
+        if (copy != nullptr)
+            (void)hipFree(copy);
+    }
+    int save(rive_hip_context* ctx, std::vector<rive_hip_target*> list)
+    {
+        std::sort(list.begin(), list.end());
+        list.erase(std::unique(list.begin(), list.end()), list.end());
+        size_t bytes = 0;
+        for (const rive_hip_target* t : list)
+            bytes += (size_t)t->width * t->height * 4;
+        if (bytes == 0)
+            return RIVE_HIP_OK;
+        HIP_TRY(hipMalloc((void**)&copy, bytes));
+        targets = std::move(list);
+        return transfer(ctx, false);
+    }
+    int restore(rive_hip_context* ctx) { return transfer(ctx, true); }
+
+private:
+    int transfer(rive_hip_context* ctx, bool back)
+    {
+        unsigned char* at = copy;
+        for (const rive_hip_target* t : targets)
+        {
+            const size_t b = (size_t)t->width * t->height * 4;
+            HIP_TRY(hipMemcpyAsync(back ? (void*)t->pixels : (void*)at, back ? (void*)at : (void*)t->pixels, b,
+                                   hipMemcpyDeviceToDevice, ctx->stream));
+            at += b;
+        }
+        return RIVE_HIP_OK;
+    }
+};
+
+// The targets whose pixels from before the frame it loads (flushes of canvas
+// lists form no launch groups and are left out).
+std::vector<rive_hip_target*> loaded_targets(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n)
+{
+    std::vector<rive_hip_target*> seen, loaded;
+    for (uint32_t k = 0; k < n; ++k)
+    {
+        rive_hip_target* t = descs[k].canvas_count == 0 ? descs[k].target : nullptr;
+        if (t == nullptr || t->ctx != ctx || std::find(seen.begin(), seen.end(), t) != seen.end())
+            continue;
+        seen.push_back(t);
+        if (descs[k].load_action == 1u)
+            loaded.push_back(t);
+    }
+    return loaded;
 }
 } // namespace
 
@@ -2342,26 +2427,30 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
         rive_hip_frame_graph_destroy(g.release());
         return hip_fail(RIVE_HIP_ERROR_OUT_OF_MEMORY, std::string("frame graph records: ") + hipGetErrorString(e));
     }
-    // 1. an eager frame that sizes every buffer and records the totals it reads
-    ctx->pendingReads.clear();
-    ctx->tape.clear();
+    // 1. an eager frame that sizes every buffer and records the totals it reads.
+    //    If a launch group was refused, the frame is recorded again from the
+    //    same pixels in the smaller groups, as the capture below then runs it.
+    SavedTargets before;
+    int rc = n > 1 ? before.save(ctx, loaded_targets(ctx, descs, n)) : RIVE_HIP_OK;
     ctx->reads = rive_hip_context::Reads::record;
     ctx->groupFellBack = false;
-    int rc = rive_hip_flush_frame(ctx, descs, n);
-    if (rc == RIVE_HIP_OK && ctx->groupFellBack)
+    for (bool again = rc == RIVE_HIP_OK; again;)
     {
-        // too large to run in groups: recorded again flush by flush, as the
-        // capture below then runs it
+        ctx->pendingReads.clear();
         ctx->tape.clear();
-        ctx->groupFlushes = false;
-        rc = rive_hip_flush_frame(ctx, descs, n);
+        if (ctx->groupFellBack)
+            rc = before.restore(ctx);
+        ctx->groupFellBack = false;
+        if (rc == RIVE_HIP_OK)
+            rc = rive_hip_flush_frame(ctx, descs, n);
+        again = rc == RIVE_HIP_OK && ctx->groupFellBack;
     }
     ctx->reads = rive_hip_context::Reads::live;
     if (rc == RIVE_HIP_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
         rc = hip_fail(RIVE_HIP_ERROR_DEVICE, "frame graph: recording flush failed");
     if (rc != RIVE_HIP_OK)
     {
-        ctx->groupFlushes = true;
+        ctx->groupMost = 0xffffffffu;
         restore();
         rive_hip_frame_graph_destroy(g.release());
         return rc;
@@ -2379,7 +2468,7 @@ extern "C" int rive_hip_frame_graph_create(rive_hip_context* ctx, const rive_hip
         e = hipStreamEndCapture(ctx->stream, &g->graph);
     }
     ctx->reads = rive_hip_context::Reads::live;
-    ctx->groupFlushes = true;
+    ctx->groupMost = 0xffffffffu;
     ctx->capturing = false;
     g->held.swap(ctx->captureHeld);
     const bool consumed = ctx->tapePos == ctx->tape.size();
@@ -2482,44 +2571,56 @@ extern "C" int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_
     std::vector<GeoLayout> layouts(n);
     RIVE_TRY(geometry_counting_frame(ctx, descs, n, layouts.data()));
     RIVE_TRY(mark(ctx, ctx->ev[1])); // the frame's counting done
-    const bool grouped = ctx->groupFlushes;
-    for (uint32_t k = 0, set = 0; k < n; ++set)
+    const uint32_t most = ctx->groupMost;
+    const uint64_t budget = ctx->groupBudget;
+    int rc = RIVE_HIP_OK;
+    for (uint32_t k = 0, set = 0; k < n && rc == RIVE_HIP_OK;)
     {
-        int rc = use_event_set(ctx, set);
+        rc = use_event_set(ctx, set);
         if (rc == RIVE_HIP_OK && set > 0)
             rc = mark(ctx, ctx->ev[6]);
         if (rc == RIVE_HIP_OK && set > 0)
             rc = mark(ctx, ctx->ev[1]);
         if (rc != RIVE_HIP_OK)
-        {
-            ctx->groupFlushes = grouped;
-            return rc;
-        }
+            break;
         ctx->evSetsUsed = set + 1;
-        uint32_t end = group_end(ctx, descs, n, layouts.data(), k);
+        uint64_t bytes = 0;
+        const uint32_t end = group_end(ctx, descs, n, layouts.data(), k, &bytes);
         const size_t taped = ctx->tape.size();
         rc = flush_impl(ctx, &descs[k], end - k, &layouts[k]);
-        if (rc == RIVE_HIP_ERROR_OUT_OF_MEMORY && end > k + 1)
+        if ((rc == RIVE_HIP_ERROR_OUT_OF_MEMORY || rc == RIVE_HIP_ERROR_UNSUPPORTED) && end > k + 1)
         {
-            // Not enough memory for the group: its flushes one by one (nothing
-            // was drawn yet, and a recording forgets the attempt's reads).
+            // Refused for its memory, or for totals that a group's flushes may
+            // each stay below (bins, guard-box pieces).  Nothing of it was
+            // drawn: halves of it, down to single flushes.  A recording forgets
+            // the attempt's reads.
             ctx->tape.resize(taped);
             ctx->pendingReads.clear();
-            ctx->groupFlushes = false;
+            ctx->groupMost = (end - k) / 2;
             ctx->groupFellBack = true;
-            end = k + 1;
-            rc = flush_impl(ctx, &descs[k], 1, &layouts[k]);
+            const bool memory = rc == RIVE_HIP_ERROR_OUT_OF_MEMORY;
+            rc = RIVE_HIP_OK;
+            if (memory)
+            {
+                // what the attempt grew goes, and the next frames ask for less
+                ctx->groupBudget = std::min(ctx->groupBudget, bytes / 2);
+                rc = release_flush_buffers(ctx);
+            }
+            continue;
         }
         if (rc != RIVE_HIP_OK)
-        {
-            ctx->groupFlushes = grouped;
-            return rc;
-        }
+            break;
         for (; k < end; ++k)
             record_frame_desc(ctx, &descs[k]);
+        ++set;
     }
-    ctx->groupFlushes = grouped;
-    return RIVE_HIP_OK;
+    if (ctx->reads != rive_hip_context::Reads::record)
+        ctx->groupMost = most;
+    // (a lowered budget comes back over some dozens of frames; not between a
+    // recording and its capture)
+    if (ctx->reads == rive_hip_context::Reads::live && ctx->groupBudget == budget)
+        ctx->groupBudget = std::min(ctx->groupBudgetMost, budget + budget / 16);
+    return rc;
 }
 
 namespace
@@ -2840,6 +2941,7 @@ extern "C" int rive_hip_set_scratch_limit(rive_hip_context* ctx, uint64_t bytes)
             RIVE_TRY(release(*b));
         forget_intermediates(ctx);
     }
+    ctx->groupBudget = ctx->groupBudgetMost;
     ctx->scratchLimit = bytes;
     return RIVE_HIP_OK;
 }
