@@ -2537,12 +2537,11 @@ extern "C" int rive_hip_flush(rive_hip_context* ctx, const rive_hip_flush_desc* 
     return rc;
 }
 
-extern "C" int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n)
+namespace
 {
-    if (ctx == nullptr || descs == nullptr || n == 0)
-        return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT, "null argument or empty frame");
-    HIP_TRY(hipSetDevice(ctx->device));
-    ctx->lastFlushNoAlloc = false;
+// Whether rive_hip_flush_frame runs one counting pass for the whole frame.
+bool counts_together(const rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n)
+{
     // One counting launch for the whole frame needs GEOMETRY flushes of one
     // target whose draw records follow each other; anything else runs flush
     // by flush.
@@ -2560,7 +2559,17 @@ extern "C" int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_
         for (int k = 0; k < RIVE_HIP_BUFFER_KIND_COUNT; ++k)
             fused = fused && !ctx->bufs[k].mapped;
     }
-    if (!fused)
+    return fused;
+}
+} // namespace
+
+extern "C" int rive_hip_flush_frame(rive_hip_context* ctx, const rive_hip_flush_desc* descs, uint32_t n)
+{
+    if (ctx == nullptr || descs == nullptr || n == 0)
+        return fail(RIVE_HIP_ERROR_INVALID_ARGUMENT, "null argument or empty frame");
+    HIP_TRY(hipSetDevice(ctx->device));
+    ctx->lastFlushNoAlloc = false;
+    if (!counts_together(ctx, descs, n))
     {
         for (uint32_t k = 0; k < n; ++k)
             RIVE_TRY(rive_hip_flush(ctx, &descs[k]));
@@ -2786,14 +2795,21 @@ extern "C" int rive_hip_autotune_frame(rive_hip_context* ctx, const rive_hip_flu
     {
         ctx->rasterConfig = kRasterCandidates[k];
         rc = rive_hip_flush_frame(ctx, descs, n); // untimed: first use, buffer growth
-        // a trial: the frame, its raster passes' time
+        // a trial: the frame, its raster passes' time; flush by flush where it
+        // runs so, since only the last flush's events are kept then
+        const bool together = counts_together(ctx, descs, n);
         for (uint32_t r = 0; r < trials && rc == RIVE_HIP_OK; ++r)
         {
             float ms[6];
-            rc = rive_hip_flush_frame(ctx, descs, n);
-            if (rc == RIVE_HIP_OK)
-                rc = rive_hip_pass_times(ctx, ms, 6);
-            t[r] = ms[4];
+            t[r] = 0.f;
+            for (uint32_t f = 0; f < (together ? 1u : n) && rc == RIVE_HIP_OK; ++f)
+            {
+                rc = together ? rive_hip_flush_frame(ctx, descs, n) : rive_hip_flush(ctx, &descs[f]);
+                if (rc == RIVE_HIP_OK)
+                    rc = rive_hip_pass_times(ctx, ms, 6);
+                if (rc == RIVE_HIP_OK)
+                    t[r] += ms[4];
+            }
         }
         if (rc != RIVE_HIP_OK)
             break;
