@@ -219,6 +219,7 @@ constexpr int kDevBufCount = 42;
 constexpr size_t kScalarBytes = 128;
 constexpr int kFarSlot = 16;
 constexpr int kSharedSlot = kFarSlot + 4; // set when a path is not binned solo
+constexpr int kClipSlot = kFarSlot + 5;   // set when a clip ID is written twice
 void devbufs(rive_hip_context* c, DevBuf** out)
 {
     DevBuf* all[kDevBufCount] = {&c->spanTexelCounts, &c->spanTexelOffsets, &c->scanPartials, &c->scalars,
@@ -1509,8 +1510,9 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(ensure(ctx, ctx->clipFirst, ((size_t)pathCount / 64 + 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->cells, (size_t)(pathCount + 1) * sizeof(PathCells)));
     path_raster_kernel<<<(pathCount + 1 + 255) / 256, 256, 0, ctx->stream>>>(
-        paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, g.flushes, g.n, P<PathRaster>(ctx->pathRaster),
-        P<PathPaint>(ctx->pathPaint), P<PathCells>(ctx->cells), P<uint32_t>(ctx->clipFirst));
+        paths, paints, aux, P<uint32_t>(ctx->pathImage), pathCount, g.flushes, g.n, P<uint32_t>(ctx->pathCanvas),
+        canvases, P<PathRaster>(ctx->pathRaster), P<PathPaint>(ctx->pathPaint), P<PathCells>(ctx->cells),
+        P<uint32_t>(ctx->clipFirst), scal + kClipSlot);
     RIVE_TRY(ensure(ctx, ctx->prims, (size_t)std::max<uint32_t>(totalPrims, 1) * 2 * sizeof(int4)));
     RIVE_TRY(ensure(ctx, ctx->primFlags, (size_t)std::max<uint32_t>(totalPrims, 1) * 4));
     RIVE_TRY(ensure(ctx, ctx->primCov, (size_t)std::max<uint32_t>(totalPrims, 1) * sizeof(PrimCov)));
@@ -1613,8 +1615,8 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
         return [&, kernel](uint32_t blocks, uint32_t threads, uint32_t lds, uint32_t minCells, uint32_t maxCells) {
             kernel<<<blocks, threads, lds, ctx->stream>>>(
                 prims, binDraws, P<PathCells>(ctx->cells), P<uint32_t>(ctx->pathDraws), minCells, maxCells,
-                P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases, P<uint2>(ctx->cellPacked),
-                P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
+                P<PathPaint>(ctx->pathPaint), P<uint32_t>(ctx->pathCanvas), canvases, scal + kClipSlot,
+                P<uint2>(ctx->cellPacked), P<uint32_t>(ctx->pathBins), P<uint32_t>(ctx->tileCover));
         };
     };
     const auto scatter = [&](auto kernel) {

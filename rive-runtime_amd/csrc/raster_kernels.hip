@@ -1709,7 +1709,8 @@ __device__ __forceinline__ float fill_rule_coverage(float count, uint32_t flags)
 // of that one's outer clip, and so on -- or i itself when it reads none.  The
 // updates are looked for among the kClipSearch paths before it (a clip is
 // nearly always drawn right before its draws); one not found there gives 0,
-// the flush's start, which is always right.
+// the flush's start, which is always right.  This takes one update for each ID:
+// a flush that reuses one (clip_id_reused) has no covers.
 constexpr uint32_t kClipSearch = 256;
 __device__ __forceinline__ uint32_t clip_reach(const uint2* __restrict__ paints, uint32_t i)
 {
@@ -1726,6 +1727,39 @@ __device__ __forceinline__ uint32_t clip_reach(const uint2* __restrict__ paints,
         }
     }
     return id == 0u ? at : 0u;
+}
+
+// Whether clip update i (`update`) may write an ID that an earlier update among
+// paths [first, i) wrote: each update's ID is held against the one before it, so
+// IDs that ascend, as the front end numbers them, are all new.  One wave, lanes
+// of consecutive paths from a multiple of 64, all active; the update before a
+// wave's first is looked for 64 paths at a time.
+__device__ __forceinline__ bool clip_id_reused(const uint2* __restrict__ paints, uint32_t i, uint32_t first, bool update)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t updates = __ballot(update);
+    if (updates == 0)
+        return false;
+    const uint32_t id = update ? paints[i].y >> 16 : 0u;
+    const uint64_t below = updates & ((1ull << lane) - 1ull);
+    const int from = below != 0 ? 63 - __clzll((long long)below) : 0;
+    const uint32_t before = (uint32_t)__shfl((int)id, from);
+    bool reused = update && below != 0 && i - (uint32_t)(lane - from) >= first && id <= before;
+    const int lead = __builtin_ctzll(updates);
+    const uint32_t lo = (uint32_t)__shfl((int)first, lead);
+    for (uint32_t end = i - (uint32_t)lane; end > lo; end -= 64u)
+    {
+        const uint32_t p = end - 64u + (uint32_t)lane;
+        const uint2 q = p >= lo ? paints[p] : make_uint2(~0u, 0u);
+        const uint64_t found = __ballot((q.x & 0xfu) == CLIP_UPDATE_PAINT_TYPE);
+        if (found != 0)
+        {
+            const uint32_t last = (uint32_t)__shfl((int)(q.y >> 16), 63 - __clzll((long long)found));
+            reused = reused || (lane == lead && id <= last);
+            break;
+        }
+    }
+    return reused;
 }
 
 // ---------------------------------------------------------------------------
@@ -2040,8 +2074,8 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
     PrimStore prims, const DrawTess* __restrict__ draws, const PathCells* __restrict__ cells,
     const uint32_t* __restrict__ pathDraws, uint32_t minCells, uint32_t maxCells,
     const PathPaint* __restrict__ pathPaint, const uint32_t* __restrict__ pathCanvas,
-    const CanvasDev* __restrict__ canvases, uint2* __restrict__ packed, uint32_t* __restrict__ pathBins,
-    uint32_t* __restrict__ tileCover)
+    const CanvasDev* __restrict__ canvases, const uint32_t* __restrict__ clipReused, uint2* __restrict__ packed,
+    uint32_t* __restrict__ pathBins, uint32_t* __restrict__ tileCover)
 {
     extern __shared__ uint32_t sCell[];
     __shared__ uint32_t sWaveSum[THREADS / 64];
@@ -2066,7 +2100,7 @@ __global__ __launch_bounds__(THREADS) void bin_count_solo_kernel(
     // fill covers the tiles without primitives that it fills
     const uint32_t rows = (uint32_t)(c.ty1 - c.ty0);
     const uint32_t kind = pathPaint[d.pathID].kind;
-    const bool opaque = (kind & kPaintOpaque) != 0u;
+    const bool opaque = (kind & kPaintOpaque) != 0u && *clipReused == 0u;
     uint32_t* cover = nullptr;
     uint32_t coverStride = 0;
     if (opaque)
@@ -3970,8 +4004,10 @@ __global__ __launch_bounds__(kWgThreads, WAVES) void raster_kernel(
 __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const uint2* __restrict__ paints,
                                    const float* __restrict__ aux, const uint32_t* __restrict__ pathImage,
                                    uint32_t pathCount, const FlushDev* __restrict__ flushes, uint32_t flushCount,
+                                   const uint32_t* __restrict__ pathCanvas, const CanvasDev* __restrict__ canvases,
                                    PathRaster* __restrict__ out, PathPaint* __restrict__ outPaint,
-                                   PathCells* __restrict__ cells, uint32_t* __restrict__ clipFirst)
+                                   PathCells* __restrict__ cells, uint32_t* __restrict__ clipFirst,
+                                   uint32_t* __restrict__ clipReused)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // the earliest path the 64 paths of this wave read clip content from
@@ -3979,10 +4015,16 @@ __global__ void path_raster_kernel(const PathDataV* __restrict__ paths, const ui
     reach = (uint32_t)wave_min((int32_t)min(reach, 0x7fffffffu));
     if ((threadIdx.x & 63) == 0 && i <= pathCount)
         clipFirst[i >> 6] = reach;
+    const FlushDev fl = flushes[flush_of<&FlushDev::pathBase>(flushes, flushCount, min(i, pathCount))];
+    // (clip IDs are numbered per flush; the buffer itself is per canvas)
+    const uint32_t canvas = i <= pathCount ? pathCanvas[i] : 0xffffffffu;
+    const uint32_t firstPath = max(fl.pathBase + 1u, canvas != 0xffffffffu ? canvases[canvas].firstPath : 0u);
+    const bool update = i <= pathCount && i != fl.pathBase && (paints[i].x & 0xfu) == CLIP_UPDATE_PAINT_TYPE;
+    if (clip_id_reused(paints, i, firstPath, update))
+        *clipReused = 1u; // every writer stores the same value
     if (i > pathCount)
         return;
     PathRaster r;
-    const FlushDev fl = flushes[flush_of<&FlushDev::pathBase>(flushes, flushCount, i)];
     const PathDataV pd = paths[i];
     const uint2 paint = paints[i];
     const float* ax = aux + (size_t)i * 32;
