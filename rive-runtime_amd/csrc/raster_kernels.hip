@@ -33,7 +33,6 @@ namespace rivehip
 __device__ __forceinline__ float u2f(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t f2u(float f) { return __float_as_uint(f); }
 
-__device__ __forceinline__ int64_t floor_div128(int64_t a) { return a >> 7; }
 __device__ __forceinline__ int64_t ceil_div128(int64_t a) { return -((-a) >> 7); }
 __device__ __forceinline__ int32_t clamp_thr(int64_t t)
 {
