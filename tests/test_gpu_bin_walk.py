@@ -3,7 +3,13 @@ line, aside and takes them 64 a wave at a time, in workgroups whose size follows
 the number of draws and the canvas.  Contours of long diagonals (every segment
 put aside), of short segments (few) and of both, in counts around a wave's queue
 and on either side of each workgroup size, against the oracle: within 2/255 on
-all but 0.1% of pixels and 8/255 everywhere."""
+all but 0.1% of pixels and 8/255 everywhere.
+
+Parity unpinned: a thousand long diagonals in one path, and feathered stars of
+more than 65.  Every edge adds what its vertices' snapping to 1/256 px moves its
+border, so the sum of so many a pixel leaves that tolerance whatever bins them.
+The diagonals are binned both ways instead -- in LDS, and by global atomics as a
+path with guard-box pieces is -- and must give the same bytes."""
 import numpy as np
 import pytest
 
@@ -28,8 +34,7 @@ def check(ctx, b):
     assert d.max() <= 8 and (d > 2).mean() <= 1e-3, f"max {d.max()}, frac>2 {(d > 2).mean()}"
 
 
-# (not 1100 long ones: a thousand diagonals through every tile leave the
-# oracle's tolerance whatever bins them, byte for byte the same as before)
+# (1100 long ones: test_routes_agree)
 COUNTS = [(k, n) for k in ("long", "short", "mixed") for n in (3, 63, 64, 65, 112, 113, 400, 1100)
           if (k, n) != ("long", 1100)]
 
@@ -49,10 +54,35 @@ def test_segments_put_aside(hip_ctx, kind, n, feather):
         else:
             x, y = x + float(rng.uniform(-7, 7)), y + float(rng.uniform(-7, 7))
         cmds.append((1, x, y))
-    # (a feathered star this dense sums hundreds of segments a pixel: fewer of them)
+    # (feathered stars of more segments: parity unpinned)
     b.draw(b.path(cmds[:1 + (n if feather == 0 else min(n, 65))] + [(5,)], fill_rule=EVENODD if n % 2 else NONZERO),
            color=0xc0f08020, feather=feather)
     check(hip_ctx, b)
+
+
+@pytest.mark.parametrize("n", [1100, 4001])
+def test_routes_agree(hip_ctx, n):
+    """A spike right of the canvas, out of the guard box and back, gives the path
+    pieces, so that it is binned by global atomics; on the canvas nothing changes."""
+    print(f"[bin-walk] routes {n}", flush=True)
+    rng = np.random.default_rng(n)
+    w, h = 333, 271
+    pts = rng.uniform([-20, -20], [w + 20, h + 20], (n, 2))
+    head = [(0, w / 2, h / 2)] + [(1, float(x), float(y)) for x, y in pts] + [(1, w + 140., h / 2), (1, w + 160., h / 2 + 10)]
+    out = []
+    for spike in ([], [(1, 60000., h / 2 + 10), (1, w + 160., h / 2 + 10)]):
+        b = StreamBuilder(w, h, clear_color=0xff203040)
+        b.draw(b.path(head + spike + [(1, w + 180., h / 2), (5,)], fill_rule=EVENODD if n % 2 else NONZERO),
+               color=0xc0f08020)
+        t = hip_ctx.target(w, h)
+        try:
+            hip_ctx.render_stream(b.build(), t)
+            assert (hip_ctx.last_flush_stats().guard_pieces > 0) == bool(spike)
+            out.append(hip_ctx.read_pixels(t, w, h))
+        finally:
+            hip_ctx.free_target(t)
+    assert len(np.unique(out[0].reshape(-1, 4), axis=0)) > 100
+    assert np.array_equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("w,h,n", [(160, 128, 512), (160, 128, 513), (160, 128, 2048), (160, 128, 2049),

@@ -2,8 +2,8 @@
 within 64 px; feathered segments within 128 px with edges up to 101 px) and
 double for the rest.  Polygons and strokes whose straight edges lie on either
 side of those limits, at offsets on and off tile corners, and feathers of
-radii around them must match the oracle with the tolerances of the other
-parity tests.  (Feathers whose radius exceeds the shape are left out: there the
+radii around them must match the oracle within 2/255 on all but 0.1% of pixels and
+8/255 everywhere, as the scenes of test_gpu_random_scenes.py do.  (Feathers whose radius exceeds the shape are left out: there the
 oracle's quarter-resolution atlas and a direct evaluation differ by design.)"""
 import numpy as np
 import pytest
@@ -25,7 +25,7 @@ def zigzag(length, x, y, n, closed):
     return [(0, *pts[0])] + [(1, *p) for p in pts[1:]] + ([(5,)] if closed else [])
 
 
-def compare(ctx, b, limit, share):
+def compare(ctx, b):
     s = b.build()
     f = ob.OracleFlush(s)
     t = ctx.target(b.width, b.height)
@@ -38,7 +38,7 @@ def compare(ctx, b, limit, share):
         f.close()
     d = np.abs(out.astype(np.int32) - ref.astype(np.int32)).max(axis=2)
     assert out.any()
-    assert d.max() <= limit and (d > 2).mean() <= share, f"max {d.max()}, frac>2 {(d > 2).mean()}"
+    assert d.max() <= 8 and (d > 2).mean() <= 1e-3, f"max {d.max()}, frac>2 {(d > 2).mean()}"
 
 
 @pytest.mark.parametrize("length", [15.99, 16.0, 47.5, 63.9, 64.0, 64.3, 100.0, 240.0, 5000.0])
@@ -49,7 +49,7 @@ def test_edges_around_the_near_limit(hip_ctx, length):
         b.draw(b.path(zigzag(length, x, y, 7, True), k % 2), color=0xa0ff8040 + 0x30507 * k)
         b.draw(b.path(zigzag(length, x + 5, y - 3, 5, False)), color=0xc040a0ff - 0x30507 * k, stroke=[1., 6., 40., .4][k],
                join=MITER)
-    compare(hip_ctx, b, 8, 1e-3)
+    compare(hip_ctx, b)
 
 
 @pytest.mark.parametrize("feather", [2.0, 20.0, 41.0, 60.0, 84.0])
@@ -59,4 +59,4 @@ def test_feathers_around_the_near_limit(hip_ctx, feather):
     b.draw(b.path([(0, 60, 50), (1, 170, 64), (4, 200, 130, 120, 190, 70, 150), (5,)], CLOCKWISE), color=0xffe0a030,
            feather=feather)
     b.draw(b.path(zigzag(90.0, 40.0, 100.0, 3, False)), color=0xc040a0ff, stroke=9.0, feather=feather / 4)
-    compare(hip_ctx, b, 24, 5e-3)
+    compare(hip_ctx, b)
