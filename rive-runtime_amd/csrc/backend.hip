@@ -1483,9 +1483,10 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     RIVE_TRY(ensure(ctx, ctx->tileQueue, queueWords * 4));
     // Until a config is set: heaviest tiles first wherever the launch has more
     // tiles than run at once, so that long tiles do not trail (the order costs
-    // two kernels, ~15 us).  Measured on MI355X, raster pass with the order's
-    // kernels: 1080p frame 9.0 -> 7.35 ms, 48 canvases 6.6 -> 4.4 ms, 24 served
-    // requests 7.0 -> 5.4 ms, 1024^2 200-path frame .27 ms either way.
+    // two kernels, 15-30 us).  Measured on MI355X as it was added, raster pass with
+    // the order's kernels: 1080p frame 9.0 -> 7.35 ms, 48 canvases 6.6 -> 4.4 ms, 24
+    // served requests 7.0 -> 5.4 ms, 1024^2 200-path frame .27 ms either way; a
+    // 1024x768 frame of 20 paths, whose tiles all cost little, .03 -> .07 ms.
     const uint32_t resident =
         (uint32_t)std::max(ctx->cuCount, 1) * (ctx->rasterConfig.waves_per_simd == 5 ? 5u : 6u);
     const bool ordered = tileTotal > 0 && (ctx->rasterConfigSet ? ctx->rasterConfig.tile_order != 0 : tileTotal > resident);
@@ -1596,8 +1597,8 @@ int raster_pipeline(rive_hip_context* ctx, const LaunchGroup& g, DrawTess* drawT
     // The solo kernels' LDS: as many words as the largest canvas has tiles, up to
     // the small limit; a second launch takes the larger grids.  A CU holds 32
     // waves: 8 workgroups of 256 threads, or fewer of 512 or 1024 where the draws
-    // or the LDS allow no more.  Measured on MI355X, both kernels, 256 threads
-    // against the form taken here: 5000 draws of up to 8160 cells 1.11 -> .83 ms
+    // or the LDS allow no more.  Measured on MI355X when the sizes were chosen, both
+    // kernels, 256 threads against the form taken here: 5000 draws of up to 8160 cells 1.11 -> .83 ms
     // (512), 722 draws .24 -> .13 ms (512), 200 draws .157 -> .107 ms (1024).
     const bool bin = totalPrims > 0 && drawCount > 0 && totalCells > 0;
     const uint32_t largeCells = std::min(maxTiles, kBinLargeCells);

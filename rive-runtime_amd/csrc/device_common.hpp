@@ -59,9 +59,9 @@ struct TessTexel
 
 // Wave-wide sums and minima by DPP: row_shr 1, 2, 4, 8 within the rows of 16
 // lanes, then row_bcast 15 and 31 across them -- six adds, where shuffles are six
-// trips through LDS.  All 64 lanes must be active.  Measured on MI355X, end to
-// end: 1080p 5000-path frame 8.16 -> 8.00 ms, 4K 20 000-draw frame 193 -> 187 ms,
-// 10-path icon .60 -> .58 ms.
+// trips through LDS.  All 64 lanes must be active.  Measured on MI355X as it was
+// added, end to end: 1080p 5000-path frame 8.16 -> 8.00 ms, 4K 20 000-draw frame
+// 193 -> 187 ms, 10-path icon .60 -> .58 ms.
 __device__ __forceinline__ int32_t row_scan16(int32_t x) // inclusive, within each row
 {
     x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);

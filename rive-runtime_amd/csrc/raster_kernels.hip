@@ -1697,10 +1697,10 @@ __device__ __forceinline__ float fill_rule_coverage(float count, uint32_t flags)
 // since draws after it may read their clip IDs; clipFirst bounds how far back
 // those reach.  The pixels are those of drawing everything.  Hidden (path,
 // tile) pairs are not scattered into the bins either.  The raster is bound by
-// VALU issue in resolving paths, so what it skips is what it gains: on random
-// scenes of which 0.4% of the solid paints are opaque, raster pass 16.7 ->
-// 14.4 ms (1080p 5000-path frame), 8.7 -> 8.1 ms (48 canvases), 10.4 -> 8.3 ms
-// (24 served scenes); scenes of opaque shapes gain in proportion to what they
+// VALU issue in resolving paths, so what it skips is what it gains: as it was
+// added, on random scenes of which 0.4% of the solid paints are opaque, raster
+// pass 16.7 -> 14.4 ms (1080p 5000-path frame, flush by flush), 8.7 -> 8.1 ms
+// (48 canvases), 10.4 -> 8.3 ms (24 served scenes); scenes of opaque shapes gain in proportion to what they
 // hide, and one that hides nothing pays a load per tile.
 //
 // clip_reach: the first path whose drawing the clip buffer content path i
@@ -1937,10 +1937,11 @@ __device__ __forceinline__ void for_prim_crossings(const Prim& p, const PathCell
 // crosses no tile line, most of the time; the few that need their cells trimmed
 // row by row or a crossing settled would make every wave take both forms, so
 // each wave puts their indices aside in its part of the queue and takes them 64
-// together.  Measured on MI355X, counting and scattering kernels (with the
-// workgroup sizes the launches choose): 1080p 5000-path frame 1.15 -> .83 ms, 48
-// canvases .59 -> .51 ms, 600 triangulated draws .24 -> .13 ms, 4K 20 000-draw frame
-// 18.6 -> 18.3 ms (there nearly every segment spans rows and columns).
+// together.  Measured on MI355X as it was added, counting and scattering kernels
+// (with the workgroup sizes the launches choose): 1080p 5000-path frame 1.15 ->
+// .83 ms, 48 canvases .59 -> .51 ms, 600 triangulated draws .24 -> .13 ms, 4K
+// 20 000-draw frame 18.6 -> 18.3 ms (there nearly every segment spans rows and
+// columns).  The scatter adds up tile costs since: .87, .58, .15 and 19.1 ms.
 constexpr uint32_t kWalkQueue = 112; // (what the largest grids leave of the LDS)
 template <int THREADS, bool CROSS, typename C, typename X>
 __device__ __forceinline__ void walk_prims(const PrimStore& prims, const DrawTess& d, const PathCells& c,
@@ -2017,9 +2018,11 @@ __device__ __forceinline__ void walk_prims(const PrimStore& prims, const DrawTes
 // (25 M cells in the 1080p 5000-path frame).  Grids of more than kBinSmallCells
 // cells (a canvas beyond 8192 tiles) take the same kernel with up to 160 KB of
 // LDS and 1024 threads, one workgroup per CU; they used to go through one
-// global atomic per (primitive, tile).  Measured on MI355X, the whole pass
-// (expansion included): 1080p 5000-path frame 3.53 -> 3.00 ms, 3840x2160
-// 20 000-path frame 126.8 -> 46.7 ms, 48-canvas batch 2.14 -> 1.79 ms.
+// global atomic per (primitive, tile).  Measured on MI355X as it was added, the
+// whole pass (expansion included): 1080p 5000-path frame 3.53 -> 3.00 ms,
+// 3840x2160 20 000-path frame 126.8 -> 46.7 ms, 48-canvas batch 2.14 -> 1.79 ms;
+// with launch groups, the walk and the expansion's own vertices 1.44, 22.3 and
+// 1.33 ms.
 //
 // Other paths (several draws, as with guard-box pieces; 32768 primitives or
 // more, which the packed LDS word cannot count; grids beyond the large LDS)
@@ -2542,10 +2545,11 @@ __device__ __forceinline__ int32_t border_fixed(float cv)
 // or.  Other primitives take double, exact for coordinates in [-2^23, 2^23):
 // every product is below 2^49.  The rows are VALU-bound; the form they replace
 // recomputed seven (fills) or five (strokes) double thresholds with their
-// floors and ceilings and two candidate searches per row.  Measured on MI355X,
-// raster pass with the batch's six barriers cut to three beside it: 1080p frame
-// 10.0 -> 9.0 ms, 48 canvases 8.1 -> 6.6 ms, feathered 961x541 frame 11.4 -> 9.6
-// ms (in double alone the feathered rows took 16.3 ms).
+// floors and ceilings and two candidate searches per row.  Measured on MI355X as
+// it was added, raster pass with the batch's six barriers cut to three beside it:
+// 1080p frame 10.0 -> 9.0 ms, 48 canvases 8.1 -> 6.6 ms, feathered 961x541 frame
+// 11.4 -> 9.6 ms (in double alone the feathered rows took 16.3 ms); with tiles
+// heaviest first and the feather table in LDS 6.9, 4.1 and 5.8 ms.
 constexpr int32_t kNearSub = 1 << 14;
 template <typename I> struct RowMath;
 template <> struct RowMath<int32_t>
@@ -2798,8 +2802,8 @@ __device__ __forceinline__ void stroke_row(const TilePrim<I>& n, uint32_t flags,
 // Out-of-line rows take their accumulators and the feather table as LDS pointers
 // and the vertices by value: through generic pointers every update was a flat
 // atomic and every sample of the table two flat loads, which bound the feathered
-// rows.  Measured on MI355X, raster pass: feathered 961x541 frame 9.3 -> 6.1 ms,
-// 4K 20 000-draw frame 72 -> 60 ms.
+// rows.  Measured on MI355X as it was added, raster pass: feathered 961x541 frame
+// 9.3 -> 6.1 ms, 4K 20 000-draw frame 72 -> 60 ms (with sums by DPP 5.8 and 55).
 typedef __attribute__((address_space(3))) int32_t LdsInt;
 typedef __attribute__((address_space(3))) uint32_t LdsUint;
 typedef __attribute__((address_space(1))) const PrimCov GlobalCov;
@@ -2833,7 +2837,9 @@ __device__ __noinline__ void stroke_far_row(TilePrim<int32_t> n, uint32_t flags,
 
 // eval_feathered_fill (draw_path_common.glsl:153-240): the feather above y0
 // plus a 4-sample midpoint integral of FEATHER(u) FEATHER'(t) across a
-// corner, signed by coverages.x.
+// corner, signed by coverages.x.  (exp2 is the hardware's, to the error that
+// exp2f has; it gives 0 where exp2f gives a denormal, which such a sum of terms
+// up to 1 does not hold.)
 __device__ __forceinline__ float eval_feathered_fill(const float* c, const uint32_t* __restrict__ table)
 {
     const float cotTheta = c[2];
@@ -3096,8 +3102,9 @@ __device__ __forceinline__ uint32_t mean4(uint32_t a, uint32_t b, uint32_t c, ui
 // one below, rounded down, so the 64x64 texels of a workgroup's block make its
 // texels of every level by themselves: they are read once, and each level made
 // is kept in LDS for the next.  One launch a level was bound by its launches:
-// measured on MI355X with the small scans and fills below, the feathered 961x541
-// frame that creates 64 images (512 launches of 2.3 us) 13.3 -> 11.4 ms.
+// measured on MI355X as it was added with the small scans and fills below, the
+// feathered 961x541 frame that creates 64 images (512 launches of 2.3 us) 13.3 ->
+// 11.4 ms (128 launches of 4.2 us).
 constexpr int kMipStep = 6, kMipBlock = 64;
 struct MipLevels
 {
@@ -3533,8 +3540,8 @@ __device__ __forceinline__ uint32_t cost_class(uint32_t cost)
 // The tiles' costs, in place, to their classes, counted in hist.  The scatter
 // adds the costs up as it reads the grids (a path that several draws bin into
 // as its grid is laid out, hidden tiles included: the order is a heuristic).  A
-// wave a tile used to look every path up again: measured on MI355X, 1080p
-// 5000-path frame 7.62 -> 7.35 ms, 24 served requests 16.5 -> 15.8 ms.
+// wave a tile used to look every path up again: measured on MI355X as it was
+// added, 1080p 5000-path frame 7.62 -> 7.35 ms, 24 served requests 16.5 -> 15.8 ms.
 __global__ __launch_bounds__(256) void tile_class_kernel(uint32_t* __restrict__ tileClass, uint32_t tileTotal,
                                                          uint32_t* __restrict__ hist)
 {
@@ -4229,8 +4236,8 @@ __global__ void scan_apply_kernel(const uint32_t* __restrict__ in, uint32_t n,
 // most three): each thread four values a step, waves' sums through LDS.  The
 // total is summed in 64 bits, as 16-bit halves within a wave.  At the limit it
 // takes four dependent steps, about what the three launches cost.  Measured on
-// MI355X with a flush's fills in one launch: 10-path icon .61 -> .48 ms, 200-path
-// 1024^2 frame 1.21 -> 1.00 ms.
+// MI355X as it was added with a flush's fills in one launch: 10-path icon .61 ->
+// .48 ms, 200-path 1024^2 frame 1.21 -> 1.00 ms.
 constexpr uint32_t kScanSmall = 16384;
 struct ScanJob
 {
