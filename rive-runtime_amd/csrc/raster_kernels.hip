@@ -768,7 +768,7 @@ __device__ FeatherEnd feather_end(const TessTexel* __restrict__ tex, int texels,
         TessTexel after = tex[min(max(k + ey, 0), texels - 1)];
         if ((after.w & (MIRRORED_CONTOUR_CONTOUR_FLAG | 0xffffu)) !=
             (before.w & (MIRRORED_CONTOUR_CONTOUR_FLAG | 0xffffu)))
-            after = tex[min((int)vertexIndex0, texels - 1)];
+            after = tex[min(vertexIndex0, (uint32_t)texels - 1u)];
         edge0 = u2f(before.z);
         const float edge1 = u2f(after.z);
         corner = edge1 - edge0;
@@ -1322,7 +1322,7 @@ __global__ __launch_bounds__(kExpandThreads) void expand_kernel(
     if (wrap)
     {
         bool isClosed = pd.strokeRadius == 0.f || cd.mx != 0.f;
-        j = isClosed ? min((int)cd.vertexIndex0, texels - 1) : i;
+        j = isClosed ? (int)min(cd.vertexIndex0, (uint32_t)texels - 1u) : i; // (a record may hold any index)
         cfj = (tex[j].w & ~MIRRORED_CONTOUR_CONTOUR_FLAG) | (cfi & MIRRORED_CONTOUR_CONTOUR_FLAG);
     }
     if (makes && feathered)
